@@ -39,12 +39,22 @@ constexpr int kBlk = 32;         // P(D) values per min/sum block
 constexpr int kWarm = 64;        // most warm-up steps of the truncated recurrences
 constexpr int kDbg = 32;         // debug scalars per (walker, field)
 constexpr int kState = 16;       // per-walker scalars handed between kernels
-constexpr int kPixBlocks = 64;   // workgroups per (walker, field), unbinned
+constexpr int kPixBlocks = 32;   // workgroups per (walker, field), unbinned
 constexpr int kGL = 32;          // Gauss-Legendre points per knot interval
 constexpr int kIPart = 8;        // partial statistics per inverse part
 constexpr int kMaxSlots = 256;   // (walker, part) slots of the split transforms
 // device scratch of the allocation-free batch entry point, per GPU
 constexpr size_t kNoallocScratchBytes = size_t(512) << 20;
+
+// One pixel of an unbinned dataset, in ascending order of flux: its flux c
+// and q, the sum of the fluxes before it in units of 2^-pexp (modulo 2^64;
+// one more entry at the end, flux +inf, holds the sum of all).  Differences
+// of q over the pixels of one P(D) cell are exact, so the cell's sum of
+// (c - cell edge) has no cancellation error.
+struct PixSum {
+  double c;
+  int64_t q;
+};
 
 // One field (dataset) of a beam set, device view.
 struct FieldDev {
@@ -55,8 +65,18 @@ struct FieldDev {
   const uint32_t* bins;   // nbins
   uint32_t nbins;
   double bincent0, bindelta;
-  const double* pix;      // npix (sorted ascending), unbinned only
+  // unbinned only
   uint64_t npix;
+  const PixSum* pix;      // npix + 1, ascending
+  int pexp;
+  // the core: pixels [pa, pb), the fluxes of the rcols P(D) cells' widths
+  // from ca that hold more pixels than cells (none: pa = pb), and their
+  // ranks on a sub-grid: entry [r * rcols + j] is the number of pixels below
+  // ca + (j 2^rlog + r) dflux / 2^rlog, 0 <= r <= 2^rlog
+  uint32_t pa, pb, rcols;
+  int rlog;
+  double ca;
+  const uint32_t* rank;
 };
 
 constexpr int kMaxFields = 16;
@@ -217,6 +237,5 @@ int launch_pd_loglike2d(const double* d_pd, int n1, int n2, double minflux1, dou
 int noalloc_init(int device);
 void* noalloc_scratch(int device);
 int launch_materialize_pd(const double* d_pofd, int N, int split, double itot,
-                          int is_log, int already_log, double* d_out,
-                          void* stream);
+                          int is_log, double* d_out, void* stream);
 }  // namespace pofd

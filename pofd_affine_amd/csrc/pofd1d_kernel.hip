@@ -18,8 +18,8 @@
 //   finalize  per (walker, dataset): findSplitPoint (:691-921), rotation,
 //             normalisation and mean (:934-1009), the binned log likelihood
 //             (src/PD.cc:557-619)
-//   pixels    unbinned log likelihood (src/PD.cc:628-677), kPixBlocks
-//             workgroups of 256 per (walker, dataset)
+//   pixels    unbinned log likelihood (src/PD.cc:628-677) by cells of the
+//             P(D) grid, kPixBlocks workgroups of 256 per (walker, dataset)
 //   combine   (curr - like_offset)/like_norm summed over the datasets in
 //             order (src/calcLike.cc:425), into the batch outputs
 //
@@ -1591,8 +1591,8 @@ __global__ __launch_bounds__(kThreads) void inverse1d_kernel(const BeamsetDev bs
 
 // ===========================================================================
 // finalize: one workgroup per (walker, dataset): findSplitPoint, rotation,
-// normalisation, mean, binned log likelihood (an unbinned dataset gets
-// log2 of its normalised P(D) in place for pixels1d_kernel)
+// normalisation, mean, binned log likelihood (an unbinned dataset's sum is
+// pixels1d_kernel's)
 // ===========================================================================
 // combine for one walker: (curr - like_offset)/like_norm summed over the
 // datasets of the beam set in order, added to the batch outputs (one
@@ -1906,17 +1906,6 @@ __global__ __launch_bounds__(kThreads) void finalize1d_kernel(const BeamsetDev b
         }
       }
       curr = 0.69314718055994530942 * block_sum(part, red);  // log2toe
-    } else {
-      __syncthreads();  // every load of the split search precedes the rewrite
-      // eight values a step per thread (N is a multiple of 8 x kThreads):
-      // their loads issued together
-      for (int j = tid; j < N; j += 8 * kThreads) {
-        double v[8];
-#pragma unroll
-        for (int u = 0; u < 8; ++u) v[u] = pofd[j + u * kThreads];
-#pragma unroll
-        for (int u = 0; u < 8; ++u) pofd[j + u * kThreads] = log2_or_small(v[u] * itot);
-      }
     }
   }
   if (tid == 0) {
@@ -1949,90 +1938,119 @@ __global__ __launch_bounds__(kThreads) void finalize1d_kernel(const BeamsetDev b
 // ===========================================================================
 // pixels: unbinned log likelihood, kPixBlocks workgroups per (walker, field)
 // ===========================================================================
+// The sum over pixels of the linear interpolation of L = log2 P(D) is a sum
+// over the cells [f_i, f_i+1) of the walker's flux grid f_i = minflux + i
+// dflux: a cell holding the pixels [p, p') adds (p' - p) L_i + (L_i+1 - L_i)
+// T, T = sum (c - f_i) / dflux.  The pixels are sorted and do not depend on
+// theta, so T comes from the running sums at p and p' and the ranks p from a
+// table and a short search, whatever the number of pixels.  The core of the
+// map is summed that way, a wavefront taking 63 cells (64 edges) a step; the
+// pixels outside it, fewer than the cells they lie in, one by one.
+// Bound by the L1-L2 lines of the searches (153 a step) and the VALU work of
+// the log2 (222 instructions a step): at 256 walkers, 1e6 pixels and nflux
+// 2^17, 416 steps of cells and 94 of pixels a walker take 96 us, where two
+// gathers a pixel took 394 us and the rewrite of the P(D) as log2 that they
+// read another 100 us.
 constexpr int kPixThreads = 256;
-constexpr int kPixU = 8;  // pixels per thread per step
 
-__global__ __launch_bounds__(kPixThreads, 8) void pixels1d_kernel(const BeamsetDev bs,
-                                                                const WorkDev wk) {
+__global__ __launch_bounds__(kPixThreads) void pixels1d_kernel(const BeamsetDev bs,
+                                                               const WorkDev wk) {
   __shared__ double red[kPixThreads / 64];
-  const int blk = blockIdx.x;
-  const int walker = blockIdx.y;
+  const int walker = blockIdx.x;  // neighbours in launch order share pixels
+  const int blk = blockIdx.y;
   const int f = blockIdx.z;
   const FieldDev& fd = bs.fields[f];
   if (fd.binned || walker >= batch_n(wk)) return;
   const size_t wf = static_cast<size_t>(walker) * bs.nfields + f;
   double* out = wk.upart + wf * kPixBlocks + blk;
   const double* dbg = wk.dbg + wf * kDbg;
-  if (walker_state(wk, walker)[ST_STATUS] != POFD_OK || dbg[15] != POFD_OK ||
-      dbg[18] == 0.0) {
+  if (walker_state(wk, walker)[ST_STATUS] != POFD_OK || dbg[15] != POFD_OK) {
     if (threadIdx.x == 0) *out = 0.0;
     return;
   }
   const int N = bs.N;
-  const double dflux = bs.dflux;
-  const int split = static_cast<int>(dbg[0]);
-  const double minflux = dbg[17];
-  const double* L = wk.pofd + wf * wk.pofd_stride;  // log2 P(D), unrotated
+  const double dflux = bs.dflux, idflux = 1.0 / dflux;
+  const uint32_t split = static_cast<uint32_t>(static_cast<int>(dbg[0]));
+  const double itot = dbg[16], minflux = dbg[17];
+  const double* pofd = wk.pofd + wf * wk.pofd_stride;  // unrotated
+  const uint32_t nm1 = static_cast<uint32_t>(N - 1);
+  auto Lrot = [&](const uint32_t i) { return log2_or_small(pofd[(i + split) & nm1] * itot); };
+  const uint32_t pa = fd.pa, pb = fd.pb, rcols = fd.rcols;
+  const int lane = threadIdx.x & 63;
+  const PixSum* pix = fd.pix;
+  // the edges [e_lo, e_hi] around the core, one cell to spare either side
+  const double dlo = floor((fd.ca - minflux) * idflux) - 1.0;
+  const int e_lo = static_cast<int>(fmin(fmax(dlo, 0.0), static_cast<double>(N - 2)));
+  const int e_hi = static_cast<int>(
+      fmin(fmax(dlo + static_cast<double>(rcols) + 3.0, 0.0), static_cast<double>(N - 2)));
+  const int nchunk = (pa < pb) ? max((e_hi - e_lo + 62) / 63, 1) : 0;
+  const uint32_t nout = static_cast<uint32_t>(fd.npix) - (pb - pa);
+  const int nstep = nchunk + static_cast<int>((nout + 63) >> 6);
+  const double unit = ldexp(1.0, fd.pexp);
+  const double tscale = ldexp(idflux, -fd.pexp);
+  const double rstep = ldexp(idflux, fd.rlog), rend = ldexp(static_cast<double>(rcols), fd.rlog);
+  const uint32_t rmask = (1u << fd.rlog) - 1u;
   double part = 0.0;
-  {
-#pragma clang fp contract(off)
-    const double maxflux = minflux + static_cast<double>(N - 1) * dflux;
-    const double idflux = 1.0 / dflux;
-    const double maxfluxval = maxflux - dflux;
-    // rotated index i -> i + split mod N (N is a power of two), as a 32-bit
-    // byte offset from the walker's table
-    const char* Lb = reinterpret_cast<const char*>(L);
-    const uint32_t nm1 = static_cast<uint32_t>(N - 1), usplit = static_cast<uint32_t>(split);
-    auto Lr = [&](const uint32_t i) {
-      return *reinterpret_cast<const double*>(Lb + (((i + usplit) & nm1) << 3));
-    };
-    // contiguous pixel ranges per workgroup: pixels are sorted, so
-    // neighbouring lanes read neighbouring P(D) values
-    const uint64_t per = (fd.npix + kPixBlocks - 1) / kPixBlocks;
-    const uint64_t p0 = per * blk;
-    const uint64_t p1 = (p0 + per < fd.npix) ? p0 + per : fd.npix;
-    const uint32_t cnt = (p1 > p0) ? static_cast<uint32_t>(p1 - p0) : 0u;
-    const char* pb = reinterpret_cast<const char*>(fd.pix + p0);
-    auto pix = [&](const uint32_t k) { return *reinterpret_cast<const double*>(pb + (k << 3)); };
-    // the term of pixel flux cflux, as PD::getLogLike takes it: Lr(0) at or
-    // below minflux, Lr(N - 1) at or above maxflux - dflux, else the linear
-    // interpolation; the end cases as weights (1, 0) of the same formula,
-    // which give the end value exactly (the table holds finite values)
-    auto term = [&](const double cflux) {
-      const bool lo = cflux <= minflux, hi = cflux >= maxfluxval;
-      const double delt = (lo || hi) ? 0.0 : (cflux - minflux) * idflux;
-      const uint32_t id0 = static_cast<uint32_t>(static_cast<int>(delt));
-      const double t0 = delt - static_cast<double>(static_cast<int>(id0));
-      const uint32_t idx = hi ? nm1 : id0;
-      const double t = hi ? 0.0 : t0;
-      return (1.0 - t) * Lr(idx) + t * Lr(idx + 1);
-    };
-    // kPixU pixels a step: their gathers are issued together, and the next
-    // step's pixel loads before them, so a step waits for one memory
-    // latency, not two; the terms are added in pixel order as a one-pixel
-    // loop would
-    constexpr uint32_t kStep = static_cast<uint32_t>(kPixU) * kPixThreads;
-    constexpr uint32_t kLast = static_cast<uint32_t>(kPixU - 1) * kPixThreads;
-    uint32_t i = threadIdx.x;
-    double cf[kPixU];
-    if (i + kLast < cnt) {
-#pragma unroll
-      for (int u = 0; u < kPixU; ++u) cf[u] = pix(i + u * kPixThreads);
+  for (int st = blk * (kPixThreads / 64) + (threadIdx.x >> 6); st < nstep;
+       st += kPixBlocks * (kPixThreads / 64)) {
+    if (st >= nchunk) {
+      // 64 pixels outside the core, as PD::getLogLike takes them: L_0 at or
+      // below minflux, L_N-1 at or above maxflux - dflux
+      const uint32_t k0 = (static_cast<uint32_t>(st - nchunk) << 6) + lane;
+      if (k0 < nout) {
+        const double c = pix[(k0 < pa) ? k0 : k0 - pa + pb].c;
+        const bool lo = c <= minflux, hi = c >= fma(static_cast<double>(N - 2), dflux, minflux);
+        const double d = (lo || hi) ? 0.0 : (c - minflux) * idflux;
+        const uint32_t i = hi ? nm1 : static_cast<uint32_t>(static_cast<int>(d));
+        const double la = Lrot(i);
+        double v = la;
+        if (!lo && !hi) v += (d - static_cast<double>(i)) * (Lrot(i + 1) - la);
+        part += v;
+      }
+      continue;
     }
-    for (; i + kLast < cnt; i += kStep) {
-      double nx[kPixU];
-      const bool more = i + kStep + kLast < cnt;  // the loop's next condition
-#pragma unroll
-      for (int u = 0; u < kPixU; ++u) nx[u] = more ? pix(i + kStep + u * kPixThreads) : 0.0;
-      double tv[kPixU];
-#pragma unroll
-      for (int u = 0; u < kPixU; ++u) tv[u] = term(cf[u]);
-#pragma unroll
-      for (int u = 0; u < kPixU; ++u) part += tv[u];
-#pragma unroll
-      for (int u = 0; u < kPixU; ++u) cf[u] = nx[u];
+    const int e = e_lo + 63 * st + lane, last = min(63, e_hi - e_lo - 63 * st);
+    const bool on = lane <= last;
+    const double de = static_cast<double>(e);
+    const double fe = fma(de, dflux, minflux);
+    // the rank of the edge among the core's pixels: from the table's bounds
+    uint32_t lo = pa, hi = pa;
+    const double x = (fe - fd.ca) * rstep;
+    if (x >= rend) {
+      lo = hi = pb;
+    } else if (on && x >= 0.0) {
+      const uint32_t xi = static_cast<uint32_t>(x);
+      const uint32_t at = (xi & rmask) * rcols + (xi >> fd.rlog);
+      lo = fd.rank[at];
+      hi = fd.rank[at + rcols];
     }
-    for (; i < cnt; i += kPixThreads) part += term(pix(i));
+    const double L = on ? Lrot(static_cast<uint32_t>(e)) : 0.0;
+    while (lo < hi) {
+      const uint32_t mid = lo + ((hi - lo) >> 1);
+      const bool below = pix[mid].c < fe;
+      lo = below ? mid + 1 : lo;
+      hi = below ? hi : mid;
+    }
+    const uint32_t p1 = __shfl_down(lo, 1);
+    const uint32_t nin = (lane < last) ? p1 - lo : 0u;
+    const long long q = pix[lo].q;
+    const double L1 = __shfl_down(L, 1);
+    const long long q1 = __shfl_down(q, 1);
+    if (nin) {
+      // the edge in the pixels' unit, e dflux in two parts
+      const double ep = de * dflux, er = fma(de, dflux, -ep);
+      const long long fx =
+          __double2ll_rn(minflux * unit) + __double2ll_rn(ep * unit) + __double2ll_rn(er * unit);
+      const long long sum = static_cast<long long>(
+          static_cast<unsigned long long>(q1) - static_cast<unsigned long long>(q) -
+          static_cast<unsigned long long>(nin) * static_cast<unsigned long long>(fx));
+      const double t = static_cast<double>(sum) * tscale;
+      part += static_cast<double>(nin) * L + (L1 - L) * t;
+    }
+    // the core's pixels below f_0 count L_0, those from f_N-2 on L_N-1
+    if (e == 0 && lane == 0) part += static_cast<double>(lo - pa) * L;
+    if (e == N - 2 && lane == last && st == nchunk - 1)
+      part += static_cast<double>(pb - lo) * Lrot(nm1);
   }
   const double s = block_sum(part, red);
   if (threadIdx.x == 0) *out = s;
@@ -2053,19 +2071,13 @@ __global__ void combine1d_kernel(const BeamsetDev bs, const WorkDev wk,
 // Writes the P(D) of (walker, field) as PDFactory::getPD leaves PD::pd_:
 // rotated at the split, normalised, log2 when is_log (debug / parity).
 __global__ void materialize_pd_kernel(const double* pofd, int N, int split,
-                                      double itot, int is_log, int already_log,
-                                      double* out) {
+                                      double itot, int is_log, double* out) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= N) return;
   int j = i + split;
   if (j >= N) j -= N;
-  const double v = pofd[j];
-  if (already_log) {
-    out[i] = v;
-  } else {
-    const double p = v * itot;
-    out[i] = is_log ? log2_or_small(p) : p;
-  }
+  const double p = pofd[j] * itot;
+  out[i] = is_log ? log2_or_small(p) : p;
 }
 
 int launch_loglike1d(const BeamsetDev& bs, const WorkDev& wk_in, int beamset_idx,
@@ -2117,7 +2129,7 @@ int launch_loglike1d(const BeamsetDev& bs, const WorkDev& wk_in, int beamset_idx
                      s, bs, wk, fuse, accumulate, d_loglike, d_status);
   mark(POFD_STAGE_PIXELS);
   if (any_unbinned)
-    hipLaunchKernelGGL(pixels1d_kernel, dim3(kPixBlocks, nwalk, bs.nfields),
+    hipLaunchKernelGGL(pixels1d_kernel, dim3(nwalk, kPixBlocks, bs.nfields),
                        dim3(kPixThreads), 0, s, bs, wk);
   mark(POFD_STAGE_COMBINE);
   if (!fuse)
@@ -2189,12 +2201,11 @@ int launch_prior1d(const BeamsetDev& bs0, const WorkDev& wk0, const PriorDev& pr
 }
 
 int launch_materialize_pd(const double* d_pofd, int N, int split, double itot,
-                          int is_log, int already_log, double* d_out,
-                          void* stream) {
+                          int is_log, double* d_out, void* stream) {
   const int nb = (N + 255) / 256;
   hipLaunchKernelGGL(materialize_pd_kernel, dim3(nb), dim3(256), 0,
                      static_cast<hipStream_t>(stream), d_pofd, N, split, itot,
-                     is_log, already_log, d_out);
+                     is_log, d_out);
   return hipGetLastError() == hipSuccess ? POFD_OK : POFD_E_INTERNAL;
 }
 
