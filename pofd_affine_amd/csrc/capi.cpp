@@ -327,6 +327,74 @@ int upload_pixels(pofd_ctx* c, FieldHost& fh, int N, double dflux, FieldDev& fd)
   return POFD_OK;
 }
 
+// The Kaiser-Bessel window of the windowed transforms, phi(x) = I0(beta
+// sqrt(1 - (x/8)^2)) for |x| <= 8 coarse points, over its transform at zero,
+// Phi(0) = 16 sinh(beta) / beta, and Phi(0) / Phi(nu) at nu = k / nc (Kaiser
+// and Schafer 1980), in long double.  beta = 39: the images at k + nc, 2 nc,
+// ..., over Phi(k) and times the noise factor stay below 1e-16 for every
+// spectral index k up to nc / 4 (38: 2.5e-16; 40: 3e-17, and a larger beta
+// magnifies roundings more where the window's transform is divided out).
+constexpr long double kWinBeta = 39.0L;
+long double window_at(long double x) {
+  const long double t = 1.0L - (x / 8) * (x / 8);
+  if (t < 0) return 0.0L;
+  const long double q = kWinBeta * kWinBeta * t / 4;
+  static const long double phi0 = kWinBeta / (16 * sinhl(kWinBeta));
+  long double term = 1.0L, sum = 1.0L;
+  for (int n = 1; term > sum * 1e-22L; ++n) {
+    term *= q / (static_cast<long double>(n) * n);
+    sum += term;
+  }
+  return sum * phi0;
+}
+// Grids from this size take windows.  Measured per call at 2^14, 2^15 and
+// 2^16, 512 nodes: 256 walkers 110, 120 and 133 us against 107, 140 and 203
+// of the pruned transforms, 4 walkers over four workgroups each 88, 93 and
+// 100 us against 77, 78 and 95: below 2^16 the small calls lose what the
+// large ones gain (the choice may not follow the batch: a walker's bits do
+// not depend on it).
+constexpr uint32_t kWinMinN = 1u << 16;
+int upload_windows(pofd_ctx* c, Beamset& s, int N, const std::vector<uint16_t>& kst) {
+  BeamsetDev& d = s.dev;
+  d.nwin = 0;
+  int rc;
+  const long double pi16 = 16 * acosl(-1.0L), phi0 = sinhl(kWinBeta) / kWinBeta;
+  for (int nc = std::max(4096, N / 32); nc <= pofd::kMaxNc && N / nc >= 8 && d.nwin < 2; nc *= 2) {
+    pofd::WindowDev& w = d.win[d.nwin];
+    w.nc = nc;
+    w.p = N / nc;
+    std::vector<double> h(static_cast<size_t>(w.p) * pofd::kTaps), inv(nc / 2 + 1),
+        invm1(nc / 2 + 1);
+    for (int b = 0; b < w.p; ++b)
+      for (int t = 0; t < pofd::kTaps; ++t)
+        h[b * pofd::kTaps + t] =
+            static_cast<double>(window_at(t - 7 - static_cast<long double>(b) / w.p));
+    for (int k = 0; k <= nc / 2; ++k) {
+      const long double a = pi16 * k / nc;
+      const long double z = kWinBeta * kWinBeta - a * a, r = sqrtl(fabsl(z));
+      const long double phi = (r == 0) ? 1.0L : (z > 0 ? sinhl(r) : sinl(r)) / r;
+      const long double v = phi0 / phi;
+      inv[k] = static_cast<double>(v);
+      invm1[k] = static_cast<double>(v - 1);
+    }
+    if ((rc = upload(c, s, h, &w.h))) return rc;
+    if ((rc = upload(c, s, inv, &w.inv))) return rc;
+    if ((rc = upload(c, s, invm1, &w.invm1))) return rc;
+    const int q = w.p / 4;
+    std::vector<uint32_t> grp(N / q);
+    for (int i = 0; i < N / q; ++i) {
+      const uint16_t* k = kst.data() + i * q;
+      int n = 1;
+      while (n < q && k[n] == k[0]) ++n;
+      grp[i] = k[0] | static_cast<uint32_t>(k[q - 1]) << 12 | static_cast<uint32_t>(n) << 24;
+    }
+    if ((rc = upload(c, s, grp, &w.grp))) return rc;
+    ++d.nwin;
+  }
+  if (!d.nwin) return POFD_OK;
+  return upload(c, s, twiddles(pofd::kMaxNc, pofd::kMaxNc / 2), &d.wc);
+}
+
 int prepare_beamset(pofd_ctx* c, Beamset& s) {
   const pofd::Beam& bm = s.beam;
   const uint32_t N = c->nflux, ninterp = c->ninterp;
@@ -569,6 +637,39 @@ int prepare_beamset(pofd_ctx* c, Beamset& s) {
       kst[b] = static_cast<uint16_t>(ninterp + bsearch_idx(xnode.data() + ninterp, ninterp, cf));
     }
   }
+  // the windowed transform takes the coefficients of a lane's first and last
+  // point for all of its eight (four) points; groups that lie in more than
+  // those two intervals (fluxes near zero, where the nodes are closer than
+  // the grid) are made ahead, into a table of kRlow points.  Where that does
+  // not reach, no window is used.
+  auto filled = [&](long j) {
+    return (j >= minit && j <= maxit) || (j >= minitn && j <= maxitn);
+  };
+  auto more = [&](uint32_t j, uint32_t n) {
+    bool second = false, bad = false;
+    for (uint32_t e = 1; e < n; ++e) {
+      second = second || kst[j + e] != kst[j];
+      // past the first interval every filled point is the last's, and no
+      // group holds filled points of both signs' fluxes
+      if (filled(j + e))
+        bad = bad || (second && kst[j + e] != kst[j + n - 1]) ||
+              (static_cast<int>(j) <= wrapRidx && static_cast<int>(j + e) > wrapRidx);
+    }
+    return bad;
+  };
+  int rlow = 0, rlown = 0;
+  bool windows = true;
+  for (uint32_t j = 0; j < N; j += 8) {
+    if (!(more(j, 8) || more(j, 4) || more(j + 4, 4) || more(j, 2) || more(j + 2, 2) ||
+          more(j + 4, 2) || more(j + 6, 2)))
+      continue;
+    if (j < static_cast<uint32_t>(pofd::kRlow))
+      rlow = static_cast<int>(j) + 8;
+    else if (N - j <= static_cast<uint32_t>(pofd::kRlow))
+      rlown = std::max(rlown, static_cast<int>(N - j));
+    else
+      windows = false;
+  }
   const uint32_t M = N / 2, M2 = M / pofd::kM1;
 
   BeamsetDev& d = s.dev;
@@ -589,6 +690,8 @@ int prepare_beamset(pofd_ctx* c, Beamset& s) {
   d.minitn = static_cast<int>(minitn);
   d.maxitn = static_cast<int>(maxitn);
   d.wrapRidx = wrapRidx;
+  d.rlow = rlow;
+  d.rlown = rlown;
   d.dflux = dflux;
   d.minflux_R = minflux_R;
   d.mval = mval;
@@ -617,6 +720,7 @@ int prepare_beamset(pofd_ctx* c, Beamset& s) {
   if ((rc = upload(c, s, w256, &d.W256))) return rc;
   if ((rc = upload(c, s, wlo, &d.Wlo))) return rc;
   if ((rc = upload(c, s, wm2, &d.Wm2))) return rc;
+  if (windows && N >= kWinMinN && (rc = upload_windows(c, s, static_cast<int>(N), kst))) return rc;
   // W_N^t - 1 for t in [0, N/2] (the rest by conjugate symmetry), formed
   // without cancellation as (-2 sin^2(pi t/N), -sin(2 pi t/N)) in long
   // double: the direct sums over the head of the grid use it
@@ -1315,15 +1419,14 @@ extern "C" int pofd1d_get_pd(pofd_ctx* c, uint32_t walker, int b, int f,
   const int N = s.dev.N;
   std::unique_ptr<DevBuf> out;
   if ((rc = dev_alloc(c, out, N * sizeof(double)))) return rc;
-  const double* pofd = s.wk.pofd + (static_cast<size_t>(walker) * s.dev.nfields + f) * s.wk.pofd_stride;
   if (rec[18] != 0.0 && is_log <= 0)
     return fail(c, POFD_E_ARG,
                 "pofd1d_get_pd: unbinned fields give only the log2 P(D)");
   // is_log < 0: the clamped, unrotated, unnormalised transform output
   const int split = (is_log < 0) ? 0 : static_cast<int>(rec[0]);
   const double itot = (is_log < 0) ? 1.0 : rec[16];
-  rc = pofd::launch_materialize_pd(pofd, N, split, itot, is_log > 0 ? 1 : 0,
-                                   static_cast<double*>(out->p), nullptr);
+  rc = pofd::launch_materialize_pd(s.dev, s.wk, static_cast<int>(walker), f, split, itot,
+                                   is_log > 0 ? 1 : 0, static_cast<double*>(out->p), nullptr);
   if (rc) return fail(c, rc, "pofd1d_get_pd: launch failed");
   hipError_t e = hipMemcpy(pd_out, out->p, N * sizeof(double), hipMemcpyDeviceToHost);
   if (e != hipSuccess) return hip_fail(c, e, "hipMemcpy(pd)");

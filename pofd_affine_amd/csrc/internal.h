@@ -81,6 +81,22 @@ struct FieldDev {
 
 constexpr int kMaxFields = 16;
 
+// The windowed transforms (pofd1d_kernel.hip): kTaps-point windows onto a
+// grid of nc = N / p points, kStrips strips of nc / kStrips points each.
+constexpr int kTaps = 16;
+constexpr int kStrips = 256;
+constexpr int kMaxNc = 8192;
+constexpr int kRlow = 2048;
+struct WindowDev {
+  int nc, p;          // coarse points, fine points per coarse point (4-32)
+  const double* h;    // p x kTaps: phi(d - 7 - b/p) at [b * kTaps + d]
+  const double* inv;  // nc/2 + 1: Phi(0) / Phi(k), 1 at k = 0
+  const double* invm1;  // the same less one
+  // N / (p/4) words, one for p/4 grid points: the node intervals of the
+  // first and of the last (12 bits each), the points in the first (8 bits)
+  const uint32_t* grp;
+};
+
 // Everything the kernels need for one beam set; theta-independent.
 struct BeamsetDev {
   int N;        // nflux
@@ -121,6 +137,7 @@ struct BeamsetDev {
   const double* bw;       // nbeam+nbeamn weights (1.0 for a raw beam)
   const double* bieta;    // nbeam+nbeamn inverse |beam| values
   const uint16_t* kst;    // N: segment*ninterp + node interval of every grid flux
+                          // (at most 4096: 12 bits)
   const double2* W256;    // 256: exp(-2 pi i s/256)
   const double2* Wlo;     // 256: exp(-2 pi i s/M)
   const double2* Wm2;     // M2: exp(-2 pi i s/M2)
@@ -130,6 +147,12 @@ struct BeamsetDev {
   // largest values (fluxes near zero); they are left out of the transform
   // and their part of R^(k) - R^(0) is summed directly (forward_tail)
   int headn, headneg;
+  // below rlow (and within rlown of the grid's end, with a negative beam)
+  // eight grid points may lie in more than two node intervals; at most kRlow
+  int rlow, rlown;
+  int nwin;               // windows, by growing nc (0: none fits N)
+  WindowDev win[2];
+  const double2* wc;      // kMaxNc/2: exp(-2 pi i t/kMaxNc)
   int nfields;
   FieldDev fields[kMaxFields];
 };
@@ -236,6 +259,6 @@ int launch_pd_loglike2d(const double* d_pd, int n1, int n2, double minflux1, dou
 // address on `device` (current) once, then look it up (nullptr: none)
 int noalloc_init(int device);
 void* noalloc_scratch(int device);
-int launch_materialize_pd(const double* d_pofd, int N, int split, double itot,
-                          int is_log, double* d_out, void* stream);
+int launch_materialize_pd(const BeamsetDev& bs, const WorkDev& wk, int walker, int f, int split,
+                          double itot, int is_log, double* d_out, void* stream);
 }  // namespace pofd

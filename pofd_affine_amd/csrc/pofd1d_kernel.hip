@@ -108,7 +108,8 @@ __device__ __forceinline__ double qnan() {
 // per-walker scalars handed between the launches (WorkDev::state)
 enum {
   ST_STATUS = 0, ST_SIGMULT, ST_MN, ST_VAR, ST_SHIFT, ST_DOSHIFT, ST_KMAXB,
-  ST_NROWS, ST_R0, ST_TPREP, ST_TFWD, ST_TSPEC
+  ST_NROWS, ST_R0, ST_TPREP, ST_TFWD, ST_TSPEC,
+  ST_WIN  // the window of the transforms + 1, 0 for the pruned ones
 };
 
 // ---- block-wide reductions (deterministic fixed trees) -------------------
@@ -226,10 +227,11 @@ __device__ void block_argmin(double& v, int& idx, double* red) {
 // The 32-value block statistics of the P(D): block b = j / kBlk (kBlk = 2
 // kChunk, so row n1 = b / nbc and chunk c = b % nbc of the inverse transform,
 // nbc = M2 / kChunk) is stored at c * kM1 + n1, so that the 16 rows of a
-// wavefront's epilogue store whole 128-byte lines
+// wavefront's epilogue store whole 128-byte lines.  The windowed transform's
+// blocks are 16 coarse rows, in order (nbc = 0).
 static_assert(kBlk == 2 * kChunk, "a block is one row of one chunk");
 __device__ __forceinline__ int blk_slot(const int b, const int nbc) {
-  return (b % nbc) * kM1 + b / nbc;
+  return nbc ? (b % nbc) * kM1 + b / nbc : b;
 }
 
 // ---- 256-point transforms of 16 swizzled LDS columns ----------------------
@@ -390,6 +392,53 @@ __device__ int spectral_rows(const BeamsetDev& bs, double sigmult, short* rowk2,
   return lo_rows + (M2 - h0);
 }
 
+// P(D) at grid point j from the coarse P(D): sum_d u[a + d - 7] phi(d - 7 -
+// b/p), j = p a + b, in ascending d.  The matrix instructions of the
+// windowed inverse round exactly so (checked on gfx950: v_mfma_f64_16x16x4
+// adds its four products in order, each with one rounding), so a value is
+// the same bits wherever it is made, and none of the N is stored.  uw[i] =
+// u[i - 7]; ht the window by tap, ht[d p + b]; lp = log2 p.
+__device__ __forceinline__ double window_value(const double* uw, const double* ht, const int lp,
+                                               const int j) {
+  const int a = j >> lp, b = j & ((1 << lp) - 1);
+  double v = 0.0;
+#pragma unroll
+  for (int d = 0; d < kTaps; ++d) v = fma(uw[a + d], ht[(d << lp) + b], v);
+  return fmax(v, 0.0);  // unwrapAndNormalizePD positivity
+}
+// the window by tap into LDS (p x kTaps values)
+__device__ __forceinline__ void load_window(const WindowDev& win, double* ht) {
+  for (int i = threadIdx.x; i < win.p * kTaps; i += blockDim.x)
+    ht[(i % kTaps) * win.p + i / kTaps] = win.h[i];
+}
+// the coarse P(D) of (walker, dataset f): where forward_tail left it
+__device__ __forceinline__ const double* coarse_pd(const BeamsetDev& bs, const WorkDev& wk,
+                                                   const int walker, const int f) {
+  return reinterpret_cast<const double*>(wk.zrows + walker * wk.zrows_stride +
+                                         static_cast<size_t>(1 + f) * bs.M);
+}
+
+// The window whose coarse grid holds the spectrum (index + 1, or 0: the
+// pruned transforms).  A window's nc must be at least four times the
+// largest kept index, and four times the index where the narrowest
+// dataset's noise factor is 2^-64 whatever the cut: the images of the
+// window rely on that factor beyond nc / 8 or so.
+__device__ int select_window(const BeamsetDev& bs, const double sigmult, int& kmaxb) {
+  kmaxb = 0;
+  if (!bs.nwin) return 0;
+  double smin = INFINITY;
+  for (int f = 0; f < bs.nfields; ++f) {
+    const double sigma = sigmult * bs.fields[f].sigma_base;
+    smin = fmin(smin, sigma);
+    kmaxb = max(kmaxb, spectral_kmax(sigma, bs.iflux, bs.spectral_cut, bs.M));
+  }
+  if (!(smin > 0.0)) return 0;
+  const double k64 = sqrt(128.0 * 0.69314718055994530942) / (smin * bs.iflux);
+  for (int w = 0; w < bs.nwin; ++w)
+    if (4 * kmaxb <= bs.win[w].nc && 4.0 * k64 <= bs.win[w].nc) return w + 1;
+  return 0;
+}
+
 __device__ __forceinline__ int batch_n(const WorkDev& wk) {
   return wk.dcount ? *wk.dcount : wk.nhost;
 }
@@ -432,6 +481,19 @@ struct XformSmem {
   int isc[2 + kMaxFields];  // nrows, kmaxb, then kmax of each dataset
 };
 
+constexpr int kCHead = 64;  // coarse points of the head (see put_coarse)
+struct WindowSmem {
+  double2 bufa[kMaxNc / 2 + 8];
+  double2 bufb[kMaxNc / 2 + 8];
+  double2 tw[kMaxNc / 8];  // exp(-2 pi i t / (nc/2)), t < nc/8
+  double ch[2 * kCHead + 32];  // the coarse head, then its block sums
+  double hd[1168];             // the grid's head (head_layout)
+  double red[kWaves * 2];
+  double ex2[32];
+  double h[32 * kTaps];  // the window
+  int isc[2 + kMaxFields];
+};
+
 __device__ void load_twiddles(const BeamsetDev& bs, XformSmem& sm) {
   for (int i = threadIdx.x; i < kM1; i += blockDim.x) sm.wlo[i] = bs.Wlo[i];
   for (int i = threadIdx.x; i < 3 * kStageTw; i += blockDim.x) {
@@ -443,25 +505,30 @@ __device__ void load_twiddles(const BeamsetDev& bs, XformSmem& sm) {
   for (int i = threadIdx.x; i < bs.M2; i += blockDim.x) sm.wm2[i] = bs.Wm2[i];
 }
 
-// 2^s * scale by Tang's table-driven method (ACM TOMS 15:144, 1989):
-// 32 s = 32 n + j + 32 r with |r| <= 1/64, 2^s = 2^n 2^(j/32) 2^r, the table
-// entries tab[j] = 2^(j/32) * scale (the fill's scale is dflux) and
-// 2^r = exp(r ln 2) as its Taylor polynomial of degree 6 (truncation below
-// 4e-18 relative).  Accurate to about one ulp; 0 below 2^-1075 and +inf
-// above 2^1024 as exp2 gives them.
-__device__ __forceinline__ double exp2_dflux(double s, const double* tab) {
-  const double t = fmin(fmax(s * 32.0, -35000.0), 33000.0);
+// 2^(u/32) = exp(u ln 2 / 32) for |u| <= 1/2 as its Taylor polynomial of
+// degree 6 (truncation below 4e-18 relative)
+__device__ __forceinline__ double exp2_near(const double u) {
+  double p = 0x1p-30 * 1.5403530393381609954e-4;      // (ln 2)^6 / 720
+  p = fma(p, u, 0x1p-25 * 1.3333558146428443423e-3);  // (ln 2)^5 / 120
+  p = fma(p, u, 0x1p-20 * 9.6181291076284771620e-3);  // (ln 2)^4 / 24
+  p = fma(p, u, 0x1p-15 * 5.5504108664821579953e-2);  // (ln 2)^3 / 6
+  p = fma(p, u, 0x1p-10 * 2.4022650695910071233e-1);  // (ln 2)^2 / 2
+  p = fma(p, u, 0x1p-5 * 6.9314718055994530942e-1);   // ln 2
+  return fma(p, u, 1.0);
+}
+
+// 2^(t/32) * scale by Tang's table-driven method (ACM TOMS 15:144, 1989):
+// t = 32 n + j + u with |u| <= 1/2, 2^(t/32) = 2^n 2^(j/32) 2^(u/32), the
+// table entries tab[j] = 2^(j/32) * scale (the fill's scale is dflux).
+// Accurate to about one ulp; 0 for t below -34400 and NaN, +inf above (the
+// conversion to int saturates).  The node splines' coefficients are kept in
+// these units of 1/32 (node_spline).
+__device__ __forceinline__ double exp2_dflux(double t, const double* tab) {
+  t = fmax(t, -35000.0);
   const double n = rint(t);
-  const double r = (t - n) * 0.03125;
-  const int ni = static_cast<int>(n);
-  double p = 1.5403530393381609954e-4;   // (ln 2)^6 / 720
-  p = fma(p, r, 1.3333558146428443423e-3);  // (ln 2)^5 / 120
-  p = fma(p, r, 9.6181291076284771620e-3);  // (ln 2)^4 / 24
-  p = fma(p, r, 5.5504108664821579953e-2);  // (ln 2)^3 / 6
-  p = fma(p, r, 2.4022650695910071233e-1);  // (ln 2)^2 / 2
-  p = fma(p, r, 6.9314718055994530942e-1);  // ln 2
-  p = fma(p, r, 1.0);
-  return ldexp(tab[ni & 31] * p, ni >> 5);
+  const double u = t - n;
+  const int ni = __double2int_rn(t);
+  return ldexp(tab[ni & 31] * exp2_near(u), ni >> 5);
 }
 
 }  // namespace
@@ -554,10 +621,11 @@ __device__ void node_spline(const BeamsetDev& bs, const WorkDev& wk, const int w
     const double dx = xnode[k + 1] - xnode[k];
     const double dy = sm.yn[k + 1] - sm.yn[k];
     double* cf = coef + 4 * k;
-    cf[0] = sm.yn[k];
-    cf[1] = (dy / dx) - dx * (c_ip1 + 2.0 * c_i) / 3.0;
-    cf[2] = c_i;
-    cf[3] = (c_ip1 - c_i) / (3.0 * dx);
+    // (times 32, exactly: the units of exp2_dflux)
+    cf[0] = 32.0 * sm.yn[k];
+    cf[1] = 32.0 * ((dy / dx) - dx * (c_ip1 + 2.0 * c_i) / 3.0);
+    cf[2] = 32.0 * c_i;
+    cf[3] = 32.0 * ((c_ip1 - c_i) / (3.0 * dx));
   }
   __syncthreads();  // LDS reused by the next segment
 }
@@ -668,6 +736,9 @@ __global__ __launch_bounds__(kThreads) void prep1d_kernel(
       if (part == 0) {
         st[ST_STATUS] = status;
         st[ST_SIGMULT] = sigmult;
+        int kmaxb = 0;
+        st[ST_WIN] = (status == POFD_OK) ? select_window(bs, sigmult, kmaxb) : 0;
+        st[ST_KMAXB] = kmaxb;
       }
       sm.isc[0] = status;
       sm.isc[1] = valid ? 1 : 0;
@@ -862,13 +933,10 @@ __device__ __forceinline__ double2 em1_add(const double2 a, const double2 b) {
 // starts from the table at a_lo and steps by E(8k) (em1_add): a run of at
 // most a few steps adds a few roundings of |E(8ak)|.  8 k a < 2^31 for
 // k <= N/2 and a < 2^11.
-__device__ double2 head_sum(const BeamsetDev& bs, const double2* elo, const double2* ehi,
-                            const double* g, const double* vsum, const int a_lo, const int a_hi,
-                            const int k, const double2* eb, const double2 e8) {
+// (ea: E(8k a_lo))
+__device__ double2 head_sum(const double* g, const double* vsum, const int a_lo, const int a_hi,
+                            const double2* eb, const double2 e8, double2 ea) {
   double2 acc = make_double2(0.0, 0.0);
-  if (a_lo >= a_hi) return acc;
-  double2 ea = em1_at(bs, elo, ehi, static_cast<uint32_t>(kHeadBlk) *
-                                        static_cast<uint32_t>(k) * static_cast<uint32_t>(a_lo));
   for (int a = a_lo; a < a_hi; ++a) {
     const double* ga = g + kHeadBlk * a;
     double2 u = make_double2(0.0, 0.0);
@@ -886,22 +954,665 @@ __device__ double2 head_sum(const BeamsetDev& bs, const double2* elo, const doub
   return acc;
 }
 
+// ---- the windowed transforms ------------------------------------------------
+// Only spectral indices k <= kmax << N/2 survive the noise factor, so R is
+// first brought onto a coarse grid of nc = N / p points by a window phi of
+// kTaps coarse points (c_m = sum_j phi(m - j/p) R_j), transformed there, and
+// divided by the window's own transform: R^(k) = c^(k) / Phi(k), as in the
+// non-uniform transforms (Dutt and Rokhlin, SIAM J. Sci. Comput. 14:1368,
+// 1993), with a Kaiser-Bessel window whose images stay below 1e-16.  The
+// inverse is the transpose: the noisy spectrum over Phi(k), a transform of
+// length nc, and P_j = sum_m phi(m - j/p) u_m.  Both sums are contractions
+// over the 16 taps or the p fine points and run on the FP64 matrix cores
+// from registers: no column transform, no twiddles, no barrier and no LDS
+// traffic for the N values.  In rounding it is the better transform too (the
+// sums of neighbours are positive and local): P(D) within 1e-15 of its peak
+// of the extended-precision value, where the pruned and plain double
+// transforms are at 6e-15.
+//
+// Complex transform of length n (a power of two) in LDS, radix-4 Stockham
+// with a radix-2 stage first when log2 n is odd; the result is left in the
+// returned buffer.  tw[turn_at(t)] = exp(-2 pi i t/n), t < n/4.  Called by
+// every thread, which has synchronised.
+// Element i is at coarse_at(i): the stages write at strides of 4, 8, 16 and
+// 32 elements between neighbours of 16 lanes, and read consecutive ones; the
+// exclusive-or of bits 4 and 5 into bits 0 to 3 keeps each of these patterns
+// on distinct banks.  turn_at does the same for the twiddles, read at a
+// stride of n / 4 Ns.  (n = 2048 takes 3.6 us, 4.1 in plain order: address
+// arithmetic and the barriers bound it, not the banks.)
+__device__ __forceinline__ int coarse_at(const int i) {
+  const int t = (i >> 4) & 3;
+  return i ^ t ^ (t << 2);
+}
+__device__ __forceinline__ int turn_at(const int t) { return t ^ ((t >> 4) & 15) ^ (t >> 8); }
+__device__ double2* fft_coarse(double2* a, double2* b, const int n, const double2* tw) {
+  double2* src = a;
+  double2* dst = b;
+  int Ns = 1;
+  if (__builtin_ctz(static_cast<unsigned>(n)) & 1) {
+    const int h = n >> 1;
+    for (int j = threadIdx.x; j < h; j += kThreads) {
+      const double2 v0 = src[coarse_at(j)], v1 = src[coarse_at(j + h)];
+      dst[coarse_at(2 * j)] = cadd(v0, v1);
+      dst[coarse_at(2 * j + 1)] = csub(v0, v1);
+    }
+    __syncthreads();
+    double2* t = src;
+    src = dst;
+    dst = t;
+    Ns = 2;
+  }
+  const int q = n >> 2;
+  // exp(-2 pi i t/n) for t < n/4, and beyond by quarter turns
+  auto turn = [&](const int t) { return tw[turn_at(t)]; };
+  auto quarter = [](const double2 v, const bool on) {
+    return on ? make_double2(v.y, -v.x) : v;
+  };
+  for (; Ns < n; Ns *= 4) {
+    const int ts = n / (4 * Ns);
+    for (int j = threadIdx.x; j < q; j += kThreads) {
+      const int jm = j & (Ns - 1);
+      // (q is a multiple of 64)
+      const double2* sj = src + coarse_at(j);
+      double2 v0 = sj[0], v1 = sj[q], v2 = sj[2 * q], v3 = sj[3 * q];
+      if (Ns > 1) {
+        const int t1 = jm * ts, t2 = 2 * t1, t3 = 3 * t1;  // t1 < n/4
+        v1 = cmul(v1, turn(t1));
+        v2 = quarter(cmul(v2, turn(t2 & (q - 1))), t2 & q);
+        v3 = cmul(v3, turn(t3 & (q - 1)));
+        v3 = quarter(v3, t3 & q);
+        if (t3 & (2 * q)) v3 = make_double2(-v3.x, -v3.y);
+      }
+      const double2 a0 = cadd(v0, v2), a1 = csub(v0, v2);
+      const double2 a2 = cadd(v1, v3), a3 = csub(v1, v3);
+      const double2 ya = make_double2(a1.x + a3.y, a1.y - a3.x);
+      const double2 yb = make_double2(a1.x - a3.y, a1.y + a3.x);
+      const int d = (j - jm) * 4 + jm;
+      dst[coarse_at(d)] = cadd(a0, a2);
+      dst[coarse_at(d + Ns)] = ya;
+      dst[coarse_at(d + 2 * Ns)] = csub(a0, a2);
+      dst[coarse_at(d + 3 * Ns)] = yb;
+    }
+    __syncthreads();
+    double2* t = src;
+    src = dst;
+    dst = t;
+  }
+  return src;
+}
+
+// v of the lane before in a row of 16 (0 in the row's first lane)
+__device__ __forceinline__ double row_shift(const double v) {
+  const unsigned long long u = static_cast<unsigned long long>(__double_as_longlong(v));
+  const int lo = __builtin_amdgcn_update_dpp(0, static_cast<int>(static_cast<unsigned>(u)), 0x111,
+                                             0xf, 0xf, true);
+  const int hi = __builtin_amdgcn_update_dpp(0, static_cast<int>(static_cast<unsigned>(u >> 32)),
+                                             0x111, 0xf, 0xf, true);
+  return __longlong_as_double(
+      static_cast<long long>((static_cast<unsigned long long>(static_cast<unsigned>(hi)) << 32) |
+                             static_cast<unsigned>(lo)));
+}
+
+// R on the coarse grid, this part's strips, and this thread's share of the
+// moments.  Strip s holds coarse rows a in [s nl, (s + 1) nl), nl = nc /
+// kStrips, of p = 4 Q fine points each; a wavefront takes 16 strips, one row
+// of each a step: lane (lj, lk) makes R at the Q fine points from Q lk of
+// row a of strip lj, the A operand of Q v_mfma_f64_16x16x4_f64 steps against
+// the window, B[b][j] = phi(8 - j - b/p).  Column j of the accumulator is
+// the running sum of coarse point a + 8 - j: it moves one lane on between
+// the steps, and column 15 is the finished point a - 7.  The first 15 points
+// of a strip miss the rows before it and go to pre[strip][t]; what the last
+// 15 miss are the next strip's.  c[i] is coarse point i + 8, i counted from
+// the part's first row.
+// Near zero flux neighbouring points lie in different node intervals, and a
+// lane would wait for its coefficients at every point: those values come
+// from the table rl that all threads made before (R(j) at j, R(N - v) at
+// kRlow + v).
+// Bound by the VALU work of R (26 instructions a point); the matrix cores
+// are busy for half of that, in its shadow.  With the tail 103 us for 256
+// walkers at 2^17, where the pruned transform took 193 (its column
+// transforms through LDS, a barrier a stage).
+template <int Q>
+__device__ __forceinline__ void forward_window(const BeamsetDev& bs, const WindowDev& win,
+                                               const double* __restrict__ coef, WindowSmem& sm,
+                                               const int part, const int parts, double& mn_part,
+                                               double& var_part) {
+  constexpr int p = 4 * Q;
+  const int tid = threadIdx.x;
+  const int lj = tid & 15, lk = (tid >> 4) & 3, wv = tid >> 6;
+  const int nw = kWaves / parts, nl = win.nc / kStrips;
+  if (wv >= nw) return;
+  double* c = reinterpret_cast<double*>(sm.bufa);
+  double* pre = reinterpret_cast<double*>(sm.bufb);
+  const double* rl = pre + kStrips * kTaps;
+  const int s0 = 16 * wv;                       // first strip, in the part
+  const int strip = 16 * (part * nw + wv) + lj;  // this lane's A row
+  f64x4 acc = {0.0, 0.0, 0.0, 0.0};
+  const double dflux = bs.dflux;
+  const int wr = bs.wrapRidx, lastn = bs.N - 1;
+  const int jrow = p * nl * strip + Q * lk;
+  // the node intervals of a step's Q points: the first's (12 bits), the
+  // last's (12 bits) and the number of points in the first
+  const uint32_t* grp = win.grp + jrow / Q;
+  struct Node {
+    double x;
+    double4 cf;
+  };
+  auto node = [&](const uint32_t k) {
+    return Node{bs.xnode[k], *reinterpret_cast<const double4*>(coef + 4 * k)};
+  };
+  uint32_t g = grp[0], gn = grp[4 * min(1, nl - 1)];
+  Node na = node(g & 0xfffu), nb = node((g >> 12) & 0xfffu);
+  for (int t = 0; t < nl; ++t) {
+    const int j0 = jrow + p * t;
+    const double jd = static_cast<double>(j0);
+    double rv[Q];
+    {
+      const double off = (bs.headneg && j0 > wr) ? bs.mval : 0.0;
+      const int ns = static_cast<int>(g >> 24);
+      const double da = fma(jd, dflux, off - na.x);
+#pragma unroll
+      for (int e = 0; e < Q; ++e) {
+        const double d = da + e * dflux;
+        rv[e] = na.cf.x + d * (na.cf.y + d * (na.cf.z + d * na.cf.w));
+      }
+      if (__any(ns < Q)) {
+        const double db = fma(jd, dflux, off - nb.x);
+#pragma unroll
+        for (int e = 1; e < Q; ++e) {
+          const double d = db + e * dflux;
+          const double sb = nb.cf.x + d * (nb.cf.y + d * (nb.cf.z + d * nb.cf.w));
+          rv[e] = (e < ns) ? rv[e] : sb;
+        }
+      }
+    }
+    // the next step's coefficients, in flight from here
+    g = gn;
+    na = node(g & 0xfffu);
+    nb = node((g >> 12) & 0xfffu);
+    gn = grp[4 * min(t + 2, nl - 1)];
+    // the window from LDS (held in registers it would spill the rest: the
+    // offset through an empty asm, so that the loads stay in the loop)
+    int ho = Q * lk * kTaps + 15 - lj;
+    asm volatile("" : "+v"(ho));
+    const double* hw = sm.h + ho;
+#pragma unroll
+    for (int rr = 0; rr < 4; ++rr) acc[rr] = row_shift(acc[rr]);
+    // near zero flux R is in the table, and the head of the grid is summed
+    // directly (forward_tail); a wavefront with none of those points, all of
+    // them in the positive fill range and below wrapRidx - 1, needs no test
+    // and takes the plain terms of the moments
+    const bool tab = j0 < bs.rlow, tabn = j0 >= bs.N - bs.rlown;
+    const bool head = j0 < bs.headn || (bs.headneg && j0 >= bs.N - bs.headn);
+    const bool plain = !tab && !tabn && !head && j0 >= 1 && j0 >= bs.minit &&
+                       j0 + Q - 1 <= bs.maxit && (j0 + Q - 1 < bs.minitn || j0 > bs.maxitn) &&
+                       j0 + Q - 1 < wr - 1;
+    if (__all(plain)) {
+      // with the points within 2^(1/64) of the middle one (all but the
+      // steepest), one full exponential for the lot
+      const double tc = rv[Q / 2];
+      double s0 = 0.0, s1 = 0.0, s2 = 0.0;
+      if (__all(fabs(rv[0] - tc) <= 0.5 && fabs(rv[Q - 1] - tc) <= 0.5)) {
+        const double rc = exp2_dflux(tc, sm.ex2);
+#pragma unroll
+        for (int e = 0; e < Q; ++e) {
+          const double r = (e == Q / 2) ? rc : rc * exp2_near(rv[e] - tc);
+          acc = __builtin_amdgcn_mfma_f64_16x16x4f64(r, hw[e * kTaps], acc, 0, 0, 0);
+          s0 += r;
+          s1 = fma(static_cast<double>(e), r, s1);
+          s2 = fma(static_cast<double>(e * e), r, s2);
+        }
+      } else {
+#pragma unroll
+        for (int e = 0; e < Q; ++e) {
+          const double r = exp2_dflux(rv[e], sm.ex2);
+          acc = __builtin_amdgcn_mfma_f64_16x16x4f64(r, hw[e * kTaps], acc, 0, 0, 0);
+          s0 += r;
+          s1 = fma(static_cast<double>(e), r, s1);
+          s2 = fma(static_cast<double>(e * e), r, s2);
+        }
+      }
+      // sum f R and sum f^2 R, f = (j0 + e) dflux
+      const double f0 = jd * dflux;
+      const double m1 = dflux * s1;
+      mn_part += fma(f0, s0, m1);
+      var_part += fma(f0, fma(f0, s0, m1 + m1), dflux * dflux * s2);
+    } else {
+#pragma unroll
+      for (int e = 0; e < Q; ++e) rv[e] = exp2_dflux(rv[e], sm.ex2);
+      if (tab || tabn) {
+#pragma unroll
+        for (int e = 0; e < Q; ++e) rv[e] = rl[tab ? j0 + e : kRlow + bs.N - j0 - e];
+      }
+#pragma unroll
+      for (int e = 0; e < Q; ++e) {
+        const int j = j0 + e;
+        if (!((j >= bs.minitn && j <= bs.maxitn) || (j >= bs.minit && j <= bs.maxit)))
+          rv[e] = 0.0;
+        // getMeanVarFromR (src/PDFactory.cc:625-679); the point 0 adds zero
+        const double cfl = (j <= wr) ? static_cast<double>(j) * dflux
+                                     : static_cast<double>(j - wr - 1) * dflux + bs.minflux_R;
+        const double prod = ((j == wr) ? 0.5 * cfl : cfl) * rv[e];
+        mn_part += prod;
+        var_part = fma(cfl, prod, var_part);
+        if (j == wr - 1 && wr < lastn) {
+          // the wrap correction reads R[wrapRidx - 1] (src/PDFactory.cc:
+          // 661-668), kept as the reference has it
+          const double cb = bs.minflux_R;
+          const double pb = 0.5 * cb * rv[e];
+          mn_part -= pb;
+          var_part -= cb * pb;
+        }
+        acc = __builtin_amdgcn_mfma_f64_16x16x4f64(head ? 0.0 : rv[e], hw[e * kTaps], acc, 0, 0,
+                                                   0);
+      }
+    }
+    if (lj == 15) {
+      if (t < 15) {
+#pragma unroll
+        for (int rr = 0; rr < 4; ++rr) pre[(s0 + lk + 4 * rr) * kTaps + t] = acc[rr];
+      } else {
+#pragma unroll
+        for (int rr = 0; rr < 4; ++rr) c[(s0 + lk + 4 * rr) * nl + t - 15] = acc[rr];
+      }
+    }
+  }
+  if (lj < 15) {
+#pragma unroll
+    for (int rr = 0; rr < 4; ++rr) c[(s0 + lk + 4 * rr) * nl + nl - 1 - lj] = acc[rr];
+  }
+}
+
+// The coarse points [0, kCHead) and, with a negative beam, [nc - kCHead, nc),
+// where R's window sums are largest, stay out of the coarse transform as the
+// first grid points stay out of either (head sums): point m at ch[m], point
+// nc - v at ch[kCHead + v].
+// coarse point m to its place, c in sm.bufa
+__device__ __forceinline__ void put_coarse(const BeamsetDev& bs, WindowSmem& sm, const int nc,
+                                           const int m, const double v) {
+  const bool lo = m < kCHead, hi = bs.headneg && m >= nc - kCHead;
+  reinterpret_cast<double*>(sm.bufa)[2 * coarse_at(m >> 1) + (m & 1)] = (lo || hi) ? 0.0 : v;
+  if (lo) sm.ch[m] = v;
+  if (hi) sm.ch[kCHead + nc - m] = v;
+}
+
+// where the grid's head is in WindowSmem::hd: R at points [0, headn), at
+// headn + v the point N - v (v <= headn; headneg), then the sums of kHeadBlk
+// consecutive values of each
+struct HeadLayout {
+  double *hp, *hn, *vp, *vn;
+  int nbp, nbn;
+};
+__device__ __forceinline__ HeadLayout head_layout(const BeamsetDev& bs, WindowSmem& sm) {
+  HeadLayout l;
+  const int H = bs.headn;
+  l.nbp = H / kHeadBlk;
+  l.nbn = bs.headneg ? H / kHeadBlk + 1 : 0;
+  l.hp = sm.hd;
+  l.hn = l.hp + H;
+  l.vp = l.hn + H + kHeadBlk;
+  l.vn = l.vp + l.nbp;
+  return l;
+}
+
+// what the tail and the coarse transforms read: the twiddles and the scalars
+__device__ void window_setup(const BeamsetDev& bs, const WindowDev& win, const double* st,
+                             WindowSmem& sm) {
+  const int ts = 2 * kMaxNc / win.nc;
+  for (int t = threadIdx.x; t < win.nc / 8; t += kThreads) sm.tw[turn_at(t)] = bs.wc[t * ts];
+  for (int i = threadIdx.x; i < win.p * kTaps; i += kThreads) sm.h[i] = win.h[i];
+  if (threadIdx.x < 32)
+    sm.ex2[threadIdx.x] = exp2(static_cast<double>(threadIdx.x) * 0.03125) * bs.dflux;
+  if (threadIdx.x == 64) {
+    sm.isc[0] = 0;
+    sm.isc[1] = static_cast<int>(st[ST_KMAXB]);
+  }
+  if (threadIdx.x >= 128 && static_cast<int>(threadIdx.x) < 128 + bs.nfields) {
+    const int f = threadIdx.x - 128;
+    sm.isc[2 + f] = spectral_kmax(st[ST_SIGMULT] * bs.fields[f].sigma_base, bs.iflux,
+                                  bs.spectral_cut, bs.M);
+  }
+}
+// R at the head of the grid (sm.ex2 is there), each side by the part whose
+// points it is of, and the block sums once the caller has synchronised
+__device__ void window_head(const BeamsetDev& bs, const double* coef, const bool pos,
+                            const bool neg, WindowSmem& sm) {
+  const HeadLayout l = head_layout(bs, sm);
+  const int H = bs.headn;
+  if (pos)
+    for (int i = threadIdx.x; i < H; i += kThreads) l.hp[i] = r_grid(bs, coef, i, sm.ex2);
+  if (neg)
+    for (int v = threadIdx.x; v < H + kHeadBlk; v += kThreads)
+      l.hn[v] = (bs.headneg && v >= 1 && v <= H) ? r_grid(bs, coef, bs.N - v, sm.ex2) : 0.0;
+}
+__device__ void window_head_sums(const BeamsetDev& bs, WindowSmem& sm) {
+  const HeadLayout l = head_layout(bs, sm);
+  for (int a = threadIdx.x; a < l.nbp + l.nbn; a += kThreads) {
+    const double* g = (a < l.nbp) ? l.hp + kHeadBlk * a : l.hn + kHeadBlk * (a - l.nbp);
+    double v = 0.0;
+    for (int b = 0; b < kHeadBlk; ++b) v += g[b];
+    l.vp[a] = v;  // vn follows vp
+  }
+}
+
+// E(t) = exp(-2 pi i t/N) - 1 from the table of half a turn
+__device__ __forceinline__ double2 em1_load(const BeamsetDev& bs, const uint32_t t) {
+  const int u = static_cast<int>(t & static_cast<uint32_t>(bs.N - 1));
+  const bool lo = u <= bs.M;
+  const double2 e = bs.em1[lo ? u : bs.N - u];
+  return make_double2(e.x, lo ? e.y : -e.y);
+}
+
+// From the coarse points of R (in sm.bufa, their head in sm.ch, the grid's
+// head in sm.hd, all synchronised): the coarse transform, R^(k) - R^(0) with
+// the heads' parts, the spectrum exp(R^ - R^0) and its phase
+// (src/PDFactory.cc:1094-1132), then per dataset the noise factor
+// (:1172-1188) and the coarse P(D) (coarse_pd).
+// 2^hs consecutive lanes share a k for the head sums, as many as keep all
+// indices in one pass.
+// kAhead: the first items' table values are loaded ahead of the transform.
+template <bool kAhead>
+__device__ void window_tail(const BeamsetDev& bs, const WorkDev& wk, const int walker,
+                            WindowSmem& sm, const WindowDev& win, const double mn,
+                            const double var, unsigned long long tmark) {
+  const int tid = threadIdx.x;
+  double* st = walker_state(wk, walker);
+  const double sigmult = st[ST_SIGMULT];
+  const int kmaxb = sm.isc[1];
+  const double sgpos0 = sqrt(var);
+  const bool doshift = (sgpos0 > bs.dflux) && (fabs(mn) > bs.dflux);
+  const double shift = doshift ? -mn : 0.0;
+  const HeadLayout hl = head_layout(bs, sm);
+  // the coarse head's negative side from v = 1, and both sides' block sums
+  constexpr int ncb = kCHead / kHeadBlk;
+  double* ch = sm.ch;
+  double* cn = ch + kCHead;
+  double* cvp = cn + kCHead + kHeadBlk;  // ncb blocks, then ncb + 1
+  if (tid < kCHead + kHeadBlk && (!bs.headneg || tid == 0 || tid > kCHead)) cn[tid] = 0.0;
+  const int h = win.nc / 2, ts = kMaxNc / win.nc;
+  const int hs = (4 * (kmaxb + 1) <= kThreads) ? 2 : ((2 * (kmaxb + 1) <= kThreads) ? 1 : 0);
+  const int nitems = (kmaxb + 1) << hs;
+  // what item `it` reads of the tables
+  struct Item {
+    double2 e1, ea, c1, ca, w;
+    double inv, im1;
+  };
+  auto item = [&](const int it) {
+    const int k = (it < nitems) ? it >> hs : 0, part = it & ((1 << hs) - 1);
+    const uint32_t k8 = static_cast<uint32_t>(kHeadBlk) * static_cast<uint32_t>(k);
+    const int kp = k * win.p;
+    Item t;
+    t.e1 = em1_load(bs, static_cast<uint32_t>(k));
+    t.ea = em1_load(bs, k8 * static_cast<uint32_t>((part * hl.nbp) >> hs));
+    t.c1 = em1_load(bs, static_cast<uint32_t>(kp));
+    t.ca = em1_load(bs, k8 * static_cast<uint32_t>(win.p * ((part * ncb) >> hs)));
+    t.w = bs.wc[k * ts];
+    t.inv = win.inv[k];
+    t.im1 = win.invm1[k];
+    return t;
+  };
+  double2* prtrans = wk.prtrans + walker * wk.spec_stride;
+  // dataset f's entries of the inverse transform's input from the spectrum
+  // pt at k: Zp = E + i O of a half-length transform, with E = X[k] +
+  // conj(X[h - k]), O = (X[k] - conj(X[h - k])) e^{+2 pi i k/nc}, where one of
+  // the two indices is always past the kept ones (kmax <= nc/4, and at nc/4
+  // itself the noise factor is below 2^-64); real and imaginary part exchanged
+  auto put_noisy = [&](const int f, const int k, const double2 pt, const double inv,
+                       const double2 w, double2* dst) {
+    if (k > sm.isc[2 + f]) return;
+    const double sigma = sigmult * bs.fields[f].sigma_base;
+    double ef = 1.0;
+    if (k > 0 && sigma > 0) {
+#pragma clang fp contract(off)
+      const double sigfac = -0.5 * sigma * sigma;
+      const double fk = bs.iflux * static_cast<double>(k);
+      ef = exp(sigfac * fk * fk);
+    }
+    const double g = ef * inv;
+    double2 x = make_double2(g * pt.x, (k == 0) ? 0.0 : g * pt.y);
+    const double2 o = cmulc(x, w);  // X e^{+2 pi i k/nc}
+    dst[coarse_at(k)] = make_double2(x.y + o.x, x.x - o.y);
+    if (k > 0 && 2 * k < h) {
+      // index h - k: E = conj X, D = -conj X, e^{i(pi - a)} = -conj(e^{ia})
+      dst[coarse_at(h - k)] = make_double2(-x.y + o.x, x.x + o.y);
+    }
+  };
+  auto put_zeros = [&](const int f, double2* dst) {  // where nothing is kept
+    const int kf = sm.isc[2 + f];
+    for (int k = kf + 1 + tid; k < h - kf; k += kThreads) dst[coarse_at(k)] = make_double2(0.0, 0.0);
+  };
+  Item im;
+  if (kAhead) im = item(tid);
+  const double2* z = fft_coarse(sm.bufa, sm.bufb, h, sm.tw);
+  double2* zf = (z == sm.bufa) ? sm.bufb : sm.bufa;
+  if (tid < 2 * ncb + 1) {
+    const double* g = ch + kHeadBlk * tid;
+    double v = 0.0;
+    for (int b = 0; b < kHeadBlk; ++b) v += g[b];
+    cvp[tid] = v;
+  }
+  put_zeros(0, zf);
+  __syncthreads();
+  double csum = 0.0;
+  for (int a = 0; a < 2 * ncb + 1; ++a) csum += cvp[a];
+  const double2 z0 = z[0];
+  const double r0 = z0.x + z0.y;  // sum of R outside the heads
+  const double wfac = shift * bs.iflux;
+  for (int it0 = 0; it0 < nitems; it0 += kThreads) {  // uniform trip count
+    const int it = it0 + tid;
+    if (!kAhead || it0 > 0) im = item(it);
+    const bool act = it < nitems;
+    const int k = act ? it >> hs : 0, part = it & ((1 << hs) - 1);
+    double2 dh = make_double2(0.0, 0.0);
+    if (act) {
+      const uint32_t k8 = static_cast<uint32_t>(kHeadBlk) * static_cast<uint32_t>(k);
+      const int kp = k * win.p;  // a coarse point is p grid points
+      const uint32_t kp8 = static_cast<uint32_t>(kHeadBlk) * static_cast<uint32_t>(kp);
+      const int al = (part * hl.nbp) >> hs, ah = ((part + 1) * hl.nbp) >> hs;
+      const int cl = (part * ncb) >> hs, cu = ((part + 1) * ncb) >> hs;
+      double2 eb[kHeadBlk];
+      auto steps = [&](const double2 one) {  // E(b t), b < 8; returns E(8 t)
+        eb[0] = make_double2(0.0, 0.0);
+        eb[1] = one;
+#pragma unroll
+        for (int b = 2; b < kHeadBlk; ++b) eb[b] = em1_add(eb[b - 1], one);
+        return em1_add(eb[kHeadBlk - 1], one);
+      };
+      double2 e8 = steps(im.e1);
+      dh = head_sum(hl.hp, hl.vp, al, ah, eb, e8, im.ea);
+      if (hl.nbn) {
+        const int an = (part * hl.nbn) >> hs, au = ((part + 1) * hl.nbn) >> hs;
+        const double2 dn = head_sum(hl.hn, hl.vn, an, au, eb, e8,
+                                    em1_load(bs, k8 * static_cast<uint32_t>(an)));
+        dh.x += dn.x;  // W^{(N - v) k} - 1 = conj(E(vk))
+        dh.y -= dn.y;
+      }
+      // sum c_m (e(mk) / Phi(k) - 1) = (sum c_m (e(mk) - 1) + sum c_m) /
+      // Phi(k) - sum c_m
+      e8 = steps(im.c1);
+      double2 dc = head_sum(ch, cvp, cl, cu, eb, e8, im.ca);
+      if (hl.nbn) {
+        const int an = (part * (ncb + 1)) >> hs, au = ((part + 1) * (ncb + 1)) >> hs;
+        const double2 dn = head_sum(cn, cvp + ncb, an, au, eb, e8,
+                                    em1_load(bs, kp8 * static_cast<uint32_t>(an)));
+        dc.x += dn.x;
+        dc.y -= dn.y;
+      }
+      const double iv = 1.0 + im.im1;
+      dh.x += dc.x * iv + ((part == 0) ? csum * im.im1 : 0.0);
+      dh.y += dc.y * iv;
+    }
+    for (int o = 1; o < (1 << hs); o <<= 1) {
+      dh.x += __shfl_xor(dh.x, o);
+      dh.y += __shfl_xor(dh.y, o);
+    }
+    if (act && part == 0) {
+      double2 pt = make_double2(1.0, 0.0);
+      if (k > 0) {
+        const double2 zk = z[coarse_at(k)], zm = z[coarse_at(h - k)];
+        const double2 A = make_double2(0.5 * (zk.x + zm.x), 0.5 * (zk.y - zm.y));
+        const double2 B = make_double2(0.5 * (zk.y + zm.y), -0.5 * (zk.x - zm.x));
+        const double2 X = cadd(A, cmul(im.w, B));
+        const double iv = im.inv;
+        double expfac, ival;
+        {
+#pragma clang fp contract(off)
+          expfac = exp((X.x * iv - r0) + dh.x);
+          ival = X.y * iv + dh.y;
+          if (doshift) ival -= wfac * static_cast<double>(k);
+        }
+        double s2, c2;
+        sincos(ival, &s2, &c2);
+        pt = make_double2(expfac * c2, expfac * s2);
+      }
+      prtrans[k] = pt;
+      put_noisy(0, k, pt, im.inv, im.w, zf);
+    }
+  }
+  if (tid >= kThreads - 64) {
+    double vh = 0.0;
+    for (int a = tid & 63; a < hl.nbp + hl.nbn; a += 64) vh += hl.vp[a];
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) vh += __shfl_xor(vh, o);
+    if (tid == kThreads - 1) {
+      st[ST_MN] = mn;
+      st[ST_VAR] = var;
+      st[ST_DOSHIFT] = doshift ? 1.0 : 0.0;
+      st[ST_SHIFT] = shift;
+      st[ST_R0] = r0 + (csum + vh);
+      st[ST_TFWD] = static_cast<double>(wall_clock64() - tmark);
+    }
+  }
+  tmark = wall_clock64();
+  for (int f = 0; f < bs.nfields; ++f) {
+    if (f > 0) {
+      // (each thread reads the spectrum values that it wrote)
+      put_zeros(f, zf);
+      for (int it = tid; it < nitems; it += kThreads)
+        if ((it & ((1 << hs) - 1)) == 0)
+          put_noisy(f, it >> hs, prtrans[it >> hs], win.inv[it >> hs], bs.wc[(it >> hs) * ts], zf);
+    }
+    __syncthreads();
+    const double2* u = fft_coarse(zf, zf == sm.bufa ? sm.bufb : sm.bufa, h, sm.tw);
+    double2* dst = wk.zrows + walker * wk.zrows_stride + static_cast<size_t>(1 + f) * bs.M;
+    for (int m = tid; m < h; m += kThreads) {
+      const double2 v = u[coarse_at(m)];
+      dst[m] = make_double2(v.y, v.x);
+    }
+    __syncthreads();
+  }
+  if (tid == 0) st[ST_TSPEC] = static_cast<double>(wall_clock64() - tmark);
+}
+
+// The windowed forward transform of one walker, split over `parts`
+// workgroups by strips: with one part the workgroup finishes the spectrum
+// itself; with more, each leaves its coarse points and partial moments in
+// its slot and spectrum1d_kernel combines them and finishes.  The strips and
+// the sums are the same either way, and with them the bits.
+__device__ __forceinline__ void forward_windowed(const BeamsetDev& bs, const WorkDev& wk,
+                                                 WindowSmem& sm, const WindowDev& win,
+                                                 const int walker, const int part,
+                                                 const int parts) {
+  const int tid = threadIdx.x;
+  double* st = walker_state(wk, walker);
+  const unsigned long long tmark = wall_clock64();
+  const double* coef = wk.coef + walker * wk.coef_stride;
+  window_setup(bs, win, st, sm);
+  __syncthreads();
+  if (tid == 0 && part == 0) st[ST_NROWS] = 0;
+  double* c = reinterpret_cast<double*>(sm.bufa);
+  double* pre = reinterpret_cast<double*>(sm.bufb);
+  double* rl = pre + kStrips * kTaps;
+  window_head(bs, coef, part == 0, part == parts - 1, sm);
+  if (part == 0)
+    for (int i = tid; i < bs.rlow; i += kThreads) rl[i] = r_grid(bs, coef, i, sm.ex2);
+  if (part == parts - 1)
+    for (int i = tid; i < bs.rlown; i += kThreads)
+      rl[kRlow + i + 1] = r_grid(bs, coef, bs.N - 1 - i, sm.ex2);
+  __syncthreads();
+  double a = 0.0, b = 0.0;
+  auto run = [&](auto q) {
+    forward_window<decltype(q)::value>(bs, win, coef, sm, part, parts, a, b);
+  };
+  switch (win.p) {
+    case 32: run(std::integral_constant<int, 8>{}); break;
+    case 16: run(std::integral_constant<int, 4>{}); break;
+    default: run(std::integral_constant<int, 2>{}); break;
+  }
+  // the moments: each wavefront's, then the tree of groups of four
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) {
+    a += __shfl_xor(a, o);
+    b += __shfl_xor(b, o);
+  }
+  if ((tid & 63) == 0) {
+    sm.red[tid >> 6] = a;
+    sm.red[kWaves + (tid >> 6)] = b;
+  }
+  __syncthreads();
+  double mom[2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const double* r = sm.red + i * kWaves;
+    auto grp = [&](const int g) {
+      return (r[4 * g] + r[4 * g + 1]) + (r[4 * g + 2] + r[4 * g + 3]);
+    };
+    mom[i] = (parts == 4) ? grp(0) : grp(0) + grp(1);
+    if (parts == 1) mom[i] += grp(2) + grp(3);
+  }
+  const int nl = win.nc / kStrips;
+  if (parts > 1) {
+    // the slot: this part's coarse points, its pre, and its side of the head
+    double* slot = reinterpret_cast<double*>(wk.zpart + static_cast<size_t>(blockIdx.x) *
+                                                           wk.zpart_stride);
+    const int cpp = win.nc / parts, npre = kStrips * kTaps / parts;
+    for (int i = tid; i < cpp; i += kThreads) slot[i] = c[i];
+    for (int i = tid; i < npre; i += kThreads) slot[cpp + i] = pre[i];
+    const HeadLayout l = head_layout(bs, sm);
+    const int H = bs.headn;
+    if (part == 0)
+      for (int i = tid; i < H; i += kThreads) slot[cpp + npre + i] = l.hp[i];
+    if (part == parts - 1)
+      for (int i = tid; i < H + kHeadBlk; i += kThreads) slot[cpp + npre + H + i] = l.hn[i];
+    if (tid == 0) {
+      wk.mpart[2 * blockIdx.x] = mom[0];
+      wk.mpart[2 * blockIdx.x + 1] = mom[1];
+    }
+    return;
+  }
+  window_head_sums(bs, sm);
+  // what the strips' first points miss, then the points in place (point i
+  // + 8 at i so far): every value is read before any is written
+  double v[kMaxNc / kThreads];
+#pragma unroll
+  for (int u = 0; u < kMaxNc / kThreads; ++u) {
+    const int i = tid + u * kThreads;
+    if (i < win.nc) {
+      const int at = i & (nl - 1), t = at - (nl - 15);
+      const int nxt = (i / nl + 1) & (kStrips - 1);
+      v[u] = (t >= 0) ? c[i] + pre[nxt * kTaps + t] : c[i];
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int u = 0; u < kMaxNc / kThreads; ++u) {
+    const int i = tid + u * kThreads;
+    if (i < win.nc) put_coarse(bs, sm, win.nc, (i + 8) & (win.nc - 1), v[u]);
+  }
+  __syncthreads();
+  window_tail<false>(bs, wk, walker, sm, win, mom[0], mom[1], tmark);
+}
+
 // The forward transform of one walker is split over `parts` workgroups
 // (1, 2 or 4) by chunk groups: with one part the workgroup finishes the
 // spectrum itself; with more, each writes its partial kept rows and partial
 // moments and spectrum1d_kernel combines them by the group tree and
 // finishes.  Either way the rows and moments are the same bits.
-__global__ __launch_bounds__(kThreads) void forward1d_kernel(const BeamsetDev bs,
-                                                              const WorkDev wk) {
-  __shared__ XformSmem sm;
+__device__ __forceinline__ void forward_pruned(const BeamsetDev& bs, const WorkDev& wk,
+                                               XformSmem& sm, const int walker, const int part,
+                                               const int parts) {
   const int tid = threadIdx.x;
-  const int n = batch_n(wk);
-  const int parts = batch_parts(n, wk.force_parts, wk.nslots, wk.parts_tab);
-  const int walker = blockIdx.x / parts;
-  const int part = blockIdx.x - walker * parts;
-  if (walker >= n) return;
   double* st = walker_state(wk, walker);
-  if (st[ST_STATUS] != POFD_OK) return;  // uniform across the workgroup
   unsigned long long tmark = wall_clock64();
   const int M2 = bs.M2;
   const double dflux = bs.dflux;
@@ -1152,11 +1863,41 @@ __global__ __launch_bounds__(kThreads) void forward1d_kernel(const BeamsetDev bs
   forward_tail(bs, wk, walker, sm, mn, var, tmark);
 }
 
-// the parts' kept rows and moments combined by the group tree, then the
-// spectrum and the noisy rows (one workgroup per walker)
+// kWindows: the beam set has windows, and a walker whose spectrum fits one
+// takes it
+template <bool kWindows>
+__global__ __launch_bounds__(kThreads) void forward1d_kernel(const BeamsetDev bs,
+                                                              const WorkDev wk) {
+  __shared__ union {
+    XformSmem x;
+    WindowSmem w;
+  } sm;
+  const int n = batch_n(wk);
+  const int parts = batch_parts(n, wk.force_parts, wk.nslots, wk.parts_tab);
+  const int walker = blockIdx.x / parts;
+  const int part = blockIdx.x - walker * parts;
+  if (walker >= n) return;
+  const double* st = walker_state(wk, walker);
+  if (st[ST_STATUS] != POFD_OK) return;  // uniform across the workgroup
+  if constexpr (kWindows) {
+    const int wsel = static_cast<int>(st[ST_WIN]);
+    if (wsel) {
+      forward_windowed(bs, wk, sm.w, bs.win[wsel - 1], walker, part, parts);
+      return;
+    }
+  }
+  forward_pruned(bs, wk, sm.x, walker, part, parts);
+}
+
+// the parts' kept rows (or coarse points) and moments combined by the group
+// tree, then the spectrum and the inverse's input (one workgroup per walker)
+template <bool kWindows>
 __global__ __launch_bounds__(kThreads) void spectrum1d_kernel(const BeamsetDev bs,
                                                                const WorkDev wk) {
-  __shared__ XformSmem sm;
+  __shared__ union {
+    XformSmem x;
+    WindowSmem w;
+  } smu;
   const int tid = threadIdx.x;
   const int walker = blockIdx.x;
   const int n = batch_n(wk);
@@ -1165,16 +1906,6 @@ __global__ __launch_bounds__(kThreads) void spectrum1d_kernel(const BeamsetDev b
   double* st = walker_state(wk, walker);
   if (st[ST_STATUS] != POFD_OK) return;  // uniform across the workgroup
   const unsigned long long tmark = wall_clock64();
-  {
-    int kmaxb;
-    const int nr = spectral_rows(bs, st[ST_SIGMULT], sm.rowk2, sm.rowof, kmaxb);
-    if (tid == 0) {
-      sm.isc[0] = nr;
-      sm.isc[1] = kmaxb;
-    }
-  }
-  __syncthreads();
-  const int nrows = sm.isc[0];
   // the group tree over the parts: 2 parts hold G0 + G1 and G2 + G3, 4
   // parts one group each
   const size_t p0 = static_cast<size_t>(walker) * parts;
@@ -1190,6 +1921,45 @@ __global__ __launch_bounds__(kThreads) void spectrum1d_kernel(const BeamsetDev b
   double2* zrows = wk.zrows + walker * wk.zrows_stride;
   const double2* zp = wk.zpart + p0 * wk.zpart_stride;
   const size_t zs = wk.zpart_stride;
+  const int wsel = kWindows ? static_cast<int>(st[ST_WIN]) : 0;
+  if (wsel) {
+    // the parts' coarse points, with what each strip's first points miss
+    WindowSmem& sm = smu.w;
+    const WindowDev& win = bs.win[wsel - 1];
+    window_setup(bs, win, st, sm);
+    const int nc = win.nc, nl = nc / kStrips, cpp = nc / parts, spp = kStrips / parts;
+    const double* seg = reinterpret_cast<const double*>(zp);
+    const size_t ss = 2 * zs;  // doubles per slot
+    for (int i = tid; i < nc; i += kThreads) {
+      const int at = i & (nl - 1), t = at - (nl - 15);
+      double v = seg[(i / cpp) * ss + i % cpp];
+      if (t >= 0) {
+        const int nxt = (i / nl + 1) & (kStrips - 1);
+        v += seg[(nxt / spp) * ss + cpp + (nxt % spp) * kTaps + t];
+      }
+      put_coarse(bs, sm, nc, (i + 8) & (nc - 1), v);
+    }
+    const HeadLayout hl = head_layout(bs, sm);
+    const int H = bs.headn;
+    const double* hs = seg + cpp + spp * kTaps;
+    for (int i = tid; i < H; i += kThreads) hl.hp[i] = hs[i];
+    for (int i = tid; i < H + kHeadBlk; i += kThreads) hl.hn[i] = hs[(parts - 1) * ss + H + i];
+    __syncthreads();
+    window_head_sums(bs, sm);
+    window_tail<true>(bs, wk, walker, sm, win, mn, var, tmark);
+    return;
+  }
+  XformSmem& sm = smu.x;
+  {
+    int kmaxb;
+    const int nr = spectral_rows(bs, st[ST_SIGMULT], sm.rowk2, sm.rowof, kmaxb);
+    if (tid == 0) {
+      sm.isc[0] = nr;
+      sm.isc[1] = kmaxb;
+    }
+  }
+  __syncthreads();
+  const int nrows = sm.isc[0];
   for (int e = tid; e < nrows * kM1; e += kThreads) {
     zrows[e] = (parts == 2) ? cadd(zp[e], zp[zs + e])
                             : cadd(cadd(zp[e], zp[zs + e]), cadd(zp[2 * zs + e], zp[3 * zs + e]));
@@ -1287,11 +2057,16 @@ __device__ void forward_tail(const BeamsetDev& bs, const WorkDev& wk, const int 
 #pragma unroll
         for (int b = 2; b < kHeadBlk; ++b) eb[b] = em1_add(eb[b - 1], e1);
         const double2 e8 = em1_add(eb[kHeadBlk - 1], e1);
-        dh = head_sum(bs, elo, ehi, hp, vp, part * nbp / kHeadSplit,
-                      (part + 1) * nbp / kHeadSplit, k, eb, e8);
+        auto e8at = [&](const int a) {  // E(8 a k)
+          return em1_at(bs, elo, ehi, static_cast<uint32_t>(kHeadBlk) * static_cast<uint32_t>(k) *
+                                          static_cast<uint32_t>(a));
+        };
+        const int al = part * nbp / kHeadSplit;
+        dh = head_sum(hp, vp, al, (part + 1) * nbp / kHeadSplit, eb, e8, e8at(al));
         if (nbn) {
-          const double2 dn = head_sum(bs, elo, ehi, hn, vn, part * nbn / kHeadSplit,
-                                      (part + 1) * nbn / kHeadSplit, k, eb, e8);
+          const int an = part * nbn / kHeadSplit;
+          const double2 dn =
+              head_sum(hn, vn, an, (part + 1) * nbn / kHeadSplit, eb, e8, e8at(an));
           dh.x += dn.x;  // W^{(N - v) k} - 1 = conj(E(vk))
           dh.y -= dn.y;
         }
@@ -1381,9 +2156,263 @@ __device__ void forward_tail(const BeamsetDev& bs, const WorkDev& wk, const int 
 // the noisy rows, clamp, P(D) and its 32-value block statistics to HBM,
 // and the whole-array statistics of the split search
 // ===========================================================================
+// getPD's sgpos / sgneg (src/PDFactory.cc:1225-1232) and findSplitPoint's
+// search range [bot, top] (:790-801) of one dataset
+struct SplitRange {
+  double sigma, sgpos, sgneg;
+  int bot, top;
+};
+__device__ __forceinline__ SplitRange split_range(const BeamsetDev& bs, const double sigma,
+                                                  const double var) {
+  SplitRange r;
+  r.sigma = sigma;
+  r.sgpos = sqrt(var + sigma * sigma);
+  r.sgneg = (9 * sigma * sigma > var) ? sigma : r.sgpos;
+  const double n1sigpos = 2.5 * r.sgpos, n1signeg = 2.5 * r.sgneg;
+  double bd = n1sigpos / bs.dflux;
+  bd = (bd > 2e9) ? 2e9 : bd;
+  r.bot = static_cast<int>(bd);
+  if (n1sigpos > fabs(bs.minflux_R)) {
+    r.top = bs.wrapRidx;
+  } else {
+    double td = -(n1signeg + bs.minflux_R) / bs.dflux + bs.wrapRidx + 1;
+    td = (td > 2e9) ? 2e9 : ((td < -2e9) ? -2e9 : td);
+    r.top = static_cast<int>(td);
+  }
+  return r;
+}
+
+// v of the lane n before in a row of 16, round the row
+template <int n>
+__device__ __forceinline__ double row_turn(const double v) {
+  const unsigned long long u = static_cast<unsigned long long>(__double_as_longlong(v));
+  const int lo = __builtin_amdgcn_update_dpp(0, static_cast<int>(static_cast<unsigned>(u)),
+                                             0x120 + n, 0xf, 0xf, false);
+  const int hi = __builtin_amdgcn_update_dpp(0, static_cast<int>(static_cast<unsigned>(u >> 32)),
+                                             0x120 + n, 0xf, 0xf, false);
+  return __longlong_as_double(
+      static_cast<long long>((static_cast<unsigned long long>(static_cast<unsigned>(hi)) << 32) |
+                             static_cast<unsigned>(lo)));
+}
+
+struct InverseSmem {
+  double uw[kMaxNc + kTaps];
+  double peak[kWaves], mnv[kWaves], mni[kWaves];
+  double s[kGroups][kWaves], sj[kGroups][kWaves];
+};
+
+// The windowed inverse over this part's ng groups of coarse rows (from
+// global row a0): the values of window_value, 16 rows x 16 fine columns a
+// step on v_mfma_f64_16x16x4_f64 (lane (lj, lk) holds A[lj][lk] and B[lk][lj]
+// of a step of four taps and receives D[lk + 4 rr][lj]; windows of p < 16
+// leave the columns past p unused), then the clamp, the statistics of the
+// split search and those of each block of 16 rows.  Nothing of size N is
+// stored: what the split search and the likelihoods need they make again.
+// The next tile's products are issued ahead of a tile's statistics, which
+// bound the kernel (VALU): 54 us for 256 walkers at 2^17, where the pruned
+// inverse took 135 and wrote the 268 MB that the next kernels read.
+template <int p>
+__device__ __forceinline__ void inverse_window(const WindowDev& win, InverseSmem& sm,
+                                               const int a0, const int ng, const int botidx,
+                                               const int topidx, double* __restrict__ bmin,
+                                               double* __restrict__ bsum, double& pk, double& mnv,
+                                               int& mni) {
+  constexpr int CT = (p + 15) / 16;  // column tiles
+  const int tid = threadIdx.x, wv = tid >> 6;
+  const int lj = tid & 15, lk = (tid >> 4) & 3;
+  const bool on = p >= 16 || lj < p;
+  double hb[CT][4];
+#pragma unroll
+  for (int ct = 0; ct < CT; ++ct)
+#pragma unroll
+    for (int s = 0; s < 4; ++s)
+      hb[ct][s] = on ? win.h[(16 * ct + lj) * kTaps + 4 * s + lk] : 0.0;
+  __syncthreads();  // uw, loaded by the caller
+  // tile i of this wavefront: rows 16 (wv + 16 i), groups of tpg tiles
+  const int tpg = win.nc / kGroups / (16 * kWaves), ntile = ng * tpg;
+  auto tile = [&](const int i, f64x4* d) {
+    const double* ur = sm.uw + 16 * (wv + kWaves * i) + lj + lk;
+    double ua[4];
+#pragma unroll
+    for (int s = 0; s < 4; ++s) ua[s] = ur[4 * s];
+#pragma unroll
+    for (int ct = 0; ct < CT; ++ct) {
+      d[ct] = f64x4{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+      for (int s = 0; s < 4; ++s)
+        d[ct] = __builtin_amdgcn_mfma_f64_16x16x4f64(ua[s], hb[ct][s], d[ct], 0, 0, 0);
+    }
+  };
+  f64x4 nx[CT];
+  tile(0, nx);
+  double s_wave = 0.0, sj_part = 0.0;
+  for (int i = 0; i < ntile; ++i) {
+    double v[4 * CT];  // this lane's values, ascending
+#pragma unroll
+    for (int q = 0; q < 4 * CT; ++q) v[q] = fmax(nx[q % CT][q / CT], 0.0);  // positivity
+    if (i + 1 < ntile) tile(i + 1, nx);
+    const int row = 16 * (wv + kWaves * i);
+    const int jt = p * (a0 + row);  // the tile's 16 p values from jt
+    const int jl = jt + p * lk + lj;
+    double bm = v[0], bx = v[0], bs = v[0], bj = 0.0;
+#pragma unroll
+    for (int q = 1; q < 4 * CT; ++q) {
+      bx = fmax(v[q], bx);
+      bm = fmin(v[q], bm);
+      bs += v[q];
+      bj = fma(static_cast<double>(4 * p * (q / CT) + 16 * (q % CT)), v[q], bj);
+    }
+    pk = fmax(bx, pk);  // (the unused columns are zero)
+    if (jt + 16 * p > botidx && jt <= topidx) {  // uniform across the wavefront
+#pragma unroll
+      for (int q = 0; q < 4 * CT; ++q) {
+        const int j = jl + 4 * p * (q / CT) + 16 * (q % CT);
+        if (on && j >= botidx && j <= topidx && (mni < 0 || v[q] < mnv)) {
+          mnv = v[q];
+          mni = j;
+        }
+      }
+    }
+    if (!on) bm = INFINITY;
+    sj_part += fma(static_cast<double>(jl), bs, bj);
+    bm = fmin(bm, row_turn<8>(bm));
+    bs += row_turn<8>(bs);
+    bm = fmin(bm, row_turn<4>(bm));
+    bs += row_turn<4>(bs);
+    bm = fmin(bm, row_turn<2>(bm));
+    bs += row_turn<2>(bs);
+    bm = fmin(bm, row_turn<1>(bm));
+    bs += row_turn<1>(bs);
+    bm = fmin(bm, __shfl_xor(bm, 16));
+    bs += __shfl_xor(bs, 16);
+    bm = fmin(bm, __shfl_xor(bm, 32));
+    bs += __shfl_xor(bs, 32);
+    s_wave += bs;
+    if ((tid & 63) == 0) {
+      bmin[(a0 + row) >> 4] = bm;
+      bsum[(a0 + row) >> 4] = bs;
+    }
+    if ((i + 1) % tpg == 0) {  // the end of a group
+#pragma unroll
+      for (int o = 32; o > 0; o >>= 1) sj_part += __shfl_xor(sj_part, o);
+      if ((tid & 63) == 0) {
+        sm.s[i / tpg][wv] = s_wave;
+        sm.sj[i / tpg][wv] = sj_part;
+      }
+      s_wave = 0.0;
+      sj_part = 0.0;
+    }
+  }
+}
+
+// (value, index) minimum with first-index tie break; idx < 0 means empty
+__device__ __forceinline__ void take_min(double& v, double& idx, const double u, const double ui) {
+  const bool take = (ui >= 0) && (idx < 0 || u < v || (u == v && ui < idx));
+  v = take ? u : v;
+  idx = take ? ui : idx;
+}
+__device__ __forceinline__ void inverse_windowed(const BeamsetDev& bs, const WorkDev& wk,
+                                                 InverseSmem& sm, const WindowDev& win,
+                                                 const int walker, const int part,
+                                                 const int parts, const int f) {
+  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+  const unsigned long long t0 = wall_clock64();
+  const double* st = walker_state(wk, walker);
+  const size_t wf = static_cast<size_t>(walker) * bs.nfields + f;
+  double* dbg = wk.dbg + wf * kDbg;
+  // this part's rows of the coarse P(D), u_m at uw[m - a0 + 7]
+  const int nc = win.nc, na = nc / parts, a0 = part * na;
+  const double* u = coarse_pd(bs, wk, walker, f);
+  for (int i = tid; i < na + kTaps - 1; i += kThreads) sm.uw[i] = u[(a0 + i - 7) & (nc - 1)];
+  const SplitRange rg =
+      split_range(bs, st[ST_SIGMULT] * bs.fields[f].sigma_base, st[ST_VAR]);
+  if (part == 0 && tid == kThreads - 1) {
+    dbg[7] = rg.sgpos;
+    dbg[8] = rg.sgneg;
+    dbg[12] = spectral_kmax(rg.sigma, bs.iflux, bs.spectral_cut, bs.M);
+    dbg[13] = 0.0;
+    dbg[19] = st[ST_KMAXB];
+    dbg[23] = rg.sigma;
+  }
+  double pk = -1.0, mnv = 0.0;
+  int mni = -1;
+  const int ng = kGroups / parts;
+  auto rows = [&](auto pc) {
+    inverse_window<decltype(pc)::value>(win, sm, a0, ng, rg.bot, rg.top,
+                                        wk.bmin + wf * wk.blk_stride,
+                                        wk.bsum + wf * wk.blk_stride, pk, mnv, mni);
+  };
+  switch (win.p) {
+    case 32: rows(std::integral_constant<int, 32>{}); break;
+    case 16: rows(std::integral_constant<int, 16>{}); break;
+    default: rows(std::integral_constant<int, 8>{}); break;
+  }
+  double mi = static_cast<double>(mni);
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) {
+    pk = fmax(pk, __shfl_xor(pk, o));
+    const double uv = __shfl_xor(mnv, o), ui = __shfl_xor(mi, o);
+    take_min(mnv, mi, uv, ui);
+  }
+  if (lane == 0) {
+    sm.peak[wv] = pk;
+    sm.mnv[wv] = mnv;
+    sm.mni[wv] = mi;
+  }
+  __syncthreads();
+  if (tid >= 16) return;
+  // the wavefronts' results over 16 lanes, the groups by the tree
+  pk = sm.peak[tid];
+  mnv = sm.mnv[tid];
+  mi = sm.mni[tid];
+  double S[kGroups], SJ[kGroups];
+#pragma unroll
+  for (int g = 0; g < kGroups; ++g) {
+    S[g] = (g < ng) ? sm.s[g][tid] : 0.0;
+    SJ[g] = (g < ng) ? sm.sj[g][tid] : 0.0;
+  }
+#pragma unroll
+  for (int o = 8; o > 0; o >>= 1) {
+    pk = fmax(pk, __shfl_xor(pk, o));
+    const double uv = __shfl_xor(mnv, o), ui = __shfl_xor(mi, o);
+    take_min(mnv, mi, uv, ui);
+#pragma unroll
+    for (int g = 0; g < kGroups; ++g) {
+      S[g] += __shfl_xor(S[g], o);
+      SJ[g] += __shfl_xor(SJ[g], o);
+    }
+  }
+  if (tid == 0) {
+    // this part's group, pair or all four
+    const double s = (ng == 1) ? S[0] : (ng == 2 ? S[0] + S[1] : (S[0] + S[1]) + (S[2] + S[3]));
+    const double sj =
+        (ng == 1) ? SJ[0] : (ng == 2 ? SJ[0] + SJ[1] : (SJ[0] + SJ[1]) + (SJ[2] + SJ[3]));
+    if (parts == 1) {
+      dbg[1] = pk;
+      dbg[2] = mi;  // -1: empty search range
+      dbg[3] = mnv;
+      dbg[20] = s;
+      dbg[21] = sj;
+    } else {
+      double* ip = wk.ipart + (static_cast<size_t>(blockIdx.x) * bs.nfields + f) * kIPart;
+      ip[0] = pk;
+      ip[1] = mi;
+      ip[2] = mnv;
+      ip[3] = s;
+      ip[4] = sj;
+    }
+    if (part == 0) dbg[28] = static_cast<double>(wall_clock64() - t0);
+  }
+}
+
+template <bool kWindows>
 __global__ __launch_bounds__(kThreads) void inverse1d_kernel(const BeamsetDev bs,
                                                               const WorkDev wk) {
-  __shared__ XformSmem sm;
+  __shared__ union {
+    XformSmem x;
+    InverseSmem w;
+  } smu;
+  XformSmem& sm = smu.x;
   const int tid = threadIdx.x;
   const int n = batch_n(wk);
   const int parts = batch_parts(n, wk.force_parts, wk.nslots, wk.parts_tab);
@@ -1393,9 +2422,15 @@ __global__ __launch_bounds__(kThreads) void inverse1d_kernel(const BeamsetDev bs
   if (walker >= n) return;
   const double* st = walker_state(wk, walker);
   if (st[ST_STATUS] != POFD_OK) return;  // uniform across the workgroup
+  if constexpr (kWindows) {
+    const int wsel = static_cast<int>(st[ST_WIN]);
+    if (wsel) {
+      inverse_windowed(bs, wk, smu.w, bs.win[wsel - 1], walker, part, parts, f);
+      return;
+    }
+  }
   const unsigned long long t0 = wall_clock64();
   const int M = bs.M, M2 = bs.M2;
-  const double dflux = bs.dflux;
   const FieldDev& fd = bs.fields[f];
   const size_t wf = static_cast<size_t>(walker) * bs.nfields + f;
   double* pofd = wk.pofd + wf * wk.pofd_stride;
@@ -1405,42 +2440,25 @@ __global__ __launch_bounds__(kThreads) void inverse1d_kernel(const BeamsetDev bs
   const double2* zp =
       wk.zrows + walker * wk.zrows_stride + static_cast<size_t>(1 + f) * M;
   const double sigmult = st[ST_SIGMULT];
-  const double var_noi = st[ST_VAR];
-  const double sigma = sigmult * fd.sigma_base;
-  // getPD: sgpos / sgneg (src/PDFactory.cc:1225-1232)
-  const double sgpos = sqrt(var_noi + sigma * sigma);
-  const double sgneg = (9 * sigma * sigma > var_noi) ? sigma : sgpos;
+  const SplitRange rg = split_range(bs, sigmult * fd.sigma_base, st[ST_VAR]);
+  const int botidx = rg.bot, topidx = rg.top;
 
   load_twiddles(bs, sm);
   int kmaxb;
   const int nr_rows = spectral_rows(bs, sigmult, sm.rowk2, sm.rowof, kmaxb);
   if (tid == 0) {
     sm.isc[0] = nr_rows;
-    // findSplitPoint search range (src/PDFactory.cc:790-801)
-    const double n1sigpos = 2.5 * sgpos, n1signeg = 2.5 * sgneg;
-    double bd = n1sigpos / dflux;
-    bd = (bd > 2e9) ? 2e9 : bd;
-    int topidx;
-    if (n1sigpos > fabs(bs.minflux_R)) {
-      topidx = bs.wrapRidx;
-    } else {
-      double td = -(n1signeg + bs.minflux_R) / dflux + bs.wrapRidx + 1;
-      td = (td > 2e9) ? 2e9 : ((td < -2e9) ? -2e9 : td);
-      topidx = static_cast<int>(td);
-    }
-    sm.isc[1] = static_cast<int>(bd);
-    sm.isc[2] = topidx;
     if (part == 0) {
-      dbg[7] = sgpos;
-      dbg[8] = sgneg;
-      dbg[12] = spectral_kmax(sigma, bs.iflux, bs.spectral_cut, M);
+      dbg[7] = rg.sgpos;
+      dbg[8] = rg.sgneg;
+      dbg[12] = spectral_kmax(rg.sigma, bs.iflux, bs.spectral_cut, M);
       dbg[13] = sm.isc[0];
       dbg[19] = kmaxb;
-      dbg[23] = sigma;
+      dbg[23] = rg.sigma;
     }
   }
   __syncthreads();
-  const int nrows = sm.isc[0], botidx = sm.isc[1], topidx = sm.isc[2];
+  const int nrows = sm.isc[0];
   const int nchunks = M2 / kChunk;
   const int g_lo = part * kGroups / parts, g_hi = (part + 1) * kGroups / parts;
   const int c_lo = group_chunk(g_lo, nchunks), c_hi = group_chunk(g_hi, nchunks);
@@ -1641,6 +2659,7 @@ __device__ void combine_walker(const BeamsetDev& bs, const WorkDev& wk, const in
 // fuse: the beam set has one dataset and it is binned, so the combine needs
 // nothing from a later launch: thread 0 does it for the walker at the end
 // (combine1d_kernel is then not launched)
+template <bool kWindows>
 __global__ __launch_bounds__(kThreads) void finalize1d_kernel(const BeamsetDev bs,
                                                                const WorkDev wk, const int fuse,
                                                                const int accumulate,
@@ -1649,6 +2668,10 @@ __global__ __launch_bounds__(kThreads) void finalize1d_kernel(const BeamsetDev b
   __shared__ double red[kWaves * 2];
   __shared__ int isc[4];
   __shared__ double sc[2];
+  __shared__ double uw[kWindows ? kMaxNc + kTaps : 1];  // a windowed P(D)
+  __shared__ double ht[kWindows ? 32 * kTaps : 1];
+  constexpr int kNear = 17;  // values before the minimum that the search reads
+  __shared__ double near[kNear + 4], ends[2];
   const int tid = threadIdx.x;
   const int walker = blockIdx.x;
   const int f = blockIdx.y;
@@ -1668,7 +2691,19 @@ __global__ __launch_bounds__(kThreads) void finalize1d_kernel(const BeamsetDev b
   double* pofd = wk.pofd + wf * wk.pofd_stride;
   const double* bmin = wk.bmin + wf * wk.blk_stride;
   const double* bsum = wk.bsum + wf * wk.blk_stride;
-  const int nbc = bs.M2 / kChunk;  // P(D) blocks per transform row
+  // the P(D): stored, or made from the coarse one
+  const int wsel = kWindows ? static_cast<int>(st[ST_WIN]) : 0;
+  int lp = 0, blk = kBlk, nbc = bs.M2 / kChunk;  // P(D) blocks per transform row
+  if (wsel) {
+    const WindowDev& win = bs.win[wsel - 1];
+    lp = __builtin_ctz(static_cast<unsigned>(win.p));
+    blk = 16 * win.p;
+    nbc = 0;
+    const double* u = coarse_pd(bs, wk, walker, f);
+    for (int i = tid; i < win.nc + kTaps - 1; i += kThreads) uw[i] = u[(i - 7) & (win.nc - 1)];
+    load_window(win, ht);
+  }
+  auto P = [&](const int i) { return wsel ? window_value(uw, ht, lp, i) : pofd[i]; };
   double* dbg = wk.dbg + wf * kDbg;
   if (parts > 1) {
     // the inverse transform's parts: peak and argmin in part (= index)
@@ -1709,20 +2744,22 @@ __global__ __launch_bounds__(kThreads) void finalize1d_kernel(const BeamsetDev b
   const double sgpos = dbg[7], sgneg = dbg[8];
   const double peak = dbg[1];
   const double S = dbg[20], SJ = dbg[21];
-  int botidx, topidx;
+  const SplitRange rg = split_range(bs, dbg[23], st[ST_VAR]);
+  const int botidx = rg.bot, topidx = rg.top;
+
+  // the values around the minimum and at the ends of the search range
+  __syncthreads();
   {
-    const double n1sigpos = 2.5 * sgpos, n1signeg = 2.5 * sgneg;
-    double bd = n1sigpos / dflux;
-    bd = (bd > 2e9) ? 2e9 : bd;
-    botidx = static_cast<int>(bd);
-    if (n1sigpos > fabs(bs.minflux_R)) {
-      topidx = bs.wrapRidx;
-    } else {
-      double td = -(n1signeg + bs.minflux_R) / dflux + bs.wrapRidx + 1;
-      td = (td > 2e9) ? 2e9 : ((td < -2e9) ? -2e9 : td);
-      topidx = static_cast<int>(td);
+    const int m0 = static_cast<int>(dbg[2]) < 0 ? botidx : static_cast<int>(dbg[2]);
+    if (tid < kNear + 4) {
+      const int i = m0 - kNear + tid;
+      near[tid] = (i >= 0 && i < N) ? P(i) : 0.0;
+    } else if (tid >= 64 && tid < 66) {
+      const int i = (tid == 64) ? botidx : topidx;
+      ends[tid - 64] = (i >= 0 && i < N) ? P(i) : 0.0;
     }
   }
+  __syncthreads();
 
   // ---- findSplitPoint (src/PDFactory.cc:691-921) -----------------------
   if (tid == 0) {
@@ -1740,19 +2777,18 @@ __global__ __launch_bounds__(kThreads) void finalize1d_kernel(const BeamsetDev b
       status = POFD_E_SPLIT;
     if (status == POFD_OK && minidx < 0) {  // empty range: minidx = botidx
       minidx = botidx;
-      minval = pofd[botidx];
+      minval = ends[0];
     }
     if (status == POFD_OK && minval > f2 * peak) status = POFD_E_SPLIT;
     int decided = 0;
     if (status == POFD_OK) {
-      const int pre_jitter_n = 17;
+      const int pre_jitter_n = kNear;
       if (minidx > pre_jitter_n) {
         bool mono = true;
-        const int initidx = minidx - pre_jitter_n;
-        double prev = pofd[initidx];
+        double prev = near[0];
         jitter = prev;
-        for (int i = initidx + 1; i < minidx; ++i) {
-          const double cv = pofd[i];
+        for (int i = 1; i < pre_jitter_n; ++i) {
+          const double cv = near[i];
           if (cv >= prev) mono = false;
           jitter += cv;
           prev = cv;
@@ -1778,15 +2814,15 @@ __global__ __launch_bounds__(kThreads) void finalize1d_kernel(const BeamsetDev b
         int bi = (minidx < botidx) ? botidx : minidx - nminup;
         const int ti = (minidx > topidx - nminup) ? topidx - nminup : minidx + nminup;
         if (bi < 0) bi = 0;
-        for (int i = bi; i < ti && i < N; ++i) {
-          const double cv = pofd[i];
+        for (int i = bi; i < ti && i < N; ++i) {  // within kNear before, 2 past
+          const double cv = near[i - minidx + kNear];
           if (cv > minval) minval = cv;
         }
       }
       if (minval > 0) jitter = (f3 * minval) < jitter ? (f3 * minval) : jitter;
       if (botidx >= topidx)
         status = POFD_E_SPLIT;
-      else if (pofd[topidx] < jitter)
+      else if (ends[1] < jitter)
         status = POFD_E_SPLIT;
     }
     isc[0] = status;
@@ -1801,14 +2837,14 @@ __global__ __launch_bounds__(kThreads) void finalize1d_kernel(const BeamsetDev b
     // largest i in [botidx, topidx-1] with pofd[i] < jitter; split = i+1
     const double jitter = sc[0];
     const int lo = botidx, hi = topidx - 1;
-    const int bl = lo / kBlk, bh = hi / kBlk;
+    const int bl = lo / blk, bh = hi / blk;
     int found;
     {  // top (possibly partial) block, value by value
-      const int a = max(lo, bh * kBlk);
+      const int a = max(lo, bh * blk);
       int cand = -1;
-      if (tid < kBlk) {
+      if (tid < blk) {
         const int i = a + tid;
-        if (i <= hi && pofd[i] < jitter) cand = i;
+        if (i <= hi && P(i) < jitter) cand = i;
       }
       found = block_max_int(cand, red);
     }
@@ -1820,9 +2856,9 @@ __global__ __launch_bounds__(kThreads) void finalize1d_kernel(const BeamsetDev b
         const int bstar = block_max_int(cb, red);
         if (bstar >= 0) {
           int cand = -1;
-          if (tid < kBlk) {
-            const int i = bstar * kBlk + tid;
-            if (pofd[i] < jitter) cand = i;
+          if (tid < blk) {
+            const int i = bstar * blk + tid;
+            if (P(i) < jitter) cand = i;
           }
           found = block_max_int(cand, red);
         }
@@ -1830,9 +2866,9 @@ __global__ __launch_bounds__(kThreads) void finalize1d_kernel(const BeamsetDev b
     }
     if (found < 0 && bl < bh) {  // bottom partial block
       int cand = -1;
-      if (tid < kBlk) {
+      if (tid < blk) {
         const int i = lo + tid;
-        if (i <= min(hi, bl * kBlk + kBlk - 1) && pofd[i] < jitter) cand = i;
+        if (i <= min(hi, bl * blk + blk - 1) && P(i) < jitter) cand = i;
       }
       found = block_max_int(cand, red);
     }
@@ -1853,16 +2889,16 @@ __global__ __launch_bounds__(kThreads) void finalize1d_kernel(const BeamsetDev b
   double integral = 0.0, itot = 0.0, minflux = 0.0, Shigh = 0.0;
   if (status == POFD_OK) {
     // sum of the P(D) at indices >= split: whole blocks + the partial one
-    const int bs0 = split / kBlk;
+    const int bs0 = split / blk;
     double part = 0.0;
-    for (int b = bs0 + 1 + tid; b < N / kBlk; b += kThreads) part += bsum[blk_slot(b, nbc)];
-    if (tid < kBlk) {
-      const int i = bs0 * kBlk + tid;
-      if (i >= split && i < N) part += pofd[i];
+    for (int b = bs0 + 1 + tid; b < N / blk; b += kThreads) part += bsum[blk_slot(b, nbc)];
+    if (tid < blk) {
+      const int i = bs0 * blk + tid;
+      if (i >= split && i < N) part += P(i);
     }
     Shigh = block_sum(part, red);
-    const double plast = pofd[(split + N - 1) % N];
-    const double pfirst = pofd[split];
+    const double plast = P((split + N - 1) % N);
+    const double pfirst = P(split);
     // trapezoid integral of the rotated array (PD::getIntegral)
     integral = (S - 0.5 * pfirst - 0.5 * plast) * dflux;
     itot = 1.0 / integral;
@@ -1886,7 +2922,7 @@ __global__ __launch_bounds__(kThreads) void finalize1d_kernel(const BeamsetDev b
       auto Lrot = [&](int i) {
         int jj = i + split;
         if (jj >= N) jj -= N;
-        return log2_or_small(pofd[jj] * itot);
+        return log2_or_small(P(jj) * itot);
       };
       double part = 0.0;
       for (uint32_t i = tid; i < fd.nbins; i += kThreads) {
@@ -1948,14 +2984,16 @@ __global__ __launch_bounds__(kThreads) void finalize1d_kernel(const BeamsetDev b
 // pixels outside it, fewer than the cells they lie in, one by one.
 // Bound by the L1-L2 lines of the searches (153 a step) and the VALU work of
 // the log2 (222 instructions a step): at 256 walkers, 1e6 pixels and nflux
-// 2^17, 416 steps of cells and 94 of pixels a walker take 96 us, where two
-// gathers a pixel took 394 us and the rewrite of the P(D) as log2 that they
-// read another 100 us.
+// 2^17, 416 steps of cells and 94 of pixels a walker take 124 us, 96 where
+// the P(D) is stored and need not be made again (the inverse then takes 81
+// more); two gathers a pixel took 394 us and the rewrite of the P(D) as log2
+// that they read another 100 us.
 constexpr int kPixThreads = 256;
 
 __global__ __launch_bounds__(kPixThreads) void pixels1d_kernel(const BeamsetDev bs,
                                                                const WorkDev wk) {
   __shared__ double red[kPixThreads / 64];
+  __shared__ double ht[32 * kTaps];
   const int walker = blockIdx.x;  // neighbours in launch order share pixels
   const int blk = blockIdx.y;
   const int f = blockIdx.z;
@@ -1972,9 +3010,34 @@ __global__ __launch_bounds__(kPixThreads) void pixels1d_kernel(const BeamsetDev 
   const double dflux = bs.dflux, idflux = 1.0 / dflux;
   const uint32_t split = static_cast<uint32_t>(static_cast<int>(dbg[0]));
   const double itot = dbg[16], minflux = dbg[17];
-  const double* pofd = wk.pofd + wf * wk.pofd_stride;  // unrotated
+  // the unrotated P(D): stored, or made from the coarse one
+  const double* pofd = wk.pofd + wf * wk.pofd_stride;
   const uint32_t nm1 = static_cast<uint32_t>(N - 1);
-  auto Lrot = [&](const uint32_t i) { return log2_or_small(pofd[(i + split) & nm1] * itot); };
+  const int wsel = static_cast<int>(walker_state(wk, walker)[ST_WIN]);
+  int lp = 0, cmask = 0;
+  if (wsel) {  // uniform across the workgroup
+    const WindowDev& win = bs.win[wsel - 1];
+    lp = __builtin_ctz(static_cast<unsigned>(win.p));
+    cmask = win.nc - 1;
+    pofd = coarse_pd(bs, wk, walker, f);
+    load_window(win, ht);
+    __syncthreads();
+  }
+  auto Lrot = [&](const uint32_t i) {
+    const int j = static_cast<int>((i + split) & nm1);
+    double v;
+    if (wsel) {  // window_value with the coarse points in global memory
+      const int a = j >> lp, b = j & ((1 << lp) - 1);
+      v = 0.0;
+#pragma unroll
+      for (int d = 0; d < kTaps; ++d)
+        v = fma(pofd[(a + d - 7) & cmask], ht[(d << lp) + b], v);
+      v = fmax(v, 0.0);
+    } else {
+      v = pofd[j];
+    }
+    return log2_or_small(v * itot);
+  };
   const uint32_t pa = fd.pa, pb = fd.pb, rcols = fd.rcols;
   const int lane = threadIdx.x & 63;
   const PixSum* pix = fd.pix;
@@ -2070,13 +3133,30 @@ __global__ void combine1d_kernel(const BeamsetDev bs, const WorkDev wk,
 
 // Writes the P(D) of (walker, field) as PDFactory::getPD leaves PD::pd_:
 // rotated at the split, normalised, log2 when is_log (debug / parity).
-__global__ void materialize_pd_kernel(const double* pofd, int N, int split,
-                                      double itot, int is_log, double* out) {
+__global__ __launch_bounds__(256) void materialize_pd_kernel(const BeamsetDev bs,
+                                                              const WorkDev wk, const int walker,
+                                                              const int f, const int split,
+                                                              const double itot, const int is_log,
+                                                              double* out) {
+  __shared__ double ht[32 * kTaps], uw[kMaxNc + kTaps];
+  const int wsel = static_cast<int>(walker_state(wk, walker)[ST_WIN]);
+  int lp = 0;
+  if (wsel) {  // uniform across the grid
+    const WindowDev& win = bs.win[wsel - 1];
+    lp = __builtin_ctz(static_cast<unsigned>(win.p));
+    const double* u = coarse_pd(bs, wk, walker, f);
+    for (int i = threadIdx.x; i < win.nc + kTaps - 1; i += blockDim.x)
+      uw[i] = u[(i - 7) & (win.nc - 1)];
+    load_window(win, ht);
+  }
+  __syncthreads();
+  const double* pofd =
+      wk.pofd + (static_cast<size_t>(walker) * bs.nfields + f) * wk.pofd_stride;
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= N) return;
+  if (i >= bs.N) return;
   int j = i + split;
-  if (j >= N) j -= N;
-  const double p = pofd[j] * itot;
+  if (j >= bs.N) j -= bs.N;
+  const double p = (wsel ? window_value(uw, ht, lp, j) : pofd[j]) * itot;
   out[i] = is_log ? log2_or_small(p) : p;
 }
 
@@ -2115,17 +3195,21 @@ int launch_loglike1d(const BeamsetDev& bs, const WorkDev& wk_in, int beamset_idx
   if (split)
     hipLaunchKernelGGL(prepspline1d_kernel, dim3(nwalk), dim3(kThreads), 0, s, bs, wk);
   mark(POFD_STAGE_FORWARD);
-  hipLaunchKernelGGL(forward1d_kernel, dim3(nxf), dim3(kThreads), 0, s, bs, wk);
+  hipLaunchKernelGGL(bs.nwin ? forward1d_kernel<true> : forward1d_kernel<false>, dim3(nxf),
+                     dim3(kThreads), 0, s, bs, wk);
   if (split)
-    hipLaunchKernelGGL(spectrum1d_kernel, dim3(nwalk), dim3(kThreads), 0, s, bs, wk);
+    hipLaunchKernelGGL(bs.nwin ? spectrum1d_kernel<true> : spectrum1d_kernel<false>,
+                       dim3(nwalk), dim3(kThreads), 0, s, bs, wk);
   mark(POFD_STAGE_INVERSE);
-  hipLaunchKernelGGL(inverse1d_kernel, dim3(nxf, bs.nfields), dim3(kThreads), 0, s, bs, wk);
+  hipLaunchKernelGGL(bs.nwin ? inverse1d_kernel<true> : inverse1d_kernel<false>,
+                     dim3(nxf, bs.nfields), dim3(kThreads), 0, s, bs, wk);
   bool any_unbinned = false;
   for (int f = 0; f < bs.nfields; ++f) any_unbinned |= !bs.fields[f].binned;
   // one binned dataset: finalize does the combine too
   const int fuse = (bs.nfields == 1 && !any_unbinned) ? 1 : 0;
   mark(POFD_STAGE_FINALIZE);
-  hipLaunchKernelGGL(finalize1d_kernel, dim3(nwalk, bs.nfields), dim3(kThreads), 0,
+  hipLaunchKernelGGL(bs.nwin ? finalize1d_kernel<true> : finalize1d_kernel<false>,
+                     dim3(nwalk, bs.nfields), dim3(kThreads), 0,
                      s, bs, wk, fuse, accumulate, d_loglike, d_status);
   mark(POFD_STAGE_PIXELS);
   if (any_unbinned)
@@ -2200,12 +3284,12 @@ int launch_prior1d(const BeamsetDev& bs0, const WorkDev& wk0, const PriorDev& pr
   return hipGetLastError() == hipSuccess ? POFD_OK : POFD_E_INTERNAL;
 }
 
-int launch_materialize_pd(const double* d_pofd, int N, int split, double itot,
-                          int is_log, double* d_out, void* stream) {
-  const int nb = (N + 255) / 256;
+int launch_materialize_pd(const BeamsetDev& bs, const WorkDev& wk, int walker, int f, int split,
+                          double itot, int is_log, double* d_out, void* stream) {
+  const int nb = (bs.N + 255) / 256;
   hipLaunchKernelGGL(materialize_pd_kernel, dim3(nb), dim3(256), 0,
-                     static_cast<hipStream_t>(stream), d_pofd, N, split, itot,
-                     is_log, d_out);
+                     static_cast<hipStream_t>(stream), bs, wk, walker, f, split, itot, is_log,
+                     d_out);
   return hipGetLastError() == hipSuccess ? POFD_OK : POFD_E_INTERNAL;
 }
 
