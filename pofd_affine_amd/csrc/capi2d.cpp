@@ -801,8 +801,6 @@ int ensure_work2(pofd_ctx* c, Ctx2& C2, Set2& s, uint32_t nwalk) {
   const size_t o_P = tot; tot += w.P_stride * nf * W;
   const size_t o_rs1 = tot; tot += w.edge_stride * nf * W;
   const size_t o_rs2 = tot; tot += w.edge_stride * nf * W;
-  const size_t o_rA = tot; tot += w.edge_stride * nf * W;
-  const size_t o_rB = tot; tot += w.edge_stride * nf * W;
   w.colpart_stride = r8(static_cast<size_t>(pofd2::kRowBlocks2) * n);
   const size_t o_cp = tot; tot += w.colpart_stride * W;
   const size_t o_rsp = tot; tot += r8(nparts * 4) * W;
@@ -837,8 +835,6 @@ int ensure_work2(pofd_ctx* c, Ctx2& C2, Set2& s, uint32_t nwalk) {
   w.P = b + o_P;
   w.rsum1 = b + o_rs1;
   w.rsum2 = b + o_rs2;
-  w.rowA = b + o_rA;
-  w.rowB = b + o_rB;
   w.colpart = b + o_cp;
   w.rstat_part = b + o_rsp;
   w.lpart = b + o_lp;

@@ -121,8 +121,6 @@ struct Work2 {
   double* P;                      // W * nf * n * n    P(D) per dataset
   double* rsum1;                  // W * nf * edge_stride
   double* rsum2;
-  double* rowA;
-  double* rowB;
   double* colpart;                // W * kRowBlocks2 * n  column partial sums
   double* rstat_part;             // W * nparts * 4
   double* lpart;                  // W * nf * kLikeBlocks
