@@ -774,28 +774,21 @@ int ensure_work2(pofd_ctx* c, Ctx2& C2, Set2& s, uint32_t nwalk) {
   const size_t n = C2.n, ne = C2.nedge, nf = s.fields.size(), W = nwalk;
   const size_t nc = n / 2 + 1;
   auto r8 = [](size_t x) { return (x + 7) & ~size_t(7); };
-  w.R_stride = r8(n * n);
   w.ex_stride = r8(ne * n);        // nedge x n (ex) or n x nedge (ey)
   w.edge_stride = r8(std::max(n, ne));
-  w.ystride = static_cast<int>(nc);
-  w.Y_stride = r8(n * nc);       // complex
   w.YT_stride = r8(nc * n);
   w.PR_stride = r8(nc * n);
-  w.Q_stride = w.YT_stride;      // Q reuses YT (consumed by the forward)
-  w.QT_stride = w.Y_stride;      // QT reuses Y
   w.P_stride = r8(n * n);
   const size_t nparts = 64;
   size_t tot = 0;
   const size_t o_model = tot; tot += r8(pofd2::kModelStride) * W;
   const size_t o_stats = tot; tot += r8(pofd2::kStats) * W;
-  const size_t o_R = tot; tot += w.R_stride * W;
   const size_t o_e00 = tot; tot += r8(ne * ne) * W;
   const size_t o_ex = tot; tot += w.ex_stride * W;
   const size_t o_ey = tot; tot += w.ex_stride * W;
   const size_t o_rx = tot; tot += w.edge_stride * W;
   const size_t o_ry = tot; tot += w.edge_stride * W;
   const size_t o_r00 = tot; tot += w.edge_stride * W;
-  const size_t o_Y = tot; tot += 2 * w.Y_stride * W;
   const size_t o_YT = tot; tot += 2 * w.YT_stride * W;
   const size_t o_PR = tot; tot += 2 * w.PR_stride * W;
   const size_t o_P = tot; tot += w.P_stride * nf * W;
@@ -820,18 +813,14 @@ int ensure_work2(pofd_ctx* c, Ctx2& C2, Set2& s, uint32_t nwalk) {
   double* b = static_cast<double*>(s.wbuf->p);
   w.model = b + o_model;
   w.stats = b + o_stats;
-  w.R = b + o_R;
   w.e00 = b + o_e00;
   w.ex = b + o_ex;
   w.ey = b + o_ey;
   w.rx = b + o_rx;
   w.ry = b + o_ry;
   w.r00rows = b + o_r00;
-  w.Y = reinterpret_cast<double2*>(b + o_Y);
   w.YT = reinterpret_cast<double2*>(b + o_YT);
   w.PR = reinterpret_cast<double2*>(b + o_PR);
-  w.Q = w.YT;
-  w.QT = w.Y;
   w.P = b + o_P;
   w.rsum1 = b + o_rs1;
   w.rsum2 = b + o_rs2;
@@ -841,8 +830,6 @@ int ensure_work2(pofd_ctx* c, Ctx2& C2, Set2& s, uint32_t nwalk) {
   w.dbg = b + o_dbg;
   w.bonus = b + o_bo;
   w.rpieces = b + o_rp;
-  s.gmain.out = w.R;
-  s.gmain.wstride = w.R_stride;
   s.g00.out = w.e00;
   s.g00.wstride = r8(ne * ne);
   s.gx.out = w.ex;

@@ -106,18 +106,15 @@ struct Work2 {
   int nwalk;
   double* model;                  // W * kModelStride
   double* stats;                  // W * kStats
-  double* R;                      // W * n * n
   double* e00;                    // W * nedge * nedge
   double* ex;                     // W * nedge * n
   double* ey;                     // W * n * nedge
   double* rx;                     // W * edge_stride (n)
   double* ry;
   double* r00rows;
-  double2* Y;                     // W * n * ystride   rows' spectra
-  double2* YT;                    // W * (n/2+1) * n   transposed
+  double2* YT;                    // W * (n/2+1) * n   rows' spectra [k2][i],
+                                  //   then per dataset the inverse columns Q
   double2* PR;                    // W * (n/2+1) * n   exp(R^ - R^0) [k2][k1]
-  double2* Q;                     // W * (n/2+1) * n   per dataset, inverse columns
-  double2* QT;                    // W * n * ystride
   double* P;                      // W * nf * n * n    P(D) per dataset
   double* rsum1;                  // W * nf * edge_stride
   double* rsum2;
@@ -130,9 +127,7 @@ struct Work2 {
                                   //   being filled, rpieces_w values (3 per
                                   //   beam element: weight, centre, width)
   int rpieces_w;
-  size_t R_stride, ex_stride, edge_stride, Y_stride, YT_stride, PR_stride,
-      Q_stride, QT_stride, P_stride, colpart_stride, rpieces_stride;
-  int ystride;                    // n/2 + 1 (complex)
+  size_t ex_stride, edge_stride, YT_stride, PR_stride, P_stride, colpart_stride, rpieces_stride;
 };
 
 // two-band state hung off pofd_ctx (capi2d.cpp) and the context accessors

@@ -537,372 +537,427 @@ __global__ void edge2d_cols_kernel(const Set2Dev s, const Work2 wk) {
   wk.rx[static_cast<size_t>(w) * wk.edge_stride + j] = acc;
 }
 
-// R[0,0] from the row sums of the nedge x nedge grid, then the patch of row
-// 0 and column 0 of the main grid (times dflux1*dflux2)
-__global__ void edge2d_patch_kernel(const Set2Dev s, const Work2 wk) {
-  const int w = blockIdx.y;
-  if (model_ptr(wk, w)[0] != POFD_OK) return;
-  const int n = s.n, ne = s.nedge;
-  double* R = wk.R + static_cast<size_t>(w) * wk.R_stride;
-  const double* rx = wk.rx + static_cast<size_t>(w) * wk.edge_stride;
-  const double* ry = wk.ry + static_cast<size_t>(w) * wk.edge_stride;
+// R[0,0] (times dflux1 dflux2) from the row sums of the nedge x nedge grid,
+// to rx[0]; rowfft2d_kernel puts rx and ry in place of row 0 and column 0
+__global__ void edge2d_r00_kernel(const Set2Dev s, const Work2 wk) {
+  const int w = blockIdx.x * blockDim.x + threadIdx.x;
+  if (w >= wk.nwalk || model_ptr(wk, w)[0] != POFD_OK) return;
+  const int ne = s.nedge;
   const double* r00rows = wk.r00rows + static_cast<size_t>(w) * wk.edge_stride;
-  const double fluxfac = s.dflux1 * s.dflux2;
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t == 0) {
+  {
 #pragma clang fp contract(off)
     double sc = 0.5 * s.edge1[0] * r00rows[0];
     for (int i = 1; i < ne - 1; ++i) sc += s.edge1[i] * r00rows[i];
     sc += 0.5 * s.edge1[ne - 1] * r00rows[ne - 1];
-    R[0] = (sc * s.iR00norm) * fluxfac;
-  }
-  if (t >= 1 && t < n) {
-#pragma clang fp contract(off)
-    R[t] = rx[t] * fluxfac;
-    R[static_cast<size_t>(t) * n] = (ry[t] * s.iRynorm) * fluxfac;
+    wk.rx[static_cast<size_t>(w) * wk.edge_stride] = (sc * s.iR00norm) * (s.dflux1 * s.dflux2);
   }
 }
 
 // ===========================================================================
-// rstats2d: trapezoid moments of R along each axis; partials per block row
+// LDS transforms
 // ===========================================================================
-__global__ __launch_bounds__(kT) void rstats2d_kernel(const Set2Dev s, const Work2 wk) {
-  __shared__ double red[kT / 64];
-  const int w = blockIdx.y;
-  if (model_ptr(wk, w)[0] != POFD_OK) return;
-  const int n = s.n;
-  const double* R = wk.R + static_cast<size_t>(w) * wk.R_stride;
-  double m1 = 0, m2 = 0, v1 = 0, v2 = 0;
-  const int rows_per = (n + gridDim.x - 1) / gridDim.x;
-  const int i0 = blockIdx.x * rows_per, i1 = min(n, i0 + rows_per);
-  for (int i = i0; i < i1; ++i) {
-    const double wi = (i == 0 || i == n - 1) ? 0.5 : 1.0;
-    const double cf1 = s.rflux1[i];
-    for (int j = threadIdx.x; j < n; j += kT) {
-      const double wj = (j == 0 || j == n - 1) ? 0.5 : 1.0;
-      const double cR = wi * R[static_cast<size_t>(i) * n + j];
-      const double p1 = wj * cf1 * cR;
-      m1 += p1;
-      v1 += cf1 * p1;
-      const double cf2 = s.rflux2[j];
-      const double p2 = wj * cf2 * cR;
-      m2 += p2;
-      v2 += cf2 * p2;
-    }
-  }
-  double* part = wk.rstat_part + (static_cast<size_t>(w) * gridDim.x + blockIdx.x) * 4;
-  const double a = block_sum(m1, red), b = block_sum(m2, red);
-  const double c = block_sum(v1, red), d = block_sum(v2, red);
-  if (threadIdx.x == 0) {
-    part[0] = a;
-    part[1] = b;
-    part[2] = c;
-    part[3] = d;
-  }
-}
+constexpr int kTR = 1024;  // threads per workgroup of the transforms
+// Rows and columns a workgroup transforms together: as many as fill 128 KB
+// with both buffers, no more than eight.  Four rows of 2048 give the 64
+// contiguous bytes in which the transposed spectra are written and read.
+inline int rows_together(const int n) { return std::min(8, 8192 / n); }
+constexpr int kMaxPairs = 4;  // pairs of a row's points per thread: n rg / 2 kTR
+inline int cols_together(const int n) { return std::min(8, 4096 / n); }
 
-// ===========================================================================
-// LDS transforms: complex length L (power of two, <= 4096), radix-4 Stockham
-// plus a final radix-2 stage when log2 L is odd.  tw[k] = e^{-2 pi i k/L}.
-// SIGN -1 forward, +1 unnormalised backward.  Returns the buffer holding the
-// result.
-// ===========================================================================
-template <int SIGN>
-__device__ double2* fft_lds(double2* a, double2* b, int L, const double2* __restrict__ tw) {
-  int Ns = 1;
+// Element i of a transform of length L is at slot(i): the exclusive-or of
+// bits 4 and 5 into bits 0 to 3 keeps a stage's writes (strides of 4 to 32
+// elements between 16 lanes) and reads on distinct banks; short transforms
+// (swz 0) are in order.  turn_slot does the same for the twiddles, which are
+// read at strides of L / 4 Ns.
+__device__ __forceinline__ int swizzle_of(const int L) { return L >= 256 ? 15 : 0; }
+__device__ __forceinline__ int slot(const int i, const int swz) {
+  const int t = (i >> 4) & 3;
+  return i ^ ((t ^ (t << 2)) & swz);
+}
+__device__ __forceinline__ int turn_slot(const int t) { return t ^ ((t >> 4) & 15) ^ (t >> 8); }
+
+// Forward transform of length L (a power of two from 32 on) from a, by T
+// threads of which this is t; every thread of the workgroup calls it, with
+// the same L.  Radix 4 after a radix-2 stage when log2 L is odd.
+// tw[turn_slot(t)] = e^{-2 pi i t/L}, t < L/4.  Returns the buffer that holds
+// the result.  (The inverse: the same with real and imaginary parts
+// exchanged before and after.)
+__device__ __forceinline__ double2* fft_lds(double2* a, double2* b, const int L,
+                                            const double2* tw, const int t, const int T) {
+  const int swz = swizzle_of(L);
   double2* src = a;
   double2* dst = b;
-  while (Ns * 4 <= L) {
-    const int q = L >> 2;
-    const int tstride = L / (4 * Ns);
-    for (int j = threadIdx.x; j < q; j += blockDim.x) {
-      double2 v0 = src[j], v1 = src[j + q], v2 = src[j + 2 * q], v3 = src[j + 3 * q];
+  int Ns = 1;
+  if (__builtin_ctz(static_cast<unsigned>(L)) & 1) {
+    const int h = L >> 1;
+    for (int j = t; j < h; j += T) {
+      const double2 v0 = src[slot(j, swz)], v1 = src[slot(j + h, swz)];
+      dst[slot(2 * j, swz)] = cadd(v0, v1);
+      dst[slot(2 * j + 1, swz)] = csub(v0, v1);
+    }
+    __syncthreads();
+    double2* u = src;
+    src = dst;
+    dst = u;
+    Ns = 2;
+  }
+  const int q = L >> 2;
+  auto quarter = [](const double2 v, const bool on) {
+    return on ? make_double2(v.y, -v.x) : v;
+  };
+  for (; Ns < L; Ns *= 4) {
+    const int ts = L / (4 * Ns);
+    for (int j = t; j < q; j += T) {
       const int jm = j & (Ns - 1);
+      const double2* sj = src + slot(j, swz);  // q is a multiple of 64, or swz 0
+      double2 v0 = sj[0], v1 = sj[q], v2 = sj[2 * q], v3 = sj[3 * q];
       if (Ns > 1) {
-        double2 t1 = tw[jm * tstride], t2 = tw[2 * jm * tstride], t3 = tw[3 * jm * tstride];
-        if (SIGN > 0) {
-          t1.y = -t1.y;
-          t2.y = -t2.y;
-          t3.y = -t3.y;
-        }
-        v1 = cmul(v1, t1);
-        v2 = cmul(v2, t2);
-        v3 = cmul(v3, t3);
+        const int t1 = jm * ts, t2 = 2 * t1, t3 = 3 * t1;  // t1 < q
+        v1 = cmul(v1, tw[turn_slot(t1)]);
+        v2 = quarter(cmul(v2, tw[turn_slot(t2 & (q - 1))]), t2 & q);
+        v3 = quarter(cmul(v3, tw[turn_slot(t3 & (q - 1))]), t3 & q);
+        if (t3 & (2 * q)) v3 = make_double2(-v3.x, -v3.y);
       }
       const double2 a0 = cadd(v0, v2), a1 = csub(v0, v2);
       const double2 a2 = cadd(v1, v3), a3 = csub(v1, v3);
-      double2 y1, y3;
-      if (SIGN < 0) {
-        y1 = make_double2(a1.x + a3.y, a1.y - a3.x);
-        y3 = make_double2(a1.x - a3.y, a1.y + a3.x);
-      } else {
-        y1 = make_double2(a1.x - a3.y, a1.y + a3.x);
-        y3 = make_double2(a1.x + a3.y, a1.y - a3.x);
-      }
-      const int d = (j / Ns) * Ns * 4 + jm;
-      dst[d] = cadd(a0, a2);
-      dst[d + Ns] = y1;
-      dst[d + 2 * Ns] = csub(a0, a2);
-      dst[d + 3 * Ns] = y3;
+      const int d = (j - jm) * 4 + jm;
+      dst[slot(d, swz)] = cadd(a0, a2);
+      dst[slot(d + Ns, swz)] = make_double2(a1.x + a3.y, a1.y - a3.x);
+      dst[slot(d + 2 * Ns, swz)] = csub(a0, a2);
+      dst[slot(d + 3 * Ns, swz)] = make_double2(a1.x - a3.y, a1.y + a3.x);
     }
     __syncthreads();
-    double2* t = src;
+    double2* u = src;
     src = dst;
-    dst = t;
-    Ns *= 4;
-  }
-  if (Ns < L) {  // radix-2 stage, Ns = L/2
-    const int h = L >> 1;
-    for (int j = threadIdx.x; j < h; j += blockDim.x) {
-      double2 v0 = src[j], v1 = src[j + h];
-      double2 t1 = tw[j];
-      if (SIGN > 0) t1.y = -t1.y;
-      v1 = cmul(v1, t1);
-      dst[j] = cadd(v0, v1);
-      dst[j + h] = csub(v0, v1);
-    }
-    __syncthreads();
-    src = dst;
+    dst = u;
   }
   return src;
 }
+__device__ __forceinline__ void load_turns(double2* tw, const double2* __restrict__ table,
+                                           const int L) {
+  for (int t = threadIdx.x; t < L / 4; t += kTR) tw[turn_slot(t)] = table[t];
+}
 
 // ===========================================================================
-// rowfft2d: r2c of every row of R (length n), outputs k2 = 0..K2 into
-// Y[i][k2] (row stride ystride complex).  One workgroup per (row, walker).
+// rowfft2d: R row by row, its trapezoid moments along each axis (partials per
+// workgroup) and the r2c transform of every row; outputs k2 = 0..K2 to
+// YT[k2][i].  R goes to memory nowhere.  rg rows together, T = kTR / rg
+// threads each (whole wavefronts, so that a row's pieces are uniform reads,
+// made once for a thread's eight points).  Bound by the exponentials of R:
+// 1648 us for 32 walkers at 2048, where R to memory, its moments, the row
+// transforms from it and their transposition took 1274 + 265 + 588 + 195
+// (2489 with the pieces read again for each point).
 // ===========================================================================
-__global__ __launch_bounds__(kT) void rowfft2d_kernel(const Set2Dev s, const Work2 wk) {
+__global__ __launch_bounds__(kTR) void rowfft2d_kernel(const Set2Dev s, const Work2 wk,
+                                                       const RGrid g, const int rg) {
   extern __shared__ double2 lds[];
+  __shared__ double red[kTR / 64];
   const int w = blockIdx.y;
   const double* m = model_ptr(wk, w);
   if (m[0] != POFD_OK) return;
   const int K2 = static_cast<int>(m[4]);
-  const int n = s.n, h = n / 2;
-  double2* a = lds;
-  double2* b = lds + h;
-  for (int i = blockIdx.x; i < n; i += gridDim.x) {
-    const double2* row =
-        reinterpret_cast<const double2*>(wk.R + static_cast<size_t>(w) * wk.R_stride +
-                                         static_cast<size_t>(i) * n);
-    for (int m = threadIdx.x; m < h; m += kT) a[m] = row[m];  // x[2m] + i x[2m+1]
+  const int n = s.n, h = n / 2, tid = threadIdx.x;
+  const int T = kTR / rg, grp = tid / T, t = tid & (T - 1);
+  const int swz = swizzle_of(h);
+  double2* tw = lds;
+  double2* rows = lds + h / 4;
+  const int rs = n + 2;  // the rows' elements k on distinct banks
+  load_turns(tw, s.tw_half, h);
+  const double* pieces = wk.rpieces + static_cast<size_t>(w) * wk.rpieces_stride;
+  const double* rx = wk.rx + static_cast<size_t>(w) * wk.edge_stride;
+  const double* ry = wk.ry + static_cast<size_t>(w) * wk.edge_stride;
+  const double fluxfac = s.dflux1 * s.dflux2;
+  double2* YT = wk.YT + static_cast<size_t>(w) * wk.YT_stride;
+  double m1 = 0, m2 = 0, v1 = 0, v2 = 0;
+  for (int i0 = blockIdx.x * rg; i0 < n; i0 += gridDim.x * rg) {
+    const int i = __builtin_amdgcn_readfirstlane(i0 + grp);
+    double2* a = rows + grp * rs;
+    const double f1val = g.f1[i];
+    const bool none = (f1val == 0) || (f1val < 0 && !s.hasneg1);  // a row of zeros
+    const int sgn1 = (f1val > 0) ? 0 : 2;
+    const double* prow = pieces + static_cast<size_t>(i) * wk.rpieces_w;
+    const double edge0 = (s.edge_integ && i > 0) ? (ry[i] * s.iRynorm) * fluxfac : 0.0;
+    const double wi = (i == 0 || i == n - 1) ? 0.5 : 1.0;
+    const double cf1 = s.rflux1[i];
+    // this thread's points: pairs t + q T of the row; the elements' pieces are
+    // read once for all of them
+    double x[2 * kMaxPairs], lf[2 * kMaxPairs];
+#pragma unroll
+    for (int q = 0; q < 2 * kMaxPairs; ++q) x[q] = 0.0;
+    if (!none) {
+#pragma unroll 1
+      for (int sg = 0; sg < 2; ++sg) {
+        const int cn = s.comp[sgn1 + sg].n;
+        if (cn == 0) continue;
+        // a point of the other sign, or of no flux: an exponent of -infinity
+#pragma unroll
+        for (int q = 0; q < 2 * kMaxPairs; ++q) {
+          const int e = t + (q >> 1) * T, j = 2 * e + (q & 1);
+          lf[q] = (e < h && g.f2inv[j] != 0 && g.f2sgn[j] == sg) ? g.f2log[j] : 1e160;
+        }
+        const double* base = prow + (sg ? 3 * s.comp[sgn1].n : 0);
+        for (int k = 0; k < cn; ++k) {
+          const double c0 = base[3 * k], c1 = base[3 * k + 1], c2 = base[3 * k + 2];
+          if (c0 == 0) continue;
+#pragma unroll
+          for (int q = 0; q < kMaxPairs; ++q) {
+#pragma clang fp contract(off)
+            if (q * T >= h) break;  // uniform
+            const double ta = lf[2 * q] - c1, tb = lf[2 * q + 1] - c1;
+            const double ea = ta * ta * c2, eb = tb * tb * c2;
+            // below the smallest number for the whole wavefront: adds nothing
+            if (__any(!(ea <= -1080.0 && eb <= -1080.0))) {
+              x[2 * q] += c0 * exp2(ea);
+              x[2 * q + 1] += c0 * exp2(eb);
+            }
+          }
+        }
+      }
+    }
+#pragma unroll
+    for (int q = 0; q < kMaxPairs; ++q) {
+      const int e = t + q * T;
+      if (e >= h) break;
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+        const int j = 2 * e + u;
+        double r = (x[2 * q + u] * g.f2inv[j]) * g.scale;
+        if (s.edge_integ && i == 0) r = (j == 0) ? rx[0] : rx[j] * fluxfac;
+        if (s.edge_integ && i > 0 && j == 0) r = edge0;
+        x[2 * q + u] = r;
+        const double wj = (j == 0 || j == n - 1) ? 0.5 : 1.0;
+        const double cR = wi * r;
+        const double p1 = wj * cf1 * cR;
+        m1 += p1;
+        v1 += cf1 * p1;
+        const double cf2 = s.rflux2[j];
+        const double p2 = wj * cf2 * cR;
+        m2 += p2;
+        v2 += cf2 * p2;
+      }
+      a[slot(e, swz)] = make_double2(x[2 * q], x[2 * q + 1]);
+    }
     __syncthreads();
-    const double2* z = fft_lds<-1>(a, b, h, s.tw_half);
-    double2* Y = wk.Y + static_cast<size_t>(w) * wk.Y_stride + static_cast<size_t>(i) * wk.ystride;
-    for (int k = threadIdx.x; k <= K2; k += kT) {
-      const int kk = (k == h) ? 0 : k, mk = (k == 0) ? 0 : h - k;
-      const double2 zk = z[kk];
-      const double2 zm = make_double2(z[mk].x, -z[mk].y);
+    const double2* z = fft_lds(a, a + h, h, tw, t, T) - grp * rs;  // row 0's
+    for (int o = tid; o < rg * (K2 + 1); o += kTR) {
+      const int k = o / rg, row = o - k * rg;
+      const double2* zr = z + row * rs;
+      const double2 zk = zr[slot((k == h) ? 0 : k, swz)];
+      const double2 zh = zr[slot((k == 0) ? 0 : h - k, swz)];
+      const double2 zm = make_double2(zh.x, -zh.y);
       const double2 A = make_double2(0.5 * (zk.x + zm.x), 0.5 * (zk.y + zm.y));
       const double2 B = make_double2(0.5 * (zk.y - zm.y), -0.5 * (zk.x - zm.x));
       const double2 wv = (k == h) ? make_double2(-1.0, 0.0) : s.tw_n[k];
-      Y[k] = cadd(A, cmul(B, wv));
+      YT[static_cast<size_t>(k) * n + i0 + row] = cadd(A, cmul(B, wv));
     }
     __syncthreads();
   }
-}
-
-// ===========================================================================
-// transpose2d: out[c][r] = in[r][c] for r < nr, c < nc (complex), 32x32
-// LDS tiles; grid (tiles, walkers)
-// ===========================================================================
-// kmode 1: the column count of `in` is K2+1 of the walker (Y -> YT);
-// kmode 2: the row count of `in` is K2+1 (Q -> QT)
-__global__ __launch_bounds__(kT) void transpose2d_kernel(const Work2 wk, const double2* in,
-                                                         size_t in_wstride, int in_stride,
-                                                         double2* out, size_t out_wstride,
-                                                         int out_stride, int nr, int nc,
-                                                         int kmode) {
-  __shared__ double2 tile[32][33];
-  const int w = blockIdx.z;
-  const double* m = model_ptr(wk, w);
-  if (m[0] != POFD_OK) return;
-  const int kk = static_cast<int>(m[4]) + 1;
-  if (kmode == 1) nc = kk;
-  if (kmode == 2) nr = kk;
-  const int tc = blockIdx.x * 32, tr = blockIdx.y * 32;
-  if (tc >= nc || tr >= nr) return;
-  const int lx = threadIdx.x & 31, ly = threadIdx.x >> 5;  // 32 x 8
-  const double2* src = in + static_cast<size_t>(w) * in_wstride;
-  double2* dst = out + static_cast<size_t>(w) * out_wstride;
-  for (int y = ly; y < 32; y += 8) {
-    const int r = tr + y, c = tc + lx;
-    tile[y][lx] = (r < nr && c < nc) ? src[static_cast<size_t>(r) * in_stride + c]
-                                     : make_double2(0.0, 0.0);
-  }
-  __syncthreads();
-  for (int y = ly; y < 32; y += 8) {
-    const int c = tc + y, r = tr + lx;
-    if (c < nc && r < nr) dst[static_cast<size_t>(c) * out_stride + r] = tile[lx][y];
+  double* part = wk.rstat_part + (static_cast<size_t>(w) * gridDim.x + blockIdx.x) * 4;
+  const double s1 = block_sum(m1, red), s2 = block_sum(m2, red);
+  const double q1 = block_sum(v1, red), q2 = block_sum(v2, red);
+  if (tid == 0) {
+    part[0] = s1;
+    part[1] = s2;
+    part[2] = q1;
+    part[3] = q2;
   }
 }
 
 // ===========================================================================
-// colfft2d: forward complex transform (length n) of every kept column
-// YT[k2][:], then the spectrum exp(X - r0) with the shifts into P[k2][k1]
-// (only kept k1).  One workgroup per (k2, walker).
+// colpass2d: for every kept column k2 the spectrum exp(X - r0) with the
+// shifts, times dataset f's noise factor, and the inverse transform into
+// Q[k2][i] (in place of YT's column).  kForward: from YT by the forward
+// transform, the spectrum kept in PR when more datasets follow; else from PR.
+// cg columns together.  Bound by LDS traffic and barriers of the stages:
+// 651 us for 32 walkers at 2048, 534 + 526 as two kernels with the spectrum
+// through memory between them.
 // ===========================================================================
-__global__ __launch_bounds__(kT) void colfft2d_kernel(const Set2Dev s, const Work2 wk) {
+template <bool kForward>
+__global__ __launch_bounds__(kTR) void colpass2d_kernel(const Set2Dev s, const Work2 wk,
+                                                        const int f, const int cg) {
   extern __shared__ double2 lds[];
   const int w = blockIdx.y;
   const double* m = model_ptr(wk, w);
   if (m[0] != POFD_OK) return;
   const int K1 = static_cast<int>(m[3]), K2 = static_cast<int>(m[4]);
-  const int n = s.n;
-  double2* a = lds;
-  double2* b = lds + n;
+  const int n = s.n, ncplx = n / 2 + 1, tid = threadIdx.x;
+  const int T = kTR / cg, grp = tid / T, t = tid & (T - 1);
+  const int swz = swizzle_of(n);
+  double2* tw = lds;
+  double2* a = lds + n / 4 + static_cast<size_t>(grp) * 2 * n;
+  double2* b = a + n;
+  load_turns(tw, s.tw_n, n);
   const double* st = wk.stats + static_cast<size_t>(w) * kStats;
   const double r0 = st[ST2_R0];
   const bool ds1 = st[ST2_DOSHIFT1] != 0.0, ds2 = st[ST2_DOSHIFT2] != 0.0;
   const double sf1 = st[ST2_SHIFT1] * s.iflux1, sf2 = st[ST2_SHIFT2] * s.iflux2;
-  const int ncplx = n / 2 + 1;
-  for (int k2 = blockIdx.x; k2 <= K2; k2 += gridDim.x) {
-    const double2* col = wk.YT + static_cast<size_t>(w) * wk.YT_stride + static_cast<size_t>(k2) * n;
-    for (int t = threadIdx.x; t < n; t += kT) a[t] = col[t];
-    __syncthreads();
-    const double2* X = fft_lds<-1>(a, b, n, s.tw_n);
-    double2* pr = wk.PR + static_cast<size_t>(w) * wk.PR_stride + static_cast<size_t>(k2) * n;
-    for (int k1 = threadIdx.x; k1 < n; k1 += kT) {
-      const bool kept = (k1 <= K1) || (k1 >= n - K1);
-      double2 v = make_double2(0.0, 0.0);
-      if (kept) {
-#pragma clang fp contract(off)
-        const double2 xv = X[k1];
-        const double rval = xv.x - r0;
-        double ival = xv.y;
-        double sp1 = 0.0;
-        if (ds1) sp1 = (k1 < ncplx) ? sf1 * static_cast<double>(k1) : -sf1 * static_cast<double>(n - k1);
-        if (ds1 && ds2)
-          ival = ival - sp1 - sf2 * static_cast<double>(k2);
-        else if (ds1)
-          ival = ival - sp1;
-        else if (ds2)
-          ival = ival - sf2 * static_cast<double>(k2);
-        const double ef = exp(rval);
-        double sn, cs;
-        sincos(ival, &sn, &cs);
-        v = make_double2(ef * cs, ef * sn);
-      }
-      if (k1 == 0 && k2 == 0) v = make_double2(1.0, 0.0);
-      pr[k1] = v;
-    }
-    __syncthreads();
-  }
-}
-
-// ===========================================================================
-// noisecol2d: per dataset, noise factor times the spectrum and the inverse
-// complex transform down every kept column into Q[k2][i]
-// ===========================================================================
-__global__ __launch_bounds__(kT) void noisecol2d_kernel(const Set2Dev s, const Work2 wk,
-                                                        const int f) {
-  extern __shared__ double2 lds[];
-  const int w = blockIdx.y;
-  const double* m = model_ptr(wk, w);
-  if (m[0] != POFD_OK) return;
-  const int K1 = static_cast<int>(m[3]), K2 = static_cast<int>(m[4]);
-  const int n = s.n, ncplx = n / 2 + 1;
-  double2* a = lds;
-  double2* b = lds + n;
   const double sigma1 = m[1] * s.fields[f].sigma_base1;
   const double sigma2 = m[2] * s.fields[f].sigma_base2;
   const bool noisy = (sigma1 > 0 || sigma2 > 0);
   const double sigfac1 = -0.5 * sigma1 * sigma1 * s.iflux1 * s.iflux1;
   const double sigfac2 = -0.5 * sigma2 * sigma2 * s.iflux2 * s.iflux2;
-  for (int k2 = blockIdx.x; k2 <= K2; k2 += gridDim.x) {
-    const double2* pr = wk.PR + static_cast<size_t>(w) * wk.PR_stride + static_cast<size_t>(k2) * n;
-    for (int k1 = threadIdx.x; k1 < n; k1 += kT) {
-      double2 v = pr[k1];
-      const bool kept = (k1 <= K1) || (k1 >= n - K1);
-      if (!kept) {
-        v = make_double2(0.0, 0.0);
-      } else if (noisy) {
+  for (int c0 = blockIdx.x * cg; c0 <= K2; c0 += gridDim.x * cg) {  // uniform
+    const int k2 = c0 + grp;
+    const bool on = k2 <= K2;
+    double2* col = wk.YT + static_cast<size_t>(w) * wk.YT_stride + static_cast<size_t>(k2) * n;
+    double2* pr = wk.PR + static_cast<size_t>(w) * wk.PR_stride + static_cast<size_t>(k2) * n;
+    const double2* X = nullptr;
+    double2* z = a;
+    if (kForward) {
+      if (on)
+        for (int e = t; e < n; e += T) a[slot(e, swz)] = col[e];
+      __syncthreads();
+      X = fft_lds(a, b, n, tw, t, T);
+      z = (X == a) ? b : a;
+    }
+    if (on) {
+      for (int k1 = t; k1 < n; k1 += T) {
+        const bool kept = (k1 <= K1) || (k1 >= n - K1);
+        double2 v = make_double2(0.0, 0.0);
+        if (kept) {
 #pragma clang fp contract(off)
-        const double didx1 = (k1 < ncplx) ? static_cast<double>(k1) : static_cast<double>(n - k1);
-        const double didx2 = static_cast<double>(k2);
-        const double ef = exp(sigfac1 * didx1 * didx1 + sigfac2 * didx2 * didx2);
-        v = make_double2(ef * v.x, ef * v.y);
+          if (kForward) {
+            const double2 xv = X[slot(k1, swz)];
+            const double rval = xv.x - r0;
+            double ival = xv.y;
+            double sp1 = 0.0;
+            if (ds1)
+              sp1 = (k1 < ncplx) ? sf1 * static_cast<double>(k1)
+                                 : -sf1 * static_cast<double>(n - k1);
+            if (ds1 && ds2)
+              ival = ival - sp1 - sf2 * static_cast<double>(k2);
+            else if (ds1)
+              ival = ival - sp1;
+            else if (ds2)
+              ival = ival - sf2 * static_cast<double>(k2);
+            const double ef = exp(rval);
+            double sn, cs;
+            sincos(ival, &sn, &cs);
+            v = make_double2(ef * cs, ef * sn);
+            if (k1 == 0 && k2 == 0) v = make_double2(1.0, 0.0);
+            if (s.nfields > 1) pr[k1] = v;
+          } else {
+            v = pr[k1];
+          }
+          if (noisy) {
+            const double didx1 =
+                (k1 < ncplx) ? static_cast<double>(k1) : static_cast<double>(n - k1);
+            const double didx2 = static_cast<double>(k2);
+            const double ef = exp(sigfac1 * didx1 * didx1 + sigfac2 * didx2 * didx2);
+            v = make_double2(ef * v.x, ef * v.y);
+          }
+          if (k1 == 0 && k2 == 0) v = make_double2(1.0, 0.0);
+        }
+        z[slot(k1, swz)] = make_double2(v.y, v.x);
       }
-      if (k1 == 0 && k2 == 0) v = make_double2(1.0, 0.0);
-      a[k1] = v;
     }
     __syncthreads();
-    const double2* q = fft_lds<+1>(a, b, n, s.tw_n);
-    double2* Q = wk.Q + static_cast<size_t>(w) * wk.Q_stride + static_cast<size_t>(k2) * n;
-    for (int i = threadIdx.x; i < n; i += kT) Q[i] = q[i];
+    const double2* q = fft_lds(z, (z == a) ? b : a, n, tw, t, T);
+    if (on)
+      for (int i = t; i < n; i += T) {
+        const double2 v = q[slot(i, swz)];
+        col[i] = make_double2(v.y, v.x);
+      }
     __syncthreads();
   }
 }
 
 // ===========================================================================
-// rowifft2d: c2r of every row from QT[i][0..n/2] (zero beyond K2), clamp,
-// store P and the row trapezoid marginal
+// rowifft2d: c2r of every row from Q[0..n/2][i] (zero beyond K2), clamp,
+// store P, the row trapezoid marginal and this workgroup's share of the
+// column one.  rg rows together, as rowfft2d.  Bound by LDS traffic and
+// barriers of the stages: 673 us for 32 walkers at 2048, 195 + 642 as a
+// transposition and the rows.
 // ===========================================================================
-__global__ __launch_bounds__(kT) void rowifft2d_kernel(const Set2Dev s, const Work2 wk,
-                                                       const int f) {
+__global__ __launch_bounds__(kTR) void rowifft2d_kernel(const Set2Dev s, const Work2 wk,
+                                                        const int f, const int rg) {
   extern __shared__ double2 lds[];
-  __shared__ double red[kT / 64];
+  __shared__ double red[kTR / 64];
   const int w = blockIdx.y;
   const double* m = model_ptr(wk, w);
   if (m[0] != POFD_OK) return;
   const int K2 = static_cast<int>(m[4]);
-  const int n = s.n, h = n / 2;
-  double2* a = lds;
-  double2* b = lds + h;
+  const int n = s.n, h = n / 2, tid = threadIdx.x;
+  const int T = kTR / rg, grp = tid / T, t = tid & (T - 1);
+  const int swz = swizzle_of(h);
+  double2* tw = lds;
+  double2* rows = lds + h / 4;
+  const int rs = n + 2;
+  load_turns(tw, s.tw_half, h);
   const size_t wf = static_cast<size_t>(w) * s.nfields + f;
-  constexpr int kMaxPairs = 4096 / 2 / kT;  // output pairs per thread, n <= 4096
+  const double2* Q = wk.YT + static_cast<size_t>(w) * wk.YT_stride;
   double cacc[2 * kMaxPairs];
 #pragma unroll
   for (int q = 0; q < 2 * kMaxPairs; ++q) cacc[q] = 0.0;
-  for (int i = blockIdx.x; i < n; i += gridDim.x) {
-    const double2* X = wk.QT + static_cast<size_t>(w) * wk.QT_stride + static_cast<size_t>(i) * wk.ystride;
-    for (int k = threadIdx.x; k < h; k += kT) {
-      double2 xa = (k <= K2) ? X[k] : make_double2(0.0, 0.0);
-      const int mk = h - k;
-      double2 xb = (mk <= K2) ? X[mk] : make_double2(0.0, 0.0);
+  for (int i0 = blockIdx.x * rg; i0 < n; i0 += gridDim.x * rg) {
+    for (int o = tid; o < rg * (h / 2 + 1); o += kTR) {
+      const int k = o / rg, row = o - k * rg, mk = h - k;
+      const double2* X = Q + i0 + row;
+      double2 xa = (k <= K2) ? X[static_cast<size_t>(k) * n] : make_double2(0.0, 0.0);
+      double2 xb = (mk <= K2) ? X[static_cast<size_t>(mk) * n] : make_double2(0.0, 0.0);
       if (k == 0) {  // FFTW's c2r ignores Im of the k2 = 0 and n/2 entries
         xa.y = 0.0;
         xb.y = 0.0;
       }
       const double2 E = make_double2(xa.x + xb.x, xa.y - xb.y);
       const double2 D = make_double2(xa.x - xb.x, xa.y + xb.y);
-      const double2 wv = make_double2(s.tw_n[k].x, -s.tw_n[k].y);  // e^{+2 pi i k/n}
-      const double2 O = cmul(D, wv);
-      a[k] = make_double2(E.x - O.y, E.y + O.x);
+      const double2 wv = s.tw_n[k];  // e^{-2 pi i k/n}
+      const double2 O = cmul(D, make_double2(wv.x, -wv.y));
+      double2* a = rows + row * rs;  // (real and imaginary parts exchanged)
+      a[slot(k, swz)] = make_double2(E.y + O.x, E.x - O.y);
+      if (k > 0 && k < mk) {  // h - k: conj E, -conj D, and the turn -wv
+        const double2 O2 = cmul(make_double2(D.x, -D.y), wv);
+        a[slot(mk, swz)] = make_double2(-E.y + O2.x, E.x - O2.y);
+      }
     }
     __syncthreads();
-    const double2* z = fft_lds<+1>(a, b, h, s.tw_half);
-    double* P = wk.P + wf * wk.P_stride + static_cast<size_t>(i) * n;
+    const int i = i0 + grp;
+    double2* a = rows + grp * rs;
+    const double2* z = fft_lds(a, a + h, h, tw, t, T);
+    double2* P = reinterpret_cast<double2*>(wk.P + wf * wk.P_stride + static_cast<size_t>(i) * n);
     const double wi = (i == 0 || i == n - 1) ? 0.5 : 1.0;
     double part = 0.0;
 #pragma unroll
     for (int q = 0; q < kMaxPairs; ++q) {
-      const int m2 = threadIdx.x + q * kT;
+      const int m2 = t + q * T;
       if (m2 < h) {
-        double x0 = z[m2].x, x1 = z[m2].y;
-        if (x0 < 0) x0 = 0.0;  // unwrapAndNormalizePD positivity
-        if (x1 < 0) x1 = 0.0;
-        P[2 * m2] = x0;
-        P[2 * m2 + 1] = x1;
-        const double w0 = (2 * m2 == 0) ? 0.5 : 1.0;
-        const double w1 = (2 * m2 + 1 == n - 1) ? 0.5 : 1.0;
+        const double2 v = z[slot(m2, swz)];
+        // unwrapAndNormalizePD positivity
+        const double x0 = (v.y < 0) ? 0.0 : v.y, x1 = (v.x < 0) ? 0.0 : v.x;
+        P[m2] = make_double2(x0, x1);
+        const double w0 = (m2 == 0) ? 0.5 : 1.0;
+        const double w1 = (m2 == h - 1) ? 0.5 : 1.0;
         part += w0 * x0 + w1 * x1;
         cacc[2 * q] += wi * x0;
         cacc[2 * q + 1] += wi * x1;
       }
     }
-    const double rs = block_sum(part, red);
-    if (threadIdx.x == 0) wk.rsum1[wf * wk.edge_stride + i] = rs;
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) part += __shfl_xor(part, o);
+    if ((tid & 63) == 0) red[tid >> 6] = part;
+    __syncthreads();
+    if (t == 0) {
+      double v = red[tid >> 6];
+      for (int u = 1; u < T / 64; ++u) v += red[(tid >> 6) + u];
+      wk.rsum1[wf * wk.edge_stride + i] = v;
+    }
+    // (red is written again behind the next transform's barriers)
   }
-  // this workgroup's share of the column trapezoid sums
-  double* cp = wk.colpart + static_cast<size_t>(w) * wk.colpart_stride +
-               static_cast<size_t>(blockIdx.x) * n;
+  // the column sums of the rg rows' threads, in row order
+  __syncthreads();
+  double2* cs = rows;
 #pragma unroll
   for (int q = 0; q < kMaxPairs; ++q) {
-    const int m2 = threadIdx.x + q * kT;
-    if (m2 < h) {
-      cp[2 * m2] = cacc[2 * q];
-      cp[2 * m2 + 1] = cacc[2 * q + 1];
-    }
+    const int m2 = t + q * T;
+    if (m2 < h) cs[grp * h + m2] = make_double2(cacc[2 * q], cacc[2 * q + 1]);
+  }
+  __syncthreads();
+  double2* cp = reinterpret_cast<double2*>(wk.colpart + static_cast<size_t>(w) * wk.colpart_stride +
+                                           static_cast<size_t>(blockIdx.x) * n);
+  for (int e = tid; e < h; e += kTR) {
+    double2 v = cs[e];
+    for (int u = 1; u < rg; ++u) v = cadd(v, cs[u * h + e]);
+    cp[e] = v;
   }
 }
 
@@ -1231,37 +1286,11 @@ __global__ void combine2d_kernel(const Set2Dev s, const Work2 wk, const int accu
   loglike[w] = prev + total;
 }
 
-// combine the rstats partials, decide the shifts, record r0 (after rowfft/
-// colfft of column k2 = 0 this is done by colfft's input: r0 = sum R)
-__global__ void rstats2d_final_kernel(const Set2Dev s, const Work2 wk, const int nparts) {
-  const int w = blockIdx.x * blockDim.x + threadIdx.x;
-  if (w >= wk.nwalk) return;
-  if (model_ptr(wk, w)[0] != POFD_OK) return;
-  const double* part = wk.rstat_part + static_cast<size_t>(w) * nparts * 4;
-  double m1 = 0, m2 = 0, v1 = 0, v2 = 0;
-  for (int b = 0; b < nparts; ++b) {
-    m1 += part[4 * b];
-    m2 += part[4 * b + 1];
-    v1 += part[4 * b + 2];
-    v2 += part[4 * b + 3];
-  }
-  double* st = wk.stats + static_cast<size_t>(w) * kStats;
-  st[ST2_MN1] = m1;
-  st[ST2_MN2] = m2;
-  st[ST2_VAR1] = v1;
-  st[ST2_VAR2] = v2;
-  const double sg1 = sqrt(v1), sg2 = sqrt(v2);
-  const bool d1 = (sg1 > s.dflux1) && (fabs(m1) > s.dflux1);
-  const bool d2 = (sg2 > s.dflux2) && (fabs(m2) > s.dflux2);
-  st[ST2_DOSHIFT1] = d1 ? 1.0 : 0.0;
-  st[ST2_DOSHIFT2] = d2 ? 1.0 : 0.0;
-  st[ST2_SHIFT1] = d1 ? -m1 : 0.0;
-  st[ST2_SHIFT2] = d2 ? -m2 : 0.0;
-}
-
-// r0 = Re X[0][0]: the k2 = 0 column transform at k1 = 0 is the sum of the
-// k2 = 0 row outputs; computed by one block per walker before colfft2d
-__global__ __launch_bounds__(kT) void r0_2d_kernel(const Set2Dev s, const Work2 wk) {
+// combine the moments' partials, decide the shifts, and r0 = Re X[0][0]: the
+// k2 = 0 column transform at k1 = 0 is the sum of the k2 = 0 row outputs;
+// one workgroup per walker
+__global__ __launch_bounds__(kT) void rstats2d_kernel(const Set2Dev s, const Work2 wk,
+                                                      const int nparts) {
   __shared__ double red[kT / 64];
   const int w = blockIdx.x;
   if (model_ptr(wk, w)[0] != POFD_OK) return;
@@ -1269,7 +1298,25 @@ __global__ __launch_bounds__(kT) void r0_2d_kernel(const Set2Dev s, const Work2 
   double a = 0.0;
   for (int i = threadIdx.x; i < s.n; i += kT) a += col[i].x;
   const double r0 = block_sum(a, red);
-  if (threadIdx.x == 0) wk.stats[static_cast<size_t>(w) * kStats + ST2_R0] = r0;
+  const double* part = wk.rstat_part + static_cast<size_t>(w) * nparts * 4;
+  double mom[4] = {0.0, 0.0, 0.0, 0.0};
+  for (int b = threadIdx.x; b < nparts; b += kT)
+    for (int q = 0; q < 4; ++q) mom[q] += part[4 * b + q];
+  for (int q = 0; q < 4; ++q) mom[q] = block_sum(mom[q], red);
+  if (threadIdx.x != 0) return;
+  double* st = wk.stats + static_cast<size_t>(w) * kStats;
+  st[ST2_R0] = r0;
+  st[ST2_MN1] = mom[0];
+  st[ST2_MN2] = mom[1];
+  st[ST2_VAR1] = mom[2];
+  st[ST2_VAR2] = mom[3];
+  const double sg1 = sqrt(mom[2]), sg2 = sqrt(mom[3]);
+  const bool d1 = (sg1 > s.dflux1) && (fabs(mom[0]) > s.dflux1);
+  const bool d2 = (sg2 > s.dflux2) && (fabs(mom[1]) > s.dflux2);
+  st[ST2_DOSHIFT1] = d1 ? 1.0 : 0.0;
+  st[ST2_DOSHIFT2] = d2 ? 1.0 : 0.0;
+  st[ST2_SHIFT1] = d1 ? -mom[0] : 0.0;
+  st[ST2_SHIFT2] = d2 ? -mom[1] : 0.0;
 }
 
 }  // namespace pofd2
@@ -1296,9 +1343,12 @@ int launch_loglike2d(const Set2Dev& s, const Work2& wk, const RGrid& gmain,
                               static_cast<int>(rg_lds));
   const int rblocks = 64;  // row blocks per walker (grid-stride over rows)
   // one R grid: its per-row beam pieces, then the grid
-  auto rgrid = [&](const RGrid& g, const int blocks) {
+  auto pieces = [&](const RGrid& g) {
     const int pb = static_cast<int>((static_cast<size_t>(g.n1) * (wk.rpieces_w / 3) + kT - 1) / kT);
     hipLaunchKernelGGL(rpieces2d_kernel, dim3(pb, W), dim3(kT), 0, st, s, wk, g);
+  };
+  auto rgrid = [&](const RGrid& g, const int blocks) {
+    pieces(g);
     hipLaunchKernelGGL(rgrid2d_kernel, dim3(blocks, W), dim3(kT), rg_lds, st, s, wk, g);
   };
   mark(POFD_STAGE_PREP);
@@ -1316,44 +1366,30 @@ int launch_loglike2d(const Set2Dev& s, const Work2& wk, const RGrid& gmain,
                        n, wk.ey, gy.wstride, wk.ry, wk.edge_stride, 0.0);
     hipLaunchKernelGGL(edge2d_cols_kernel, dim3((n + 255) / 256, W), dim3(256), 0, st, s, wk);
   }
-  rgrid(gmain, rblocks * 4);
+  pieces(gmain);
   if (s.edge_integ)
-    hipLaunchKernelGGL(edge2d_patch_kernel, dim3((n + 255) / 256, W), dim3(256), 0, st, s, wk);
+    hipLaunchKernelGGL(edge2d_r00_kernel, dim3((W + 63) / 64), dim3(64), 0, st, s, wk);
   const int nparts = 64;
-  hipLaunchKernelGGL(rstats2d_kernel, dim3(nparts, W), dim3(kT), 0, st, s, wk);
-  hipLaunchKernelGGL(rstats2d_final_kernel, dim3((W + 63) / 64), dim3(64), 0, st, s, wk, nparts);
-  const size_t lds_row = static_cast<size_t>(n) * sizeof(double2);      // 2 x n/2
-  const size_t lds_col = static_cast<size_t>(2 * n) * sizeof(double2);  // 2 x n
-  if (lds_row + 1024 > 65536) {  // n = 4096: 64 KB plus the static reduction slots
-    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(rowfft2d_kernel),
-                              hipFuncAttributeMaxDynamicSharedMemorySize,
+  const int rg = rows_together(n), cg = cols_together(n);
+  // a quarter turn of twiddles and both buffers of each row or column
+  const size_t lds_row = (static_cast<size_t>(n / 8) + rg * (n + 2)) * sizeof(double2);
+  const size_t lds_col = (static_cast<size_t>(n / 4) + cg * 2 * n) * sizeof(double2);
+  for (const void* k : {reinterpret_cast<const void*>(rowfft2d_kernel),
+                        reinterpret_cast<const void*>(rowifft2d_kernel)})
+    (void)hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize,
                               static_cast<int>(lds_row));
-    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(rowifft2d_kernel),
-                              hipFuncAttributeMaxDynamicSharedMemorySize,
-                              static_cast<int>(lds_row));
-  }
-  if (lds_col > 65536) {  // n = 4096: 128 KB of the CU's 160 KB
-    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(colfft2d_kernel),
-                              hipFuncAttributeMaxDynamicSharedMemorySize,
+  for (const void* k : {reinterpret_cast<const void*>(colpass2d_kernel<true>),
+                        reinterpret_cast<const void*>(colpass2d_kernel<false>)})
+    (void)hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize,
                               static_cast<int>(lds_col));
-    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(noisecol2d_kernel),
-                              hipFuncAttributeMaxDynamicSharedMemorySize,
-                              static_cast<int>(lds_col));
-  }
-  hipLaunchKernelGGL(rowfft2d_kernel, dim3(256, W), dim3(kT), lds_row, st, s, wk);
-  const int nc = n / 2 + 1;
-  hipLaunchKernelGGL(transpose2d_kernel, dim3((nc + 31) / 32, (n + 31) / 32, W), dim3(kT), 0, st,
-                     wk, static_cast<const double2*>(wk.Y), wk.Y_stride, wk.ystride, wk.YT,
-                     wk.YT_stride, n, n, nc, 1);
-  hipLaunchKernelGGL(r0_2d_kernel, dim3(W), dim3(kT), 0, st, s, wk);
-  hipLaunchKernelGGL(colfft2d_kernel, dim3(64, W), dim3(kT), lds_col, st, s, wk);
+  hipLaunchKernelGGL(rowfft2d_kernel, dim3(nparts, W), dim3(kTR), lds_row, st, s, wk, gmain, rg);
+  hipLaunchKernelGGL(rstats2d_kernel, dim3(W), dim3(kT), 0, st, s, wk, nparts);
   mark(POFD_STAGE_INVERSE);
   for (int f = 0; f < s.nfields; ++f) {
-    hipLaunchKernelGGL(noisecol2d_kernel, dim3(64, W), dim3(kT), lds_col, st, s, wk, f);
-    hipLaunchKernelGGL(transpose2d_kernel, dim3((n + 31) / 32, (nc + 31) / 32, W), dim3(kT), 0,
-                       st, wk, static_cast<const double2*>(wk.Q), wk.Q_stride, n, wk.QT,
-                       wk.QT_stride, wk.ystride, nc, n, 2);
-    hipLaunchKernelGGL(rowifft2d_kernel, dim3(kRowBlocks2, W), dim3(kT), lds_row, st, s, wk, f);
+    hipLaunchKernelGGL(f == 0 ? colpass2d_kernel<true> : colpass2d_kernel<false>, dim3(64, W),
+                       dim3(kTR), lds_col, st, s, wk, f, cg);
+    hipLaunchKernelGGL(rowifft2d_kernel, dim3(kRowBlocks2, W), dim3(kTR), lds_row, st, s, wk, f,
+                       rg);
     hipLaunchKernelGGL(colsum2d_kernel, dim3((n + 255) / 256, W), dim3(256), 0, st, s, wk, f);
   }
   mark(POFD_STAGE_FINALIZE);

@@ -1,0 +1,49 @@
+"""The two-band transforms at the grid sizes where their work divides
+differently: eight short rows a workgroup (and transforms too short for the
+swizzled order), four and two long ones, one column at the largest grid; odd
+and even powers of two, with and without the edge integrals, and a second
+dataset, against the CPU oracle."""
+import numpy as np
+import pytest
+
+from oracle2d_side import build_oracle2d, make_inputs2d
+from pofd_affine_amd import synth2d, workload2d
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("n,nedge,edge,nwalk", [
+    (64, 16, True, 3), (128, 16, False, 3), (256, 32, True, 5), (512, 64, False, 3),
+    (1024, 64, True, 2), (4096, 32, True, 1)])
+def test_sizes_against_oracle(n, nedge, edge, nwalk):
+    print("[gpu2d-size-case] %d edge=%s" % (n, edge), flush=True)
+    inp = make_inputs2d(npix_side=60, seed=5, nbins=40, nbeamhist=30)
+    th0 = synth2d.true_theta()
+    th = synth2d.walker_thetas(nwalk, seed=17)
+    ctx = workload2d.build_context2d(inp, n, th0, nedge=nedge, edge_integ=edge)
+    L = build_oracle2d(inp, n, th0, nedge=nedge, edge_integ=edge)
+    ll, st = ctx.loglike2d_batch(th)
+    ref, rst = L.loglike_batch(th, nwalk)
+    assert np.array_equal(st, rst), (st, rst)
+    ok = st == 0
+    # the contract of every 2D path: 1e-6 of the oracle
+    np.testing.assert_allclose(ll[ok], ref[ok], rtol=0, atol=1e-6)
+
+
+@pytest.mark.parametrize("n", [64, 512, 4096])
+def test_second_dataset_is_the_first(n):
+    """The same pixels as the second dataset take the other column pass: the
+    likelihood doubles (the stored spectrum is the first pass's)."""
+    print("[gpu2d-size-case] two datasets %d" % n, flush=True)
+    inp = make_inputs2d(npix_side=60, seed=5, nbins=40, nbeamhist=30)
+    th0 = synth2d.true_theta()
+    th = synth2d.walker_thetas(2, seed=18)
+    one = workload2d.build_context2d(inp, n, th0, nedge=16)
+    two = workload2d.build_context2d(inp, n, th0, nedge=16)
+    two.add_field2d(0, inp["d1"], inp["d2"], synth2d.SIGMA1, synth2d.SIGMA2)
+    two.prepare2d(th0)
+    a, sa = one.loglike2d_batch(th)
+    b, sb = two.loglike2d_batch(th)
+    assert np.array_equal(sa, sb)
+    ok = sa == 0
+    assert np.array_equal(b[ok], a[ok] + a[ok])
