@@ -96,13 +96,13 @@ int forward(pofd_mlp* s, int n) {
     const bf16* W = s->wb + s->off[2 * l];
     const float* b = s->w + s->off[2 * l + 1];
     // Z = in . W^T + b: A(m,k) = in[m*K + k]; B(k,n) = W[n*K + k]
-    rc |= md::gemm(0, in, K, 0, 0, W, K, 1, s->Z[l], H, b, n, H, K, s->stream);
-    rc |= md::gelu_fwd(s->Z[l], s->A[l], static_cast<size_t>(n) * H, s->stream);
+    rc |= md::gemm(0, in, K, 0, 0, W, K, 1, s->Z[l], H, b, nullptr, s->A[l], n, H, K,
+                   s->stream);
     in = s->A[l];
     K = H;
   }
-  rc |= md::gemm(0, in, H, 0, 0, s->wb + s->off[6], H, 1, s->out, 1, s->w + s->off[7], n, 1, H,
-                 s->stream);
+  rc |= md::gemm(0, in, H, 0, 0, s->wb + s->off[6], H, 1, s->out, 1, s->w + s->off[7],
+                 nullptr, nullptr, n, 1, H, s->stream);
   return rc;
 }
 
@@ -111,26 +111,25 @@ int backward(pofd_mlp* s, int n) {
   const int H = s->H;
   int rc = md::mse_grad(s->out, s->y, n, s->dout, s->se, s->stream);
   // output layer: gW4[0][j] = sum_m dout[m] A3[m][j]; gb4 = sum dout
-  rc |= md::gemm(1, s->dout, n, 0, 0, s->A[2], H, 0, s->g + s->off[6], H, nullptr, 1, H, n,
-                 s->stream);
+  rc |= md::gemm(1, s->dout, n, 0, 0, s->A[2], H, 0, s->g + s->off[6], H, nullptr, nullptr,
+                 nullptr, 1, H, n, s->stream);
   rc |= md::colsum(s->dout, n, 1, s->g + s->off[7], s->stream);
-  // dA3 = dout . W4
-  rc |= md::gemm(1, s->dout, 1, 0, 0, s->wb + s->off[6], H, 0, s->dA, H, nullptr, n, H, 1,
-                 s->stream);
+  // dZ3 = (dout . W4) gelu'(Z3)
+  rc |= md::gemm(1, s->dout, 1, 0, 0, s->wb + s->off[6], H, 0, s->dA, H, nullptr, s->Z[2],
+                 nullptr, n, H, 1, s->stream);
   float* dA = s->dA;
   float* dnext = s->dA2;
   for (int l = 2; l >= 0; --l) {
-    rc |= md::gelu_bwd(s->Z[l], dA, static_cast<size_t>(n) * H, s->stream);  // dZ
     const int K = (l == 0) ? s->nin : H;
     const bf16* in = (l == 0) ? s->X : s->A[l - 1];
     // gW[o][i] = sum_m dZ[m][o] in[m][i]
-    rc |= md::gemm(1, dA, H, 1, 0, in, K, 0, s->g + s->off[2 * l], K, nullptr, H, K, n,
-                   s->stream);
+    rc |= md::gemm(1, dA, H, 1, 0, in, K, 0, s->g + s->off[2 * l], K, nullptr, nullptr,
+                   nullptr, H, K, n, s->stream);
     rc |= md::colsum(dA, n, H, s->g + s->off[2 * l + 1], s->stream);
     if (l > 0) {
-      // dA_prev[m][i] = sum_o dZ[m][o] W[o][i]
-      rc |= md::gemm(1, dA, H, 0, 0, s->wb + s->off[2 * l], H, 0, dnext, H, nullptr, n, H, H,
-                     s->stream);
+      // dZ_prev[m][i] = gelu'(Z_prev[m][i]) sum_o dZ[m][o] W[o][i]
+      rc |= md::gemm(1, dA, H, 0, 0, s->wb + s->off[2 * l], H, 0, dnext, H, nullptr,
+                     s->Z[l - 1], nullptr, n, H, H, s->stream);
       std::swap(dA, dnext);
     }
   }

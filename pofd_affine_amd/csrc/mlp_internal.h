@@ -12,14 +12,12 @@ typedef uint16_t bf16;  // bfloat16 bit pattern
 
 // C[m][n] = sum_k A(m,k) B(k,n) (+ bias[n]) with FP32 accumulation.
 // A(m,k) = ta ? A[k*lda + m] : A[m*lda + k]; B(k,n) likewise with tb.
-// Element types: bf16 (0) or float (1) for A and B; C is float.
+// Element types: bf16 (0) or float (1) for A and B; C is float.  With zg, C
+// is multiplied by gelu'(zg) (both [m][n], ldc); with act, gelu(C) goes there
+// as bf16.
 int gemm(int atype, const void* A, int lda, int ta, int btype, const void* B, int ldb, int tb,
-         float* C, int ldc, const float* bias, int M, int N, int K, hipStream_t st);
-
-// out_bf16 = gelu(z) (z already includes the bias)
-int gelu_fwd(const float* z, bf16* out, size_t n, hipStream_t st);
-// dz = dA * gelu'(z), in place on dA
-int gelu_bwd(const float* z, float* dA, size_t n, hipStream_t st);
+         float* C, int ldc, const float* bias, const float* zg, bf16* act, int M, int N, int K,
+         hipStream_t st);
 // float -> bf16 (round to nearest even)
 int to_bf16(const float* in, bf16* out, size_t n, hipStream_t st);
 // whitened inputs: x[r][i] = sum_j wz[i][j] (src[r*stride + idx[j]] - mean[j]),

@@ -17,114 +17,122 @@ __device__ __forceinline__ float ld(const void* p, size_t i) {
   return static_cast<const float*>(p)[i];
 }
 
-constexpr int kTile = 64, kKs = 32;
+__device__ __forceinline__ float gelu(const float x) {
+  return 0.5f * x * (1.0f + erff(x * 0.70710678118654752f));
+}
+__device__ __forceinline__ float gelu_grad(const float x) {
+  const float cdf = 0.5f * (1.0f + erff(x * 0.70710678118654752f));
+  const float pdf = 0.39894228040143268f * expf(-0.5f * x * x);
+  return cdf + x * pdf;
+}
 
-// One K-slice of A and B into registers (kKs x 64 of each per workgroup,
-// 8 values per thread); zeros outside the matrices.
-template <int TA, int TB>
-__device__ __forceinline__ void load_slice(const void* A, int lda, int ta, const void* B, int ldb,
-                                           int tb, int M, int N, int K, int m0, int n0, int k0,
-                                           float* va, float* vb) {
-  const int tid = threadIdx.x;
-  const bool inner = (m0 + kTile <= M) && (n0 + kTile <= N) && (k0 + kKs <= K);
+// One K-slice (kKs long) of a tile's kTile rows of A, or columns of B, into
+// registers, 8 values per thread: element o of the tile at depth k is at
+// p[k ld + o] (along) or p[o ld + k], and neighbouring lanes take
+// neighbouring addresses.  Zeros outside the matrix (loaded from its edge, so
+// that no load waits behind a branch).
+template <int T, int kTile, int kKs>
+__device__ __forceinline__ void load_slice(const void* p, const int ld, const int along,
+                                           const int O, const int K, const int o0, const int k0,
+                                           float* v) {
 #pragma unroll
   for (int q = 0; q < kKs * kTile / 256; ++q) {
-    const int e = tid + 256 * q;
-    const int kk = e / kTile, mm = e % kTile;
-    const int m = m0 + mm, n = n0 + mm, k = k0 + kk;
-    if (inner) {  // uniform over the workgroup: unguarded loads
-      va[q] = ld<TA>(A, ta ? static_cast<size_t>(k) * lda + m : static_cast<size_t>(m) * lda + k);
-      vb[q] = ld<TB>(B, tb ? static_cast<size_t>(n) * ldb + k : static_cast<size_t>(k) * ldb + n);
-    } else {
-      va[q] = (m < M && k < K)
-                  ? ld<TA>(A, ta ? static_cast<size_t>(k) * lda + m : static_cast<size_t>(m) * lda + k)
-                  : 0.0f;
-      vb[q] = (n < N && k < K)
-                  ? ld<TB>(B, tb ? static_cast<size_t>(n) * ldb + k : static_cast<size_t>(k) * ldb + n)
-                  : 0.0f;
-    }
+    const int e = static_cast<int>(threadIdx.x) + 256 * q;
+    const int oo = along ? e % kTile : e / kKs, kk = along ? e / kTile : e % kKs;
+    const int o = o0 + oo, k = k0 + kk;
+    const int oc = min(o, O - 1), kc = min(k, K - 1);
+    const size_t at =
+        along ? static_cast<size_t>(kc) * ld + oc : static_cast<size_t>(oc) * ld + kc;
+    const float x = pofd_mlp_dev::ld<T>(p, at);
+    v[q] = (o < O && k < K) ? x : 0.0f;
+  }
+}
+template <int kTile, int kKs>
+__device__ __forceinline__ void store_slice(float (*s)[kTile + 1], const int along,
+                                            const float* v) {
+#pragma unroll
+  for (int q = 0; q < kKs * kTile / 256; ++q) {
+    const int e = static_cast<int>(threadIdx.x) + 256 * q;
+    const int oo = along ? e % kTile : e / kKs, kk = along ? e / kTile : e % kKs;
+    s[kk][oo] = v[q];
   }
 }
 
-// C = A B (+ bias) on the matrix cores in float: a 64 x 64 tile per
-// workgroup of four waves, each wave 2 x 2 tiles of v_mfma_f32_16x16x4_f32
+// C = A B (+ bias) on the matrix cores in float: a kTile x kTile tile per
+// workgroup of four waves, each wave kW x kW tiles of v_mfma_f32_16x16x4_f32
 // (lane l holds A[l%16][l/16] and B[l/16][l%16] of a 16 x 4 / 4 x 16 step
-// and receives D[4(l/16)..+3][l%16]).  The next K-slice is loaded into
-// registers while the current one is multiplied out of LDS.
+// and receives D[4(l/16)..+3][l%16]), K in ascending order whatever the
+// tile.  The next K-slice is loaded into registers while the current one is
+// multiplied out of LDS.  What follows the product element by element is
+// done here: C times gelu'(zg), or gelu(C) as bf16 into act.
+// Bound by the latency of the slices, K / kKs of them, at the sizes of a
+// training batch: 512 x 256 x 256 takes 8 us, 256 x 256 x 512 with a float
+// operand 16; 22 and 42 with lanes along the tile whatever the layout, slices
+// of 32 and 64 x 64 tiles.
 typedef float float4m __attribute__((ext_vector_type(4)));
 
-template <int TA, int TB>
+template <int TA, int TB, int kTile, int kKs>
 __global__ __launch_bounds__(256) void gemm_kernel(const void* A, int lda, int ta, const void* B,
                                                    int ldb, int tb, float* C, int ldc,
-                                                   const float* bias, int M, int N, int K) {
-  __shared__ float As[kKs][kTile + 4];
-  __shared__ float Bs[kKs][kTile + 4];
+                                                   const float* bias, const float* zg, bf16* act,
+                                                   int M, int N, int K) {
+  __shared__ float As[kKs][kTile + 1];
+  __shared__ float Bs[kKs][kTile + 1];
+  constexpr int kW = kTile / 32;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int m0 = blockIdx.y * kTile, n0 = blockIdx.x * kTile;
-  const int wm = (wave >> 1) * 32, wn = (wave & 1) * 32;
+  const int wm = (wave >> 1) * 16 * kW, wn = (wave & 1) * 16 * kW;
   const int li = lane & 15, lk = lane >> 4;
-  float4m acc[2][2];
+  float4m acc[kW][kW];
 #pragma unroll
-  for (int i = 0; i < 2; ++i)
+  for (int i = 0; i < kW; ++i)
 #pragma unroll
-    for (int j = 0; j < 2; ++j) acc[i][j] = float4m{0.0f, 0.0f, 0.0f, 0.0f};
+    for (int j = 0; j < kW; ++j) acc[i][j] = float4m{0.0f, 0.0f, 0.0f, 0.0f};
   constexpr int kPer = kKs * kTile / 256;
   float va[kPer], vb[kPer];
-  load_slice<TA, TB>(A, lda, ta, B, ldb, tb, M, N, K, m0, n0, 0, va, vb);
+  load_slice<TA, kTile, kKs>(A, lda, ta, M, K, m0, 0, va);
+  load_slice<TB, kTile, kKs>(B, ldb, !tb, N, K, n0, 0, vb);
   for (int k0 = 0; k0 < K; k0 += kKs) {
-#pragma unroll
-    for (int q = 0; q < kPer; ++q) {
-      const int e = tid + 256 * q;
-      As[e / kTile][e % kTile] = va[q];
-      Bs[e / kTile][e % kTile] = vb[q];
-    }
+    store_slice<kTile, kKs>(As, ta, va);
+    store_slice<kTile, kKs>(Bs, !tb, vb);
     __syncthreads();
-    if (k0 + kKs < K)
-      load_slice<TA, TB>(A, lda, ta, B, ldb, tb, M, N, K, m0, n0, k0 + kKs, va, vb);
+    if (k0 + kKs < K) {
+      load_slice<TA, kTile, kKs>(A, lda, ta, M, K, m0, k0 + kKs, va);
+      load_slice<TB, kTile, kKs>(B, ldb, !tb, N, K, n0, k0 + kKs, vb);
+    }
 #pragma unroll
     for (int kk = 0; kk < kKs; kk += 4) {
-      float a[2], b[2];
+      float a[kW], b[kW];
 #pragma unroll
-      for (int i = 0; i < 2; ++i) a[i] = As[kk + lk][wm + 16 * i + li];
+      for (int i = 0; i < kW; ++i) a[i] = As[kk + lk][wm + 16 * i + li];
 #pragma unroll
-      for (int j = 0; j < 2; ++j) b[j] = Bs[kk + lk][wn + 16 * j + li];
+      for (int j = 0; j < kW; ++j) b[j] = Bs[kk + lk][wn + 16 * j + li];
 #pragma unroll
-      for (int i = 0; i < 2; ++i)
+      for (int i = 0; i < kW; ++i)
 #pragma unroll
-        for (int j = 0; j < 2; ++j)
+        for (int j = 0; j < kW; ++j)
           acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i], b[j], acc[i][j], 0, 0, 0);
     }
     __syncthreads();
   }
 #pragma unroll
-  for (int i = 0; i < 2; ++i)
+  for (int i = 0; i < kW; ++i)
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
+    for (int j = 0; j < kW; ++j) {
       const int n = n0 + wn + 16 * j + li;
       if (n >= N) continue;
       const float bn = bias ? bias[n] : 0.0f;
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
         const int m = m0 + wm + 16 * i + 4 * lk + q;
-        if (m < M) C[static_cast<size_t>(m) * ldc + n] = acc[i][j][q] + bn;
+        if (m >= M) continue;
+        const size_t at = static_cast<size_t>(m) * ldc + n;
+        float v = acc[i][j][q] + bn;
+        if (zg) v *= gelu_grad(zg[at]);
+        C[at] = v;
+        if (act) act[at] = f2bf(gelu(v));
       }
     }
-}
-
-__global__ void gelu_fwd_kernel(const float* z, bf16* out, size_t n) {
-  const size_t i = static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const float x = z[i];
-  out[i] = f2bf(0.5f * x * (1.0f + erff(x * 0.70710678118654752f)));
-}
-
-__global__ void gelu_bwd_kernel(const float* z, float* dA, size_t n) {
-  const size_t i = static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const float x = z[i];
-  const float cdf = 0.5f * (1.0f + erff(x * 0.70710678118654752f));
-  const float pdf = 0.39894228040143268f * expf(-0.5f * x * x);
-  dA[i] *= cdf + x * pdf;
 }
 
 __global__ void to_bf16_kernel(const float* in, bf16* out, size_t n) {
@@ -156,18 +164,28 @@ __global__ void gather_rows_kernel(const float* tx, const float* ty, const int* 
     y[r] = ty[row];
 }
 
-// column sums: a workgroup of 256 threads per 64 columns, 4 row phases
-// reduced through LDS in a fixed order
+// column sums: a workgroup of 256 threads per 16 columns, 16 row phases
+// reduced through LDS by halves.  Bound by the latency of M / 64 rounds of
+// four loads: 4.5 us for 512 x 256, where 64 columns a workgroup and four
+// phases took 22.
 __global__ __launch_bounds__(256) void colsum_kernel(const float* dz, int M, int N, float* g) {
-  __shared__ float part[4][64];
-  const int c = threadIdx.x & 63, ph = threadIdx.x >> 6;
-  const int n = blockIdx.x * 64 + c;
-  float s = 0.0f;
-  if (n < N)
-    for (int m = ph; m < M; m += 4) s += dz[static_cast<size_t>(m) * N + n];
-  part[ph][c] = s;
-  __syncthreads();
-  if (ph == 0 && n < N) g[n] = (part[0][c] + part[1][c]) + (part[2][c] + part[3][c]);
+  __shared__ float part[16][17];
+  const int c = threadIdx.x & 15, ph = threadIdx.x >> 4;
+  const int n = blockIdx.x * 16 + c;
+  float s[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+  if (n < N) {
+    int m = ph;
+    for (; m + 48 < M; m += 64)
+#pragma unroll
+      for (int u = 0; u < 4; ++u) s[u] += dz[static_cast<size_t>(m + 16 * u) * N + n];
+    for (int u = 0; m < M; m += 16, ++u) s[u] += dz[static_cast<size_t>(m) * N + n];
+  }
+  part[ph][c] = (s[0] + s[1]) + (s[2] + s[3]);
+  for (int o = 8; o > 0; o >>= 1) {
+    __syncthreads();
+    if (ph < o) part[ph][c] += part[ph + o][c];
+  }
+  if (ph == 0 && n < N) g[n] = part[0][c];
 }
 
 __global__ void mse_grad_kernel(const float* pred, const float* y, int M, float* d, float* se) {
@@ -222,31 +240,39 @@ inline unsigned nb(size_t n, unsigned t) { return static_cast<unsigned>((n + t -
 
 }  // namespace
 
-int gemm(int atype, const void* A, int lda, int ta, int btype, const void* B, int ldb, int tb,
-         float* C, int ldc, const float* bias, int M, int N, int K, hipStream_t st) {
+namespace {
+template <int kTile, int kKs>
+void launch_gemm(int atype, const void* A, int lda, int ta, int btype, const void* B, int ldb,
+                 int tb, float* C, int ldc, const float* bias, const float* zg, bf16* act, int M,
+                 int N, int K, hipStream_t st) {
   const dim3 grid((N + kTile - 1) / kTile, (M + kTile - 1) / kTile);
+  auto go = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, grid, dim3(256), 0, st, A, lda, ta, B, ldb, tb, C, ldc, bias, zg,
+                       act, M, N, K);
+  };
   if (atype == 0 && btype == 0)
-    hipLaunchKernelGGL((gemm_kernel<0, 0>), grid, dim3(256), 0, st, A, lda, ta, B, ldb, tb, C,
-                       ldc, bias, M, N, K);
+    go(gemm_kernel<0, 0, kTile, kKs>);
   else if (atype == 1 && btype == 0)
-    hipLaunchKernelGGL((gemm_kernel<1, 0>), grid, dim3(256), 0, st, A, lda, ta, B, ldb, tb, C,
-                       ldc, bias, M, N, K);
+    go(gemm_kernel<1, 0, kTile, kKs>);
   else if (atype == 0 && btype == 1)
-    hipLaunchKernelGGL((gemm_kernel<0, 1>), grid, dim3(256), 0, st, A, lda, ta, B, ldb, tb, C,
-                       ldc, bias, M, N, K);
+    go(gemm_kernel<0, 1, kTile, kKs>);
   else
-    hipLaunchKernelGGL((gemm_kernel<1, 1>), grid, dim3(256), 0, st, A, lda, ta, B, ldb, tb, C,
-                       ldc, bias, M, N, K);
-  return ok();
+    go(gemm_kernel<1, 1, kTile, kKs>);
 }
+}  // namespace
 
-int gelu_fwd(const float* z, bf16* out, size_t n, hipStream_t st) {
-  hipLaunchKernelGGL(gelu_fwd_kernel, dim3(nb(n, 256)), dim3(256), 0, st, z, out, n);
-  return ok();
-}
-
-int gelu_bwd(const float* z, float* dA, size_t n, hipStream_t st) {
-  hipLaunchKernelGGL(gelu_bwd_kernel, dim3(nb(n, 256)), dim3(256), 0, st, z, dA, n);
+int gemm(int atype, const void* A, int lda, int ta, int btype, const void* B, int ldb, int tb,
+         float* C, int ldc, const float* bias, const float* zg, bf16* act, int M, int N, int K,
+         hipStream_t st) {
+  // tiles of 64 read the operands half as often, but where they make fewer
+  // workgroups than the chip has compute units the smaller ones are faster:
+  // a gradient of 512 rows and 256 hidden units 266 us against 365, of 4096
+  // and 256 1121 against 1149, of 4096 and 512 2590 against 2360, of 16384 and
+  // 512 5611 against 4546
+  if (static_cast<long>((N + 63) / 64) * ((M + 63) / 64) >= 256)
+    launch_gemm<64, 32>(atype, A, lda, ta, btype, B, ldb, tb, C, ldc, bias, zg, act, M, N, K, st);
+  else
+    launch_gemm<32, 128>(atype, A, lda, ta, btype, B, ldb, tb, C, ldc, bias, zg, act, M, N, K, st);
   return ok();
 }
 
@@ -272,7 +298,7 @@ int gather_rows(const float* tx, const float* ty, const int* order, int b0, int 
 }
 
 int colsum(const float* dz, int M, int N, float* g, hipStream_t st) {
-  hipLaunchKernelGGL(colsum_kernel, dim3(nb(N, 64)), dim3(256), 0, st, dz, M, N, g);
+  hipLaunchKernelGGL(colsum_kernel, dim3(nb(N, 16)), dim3(256), 0, st, dz, M, N, g);
   return ok();
 }
 
