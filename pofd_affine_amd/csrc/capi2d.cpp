@@ -720,13 +720,13 @@ int prepare_set2(pofd_ctx* c, Ctx2& C2, Set2& s) {
   if ((rc = upload(c, s, sg_e, &d_sg_e))) return rc;
   d_e1 = d.edge1;
   s.gmain = pofd2::RGrid{static_cast<int>(n), static_cast<int>(n), d.rflux1, d_inv_m, d_lg_m,
-                         d_sg_m, nullptr, 0, static_cast<int>(n), dflux1 * dflux2};
+                         d_sg_m, dflux1 * dflux2};
   s.g00 = pofd2::RGrid{static_cast<int>(ne), static_cast<int>(ne), d_e1, d_inv_e, d_lg_e,
-                       d_sg_e, nullptr, 0, static_cast<int>(ne), 1.0};
+                       d_sg_e, 1.0};
   s.gx = pofd2::RGrid{static_cast<int>(ne), static_cast<int>(n), d_e1, d_inv_m, d_lg_m,
-                      d_sg_m, nullptr, 0, static_cast<int>(n), 1.0};
+                      d_sg_m, 1.0};
   s.gy = pofd2::RGrid{static_cast<int>(n), static_cast<int>(ne), d.rflux1, d_inv_e, d_lg_e,
-                      d_sg_e, nullptr, 0, static_cast<int>(ne), 1.0};
+                      d_sg_e, 1.0};
   // datasets
   d.nfields = static_cast<int>(s.fields.size());
   for (size_t f = 0; f < s.fields.size(); ++f) {
@@ -774,7 +774,7 @@ int ensure_work2(pofd_ctx* c, Ctx2& C2, Set2& s, uint32_t nwalk) {
   const size_t n = C2.n, ne = C2.nedge, nf = s.fields.size(), W = nwalk;
   const size_t nc = n / 2 + 1;
   auto r8 = [](size_t x) { return (x + 7) & ~size_t(7); };
-  w.ex_stride = r8(ne * n);        // nedge x n (ex) or n x nedge (ey)
+  w.ex_stride = r8(pofd2::kEdgeParts * n);
   w.edge_stride = r8(std::max(n, ne));
   w.YT_stride = r8(nc * n);
   w.PR_stride = r8(nc * n);
@@ -783,9 +783,7 @@ int ensure_work2(pofd_ctx* c, Ctx2& C2, Set2& s, uint32_t nwalk) {
   size_t tot = 0;
   const size_t o_model = tot; tot += r8(pofd2::kModelStride) * W;
   const size_t o_stats = tot; tot += r8(pofd2::kStats) * W;
-  const size_t o_e00 = tot; tot += r8(ne * ne) * W;
   const size_t o_ex = tot; tot += w.ex_stride * W;
-  const size_t o_ey = tot; tot += w.ex_stride * W;
   const size_t o_rx = tot; tot += w.edge_stride * W;
   const size_t o_ry = tot; tot += w.edge_stride * W;
   const size_t o_r00 = tot; tot += w.edge_stride * W;
@@ -813,9 +811,7 @@ int ensure_work2(pofd_ctx* c, Ctx2& C2, Set2& s, uint32_t nwalk) {
   double* b = static_cast<double*>(s.wbuf->p);
   w.model = b + o_model;
   w.stats = b + o_stats;
-  w.e00 = b + o_e00;
   w.ex = b + o_ex;
-  w.ey = b + o_ey;
   w.rx = b + o_rx;
   w.ry = b + o_ry;
   w.r00rows = b + o_r00;
@@ -830,12 +826,6 @@ int ensure_work2(pofd_ctx* c, Ctx2& C2, Set2& s, uint32_t nwalk) {
   w.dbg = b + o_dbg;
   w.bonus = b + o_bo;
   w.rpieces = b + o_rp;
-  s.g00.out = w.e00;
-  s.g00.wstride = r8(ne * ne);
-  s.gx.out = w.ex;
-  s.gx.wstride = w.ex_stride;
-  s.gy.out = w.ey;
-  s.gy.wstride = w.ex_stride;
   s.wcap = nwalk;
   // zero once so that debug reads of never-written slots are defined
   hipError_t e = hipMemset(s.wbuf->p, 0, tot * sizeof(double));

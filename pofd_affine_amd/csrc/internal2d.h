@@ -20,12 +20,13 @@ namespace pofd2 {
 constexpr int kMaxK = 32;          // knots, sigma knots, offset knots (each)
 constexpr int kMaxFields2 = 8;     // datasets per beam set
 constexpr int kLikeBlocks = 64;    // workgroups per (walker, dataset) in like2d
+constexpr int kEdgeParts = 32;     // parts of the edge rows' sum in the edge integrals
 constexpr int kRowBlocks2 = 64;    // workgroups per walker in the inverse row transforms
 // per-walker model block: header, knot spline, sigma and offset interpolants
 // (4 coefficients per interval each), raw sigma and offset values
 constexpr int kModelStride = 8 + 14 * kMaxK;
 constexpr int kStats = 16;
-// dynamic LDS ceiling of the R-grid kernel (3 doubles per beam element)
+// limit of a row's beam pieces (3 doubles per beam element)
 constexpr size_t kRgridMaxLds = 144 * 1024;
 constexpr int kDbg2 = 32;
 
@@ -60,16 +61,13 @@ struct Field2Dev {
   uint64_t npix;
 };
 
-// one flux grid for rgrid2d (theta-independent tables)
+// one flux grid that R is made on (theta-independent tables)
 struct RGrid {
   int n1, n2;
   const double* f1;         // n1 band-1 fluxes
   const double* f2inv;      // n2: 1/|f2| or 0 (f2 == 0)
   const double* f2log;      // n2: log|f2|
   const int* f2sgn;         // n2: 0 for f2 > 0, 1 for f2 < 0
-  double* out;              // + walker * wstride + i * ostride + j
-  size_t wstride;
-  int ostride;
   double scale;
 };
 
@@ -106,9 +104,7 @@ struct Work2 {
   int nwalk;
   double* model;                  // W * kModelStride
   double* stats;                  // W * kStats
-  double* e00;                    // W * nedge * nedge
-  double* ex;                     // W * nedge * n
-  double* ey;                     // W * n * nedge
+  double* ex;                     // W * kEdgeParts * n: parts of Rx
   double* rx;                     // W * edge_stride (n)
   double* ry;
   double* r00rows;

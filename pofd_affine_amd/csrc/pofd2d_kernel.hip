@@ -37,6 +37,7 @@
 
 #include <algorithm>
 
+#include "exp2.h"
 #include "internal2d.h"
 
 namespace pofd2 {
@@ -374,7 +375,7 @@ __global__ __launch_bounds__(64) void bonus2d_kernel(const Set2Dev s, const Work
 // The pieces of R that depend on the row flux f1 but not on f2, per row
 // of the grid and beam element (RWork, :1868-1950): weight (0 where the
 // element adds nothing), log-flux centre and Gaussian width factor, into
-// wk.rpieces for rgrid2d_kernel.  One thread per (row, element), so that
+// wk.rpieces for the kernels that make R.  One thread per (row, element), so that
 // their logs, exp2s and colour splines run in parallel rather than on a
 // few threads of each row's workgroup.
 __global__ __launch_bounds__(kT) void rpieces2d_kernel(const Set2Dev s, const Work2 wk,
@@ -438,118 +439,154 @@ __global__ __launch_bounds__(kT) void rpieces2d_kernel(const Set2Dev s, const Wo
   }
   c[0] = c0;
   c[1] = c1;
-  c[2] = c2;
+  c[2] = 32.0 * c2;  // the exponent in the units of exp2_32
 }
 
-// R on one flux grid, a row per workgroup step: the row's pieces (from
-// rpieces2d_kernel) into LDS, then every f2 of the row sums its beam
-// elements' Gaussian colour terms in element order.
-__global__ __launch_bounds__(kT) void rgrid2d_kernel(const Set2Dev s, const Work2 wk,
-                                                     const RGrid g) {
-  extern __shared__ double rw[];  // 3 * (np + nn) per row
-  const int w = blockIdx.y;
-  const double* m = model_ptr(wk, w);
-  if (m[0] != POFD_OK) return;  // uniform
-  const double* pieces = wk.rpieces + static_cast<size_t>(w) * wk.rpieces_stride;
-  for (int i = blockIdx.x; i < g.n1; i += gridDim.x) {
-    double f1val = g.f1[i];
-    if ((f1val == 0) || (f1val < 0 && !s.hasneg1)) {
-      for (int j = threadIdx.x; j < g.n2; j += kT)
-        g.out[static_cast<size_t>(w) * g.wstride + static_cast<size_t>(i) * g.ostride + j] = 0.0;
-      continue;
+// 2^(t/32) by Tang's table-driven method (ACM TOMS 15:144, 1989): t = 32 n +
+// j + u, 2^n tab[j] 2^(u/32).  Zero from t = -34560 (2^-1080) down; NaN stays.
+// About one ulp, in 12 instructions of the 20 of exp2.
+__device__ __forceinline__ double exp2_32(double t, const double* tab) {
+  t = (t < -35000.0) ? -35000.0 : t;
+  const double n = rint(t);
+  const int ni = __double2int_rn(t);
+  return ldexp(tab[ni & 31] * pofd::exp2_near(t - n), ni >> 5);
+}
+__device__ __forceinline__ void load_exp2(double* tab) {
+  if (threadIdx.x < 32) tab[threadIdx.x] = exp2(static_cast<double>(threadIdx.x) * 0.03125);
+}
+
+// R at f1val and the kEdgePts points f2[j0 + q step], j < n2, of a grid from
+// the row's pieces, the beam elements' Gaussian colour terms summed in element
+// order; the pieces are read once for all points.
+constexpr int kEdgePts = 4;
+__device__ __forceinline__ void r_values(const Set2Dev& s, const RGrid& g, const double f1val,
+                                         const double* __restrict__ prow, const int j0,
+                                         const int step, const double* tab, double* r) {
+#pragma unroll
+  for (int q = 0; q < kEdgePts; ++q) r[q] = 0.0;
+  if ((f1val == 0) || (f1val < 0 && !s.hasneg1)) return;
+  const int sgn1 = (f1val > 0) ? 0 : 2;
+  double lf[kEdgePts];
+#pragma unroll 1
+  for (int sg = 0; sg < 2; ++sg) {
+    const int cn = s.comp[sgn1 + sg].n;
+    if (cn == 0) continue;
+    // a point of the other sign, or of no flux: an exponent of -infinity
+#pragma unroll
+    for (int q = 0; q < kEdgePts; ++q) {
+      const int j = j0 + q * step;
+      lf[q] = (j < g.n2 && g.f2inv[j] != 0 && g.f2sgn[j] == sg) ? g.f2log[j] : 1e160;
     }
-    const int sgn1 = (f1val > 0) ? 0 : 2;
-    const int np = s.comp[sgn1].n, nn = s.comp[sgn1 + 1].n;
-    const double* prow = pieces + static_cast<size_t>(i) * wk.rpieces_w;
-    for (int e = threadIdx.x; e < 3 * (np + nn); e += kT) rw[e] = prow[e];
-    __syncthreads();
-    double* orow = g.out + static_cast<size_t>(w) * g.wstride + static_cast<size_t>(i) * g.ostride;
-    for (int j = threadIdx.x; j < g.n2; j += kT) {
-      const double if2 = g.f2inv[j];
-      double r = 0.0;
-      if (if2 != 0) {
-        const int fs = g.f2sgn[j];
-        const int sgn = sgn1 + fs;
-        if (s.comp[sgn].n > 0) {
+    const double* base = prow + (sg ? 3 * s.comp[sgn1].n : 0);
+    for (int k = 0; k < cn; ++k) {
 #pragma clang fp contract(off)
-          const int cn = s.comp[sgn].n;
-          const double* base = rw + 3 * (fs ? np : 0);
-          const double lf2 = g.f2log[j];
-          double workval = 0.0;
-          for (int k = 0; k < cn; ++k) {
-            const double c0 = base[3 * k];
-            if (c0 != 0) {
-              const double tfac = lf2 - base[3 * k + 1];
-              workval += c0 * exp2(tfac * tfac * base[3 * k + 2]);
-            }
-          }
-          r = (workval * if2) * g.scale;
-        }
+      const double c0 = base[3 * k], c1 = base[3 * k + 1], c2 = base[3 * k + 2];
+      if (c0 == 0) continue;
+#pragma unroll
+      for (int q = 0; q < kEdgePts; ++q) {
+        const double tfac = lf[q] - c1;
+        r[q] += c0 * exp2_32(tfac * tfac * c2, tab);
       }
-      orow[j] = r;
     }
-    __syncthreads();
+  }
+#pragma unroll
+  for (int q = 0; q < kEdgePts; ++q) {
+    const int j = j0 + q * step;
+    r[q] = (j < g.n2) ? (r[q] * g.f2inv[j]) * g.scale : 0.0;
   }
 }
 
 // ===========================================================================
 // edge integrals (initR with setEdge, src/PDFactoryDouble.cc:386-544)
 // ===========================================================================
-// Ry[i] = trapezoid over the linear edge in band 2 of R(RFlux1[i], edge2)
-// and the y integral of the nedge x nedge grid (row sums), thread per row
-__global__ void edge2d_rows_kernel(const Set2Dev s, const Work2 wk, const int nrows,
-                                   const double* __restrict__ grid, const size_t gstride,
-                                   double* __restrict__ out, const size_t ostride,
-                                   const double norm) {
+// Per row of a grid the trapezoid over its columns (the linear edge in band
+// 2): a wavefront per row, R summed as it is made.  With edge2d_cols_kernel
+// XX us for 32 walkers at 2048 and 256 edge points, bound by the exponentials;
+// three grids to memory and one thread per sum took 306 + 237.
+__global__ __launch_bounds__(kT) void edge2d_rows_kernel(const Set2Dev s, const Work2 wk,
+                                                         const RGrid g,
+                                                         double* __restrict__ out) {
+  __shared__ double tab[32];
   const int w = blockIdx.y;
-  if (model_ptr(wk, w)[0] != POFD_OK) return;
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= nrows) return;
-  const int ne = s.nedge;
-  const double* r = grid + static_cast<size_t>(w) * gstride + static_cast<size_t>(i) * ne;
-  double sc;
-  {
-#pragma clang fp contract(off)
-    sc = 0.5 * r[0];
-    for (int j = 1; j < ne - 1; ++j) sc += r[j];
-    sc += 0.5 * r[ne - 1];
-    if (norm != 0.0) sc *= norm;
+  if (model_ptr(wk, w)[0] != POFD_OK) return;  // uniform
+  load_exp2(tab);
+  __syncthreads();
+  const int lane = threadIdx.x & 63;
+  const int i = __builtin_amdgcn_readfirstlane(
+      static_cast<int>(blockIdx.x * (kT / 64) + (threadIdx.x >> 6)));
+  if (i >= g.n1) return;
+  const double f1val = g.f1[i];
+  const double* prow = wk.rpieces + static_cast<size_t>(w) * wk.rpieces_stride +
+                       static_cast<size_t>(i) * wk.rpieces_w;
+  double sc = 0.0;
+  for (int j0 = lane; j0 - lane < g.n2; j0 += 64 * kEdgePts) {
+    double r[kEdgePts];
+    r_values(s, g, f1val, prow, j0, 64, tab, r);
+#pragma unroll
+    for (int q = 0; q < kEdgePts; ++q) {
+      const int j = j0 + 64 * q;
+      sc += ((j == 0 || j == g.n2 - 1) ? 0.5 : 1.0) * r[q];
+    }
   }
-  out[static_cast<size_t>(w) * ostride + i] = sc;
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) sc += __shfl_xor(sc, o);
+  if (lane == 0) out[static_cast<size_t>(w) * wk.edge_stride + i] = sc;
 }
 
-// Rx[j] = log-x trapezoid over the nedge rows of R(edge1, RFlux2[j])
-__global__ void edge2d_cols_kernel(const Set2Dev s, const Work2 wk) {
-  const int w = blockIdx.y;
-  if (model_ptr(wk, w)[0] != POFD_OK) return;
-  const int j = blockIdx.x * blockDim.x + threadIdx.x;
-  const int n = s.n, ne = s.nedge;
-  if (j >= n) return;
-  const double* ex = wk.ex + static_cast<size_t>(w) * wk.ex_stride;
-  double acc;
-  {
-#pragma clang fp contract(off)
-    acc = 0.5 * s.edge1[0] * ex[j];
-    for (int i = 1; i < ne - 1; ++i) acc += s.edge1[i] * ex[static_cast<size_t>(i) * n + j];
-    acc += 0.5 * s.edge1[ne - 1] * ex[static_cast<size_t>(ne - 1) * n + j];
-    acc *= s.iRxnorm;
+// The log-x trapezoid over the nedge rows of R(edge1, RFlux2[j]), kEdgePts
+// columns a thread: the rows of part blockIdx.y, for edge2d_sum_kernel
+__global__ __launch_bounds__(kT) void edge2d_cols_kernel(const Set2Dev s, const Work2 wk,
+                                                         const RGrid g) {
+  __shared__ double tab[32];
+  const int w = blockIdx.z;
+  if (model_ptr(wk, w)[0] != POFD_OK) return;  // uniform
+  load_exp2(tab);
+  __syncthreads();
+  const int j0 = blockIdx.x * kT * kEdgePts + threadIdx.x;
+  const int ne = g.n1, part = blockIdx.y, parts = gridDim.y;
+  const int i0 = part * ne / parts, i1 = (part + 1) * ne / parts;
+  double acc[kEdgePts] = {0.0, 0.0, 0.0, 0.0};
+  for (int i = i0; i < i1; ++i) {
+    const double* prow = wk.rpieces + static_cast<size_t>(w) * wk.rpieces_stride +
+                         static_cast<size_t>(i) * wk.rpieces_w;
+    const double wi = ((i == 0 || i == ne - 1) ? 0.5 : 1.0) * s.edge1[i];
+    double r[kEdgePts];
+    r_values(s, g, g.f1[i], prow, j0, kT, tab, r);
+#pragma unroll
+    for (int q = 0; q < kEdgePts; ++q) acc[q] += wi * r[q];
   }
-  wk.rx[static_cast<size_t>(w) * wk.edge_stride + j] = acc;
+#pragma unroll
+  for (int q = 0; q < kEdgePts; ++q) {
+    const int j = j0 + q * kT;
+    if (j < g.n2)
+      wk.ex[static_cast<size_t>(w) * wk.ex_stride + static_cast<size_t>(part) * g.n2 + j] = acc[q];
+  }
 }
 
-// R[0,0] (times dflux1 dflux2) from the row sums of the nedge x nedge grid,
-// to rx[0]; rowfft2d_kernel puts rx and ry in place of row 0 and column 0
-__global__ void edge2d_r00_kernel(const Set2Dev s, const Work2 wk) {
-  const int w = blockIdx.x * blockDim.x + threadIdx.x;
-  if (w >= wk.nwalk || model_ptr(wk, w)[0] != POFD_OK) return;
-  const int ne = s.nedge;
-  const double* r00rows = wk.r00rows + static_cast<size_t>(w) * wk.edge_stride;
-  {
-#pragma clang fp contract(off)
-    double sc = 0.5 * s.edge1[0] * r00rows[0];
-    for (int i = 1; i < ne - 1; ++i) sc += s.edge1[i] * r00rows[i];
-    sc += 0.5 * s.edge1[ne - 1] * r00rows[ne - 1];
-    wk.rx[static_cast<size_t>(w) * wk.edge_stride] = (sc * s.iR00norm) * (s.dflux1 * s.dflux2);
+// Rx[j] from its parts, and R[0,0] (times dflux1 dflux2) from the row sums of
+// the nedge x nedge grid to rx[0]; rowfft2d_kernel puts rx and ry in place of
+// row 0 and column 0
+__global__ __launch_bounds__(kT) void edge2d_sum_kernel(const Set2Dev s, const Work2 wk,
+                                                        const int parts) {
+  __shared__ double red[kT / 64];
+  const int w = blockIdx.y;
+  if (model_ptr(wk, w)[0] != POFD_OK) return;  // uniform
+  double* rx = wk.rx + static_cast<size_t>(w) * wk.edge_stride;
+  const int j = blockIdx.x * kT + threadIdx.x;
+  if (j > 0 && j < s.n) {
+    const double* ex = wk.ex + static_cast<size_t>(w) * wk.ex_stride + j;
+    double acc = 0.0;
+    for (int p = 0; p < parts; ++p) acc += ex[static_cast<size_t>(p) * s.n];
+    rx[j] = acc * s.iRxnorm;
+  }
+  if (blockIdx.x == 0) {
+    const double* r00rows = wk.r00rows + static_cast<size_t>(w) * wk.edge_stride;
+    const int ne = s.nedge;
+    double sc = 0.0;
+    for (int i = threadIdx.x; i < ne; i += kT)
+      sc += ((i == 0 || i == ne - 1) ? 0.5 : 1.0) * s.edge1[i] * r00rows[i];
+    sc = block_sum(sc, red);
+    if (threadIdx.x == 0) rx[0] = (sc * s.iR00norm) * (s.dflux1 * s.dflux2);
   }
 }
 
@@ -651,7 +688,7 @@ __device__ __forceinline__ void load_turns(double2* tw, const double2* __restric
 __global__ __launch_bounds__(kTR) void rowfft2d_kernel(const Set2Dev s, const Work2 wk,
                                                        const RGrid g, const int rg) {
   extern __shared__ double2 lds[];
-  __shared__ double red[kTR / 64];
+  __shared__ double red[kTR / 64], ex2[32];
   const int w = blockIdx.y;
   const double* m = model_ptr(wk, w);
   if (m[0] != POFD_OK) return;
@@ -663,6 +700,8 @@ __global__ __launch_bounds__(kTR) void rowfft2d_kernel(const Set2Dev s, const Wo
   double2* rows = lds + h / 4;
   const int rs = n + 2;  // the rows' elements k on distinct banks
   load_turns(tw, s.tw_half, h);
+  load_exp2(ex2);
+  __syncthreads();
   const double* pieces = wk.rpieces + static_cast<size_t>(w) * wk.rpieces_stride;
   const double* rx = wk.rx + static_cast<size_t>(w) * wk.edge_stride;
   const double* ry = wk.ry + static_cast<size_t>(w) * wk.edge_stride;
@@ -706,9 +745,9 @@ __global__ __launch_bounds__(kTR) void rowfft2d_kernel(const Set2Dev s, const Wo
             const double ta = lf[2 * q] - c1, tb = lf[2 * q + 1] - c1;
             const double ea = ta * ta * c2, eb = tb * tb * c2;
             // below the smallest number for the whole wavefront: adds nothing
-            if (__any(!(ea <= -1080.0 && eb <= -1080.0))) {
-              x[2 * q] += c0 * exp2(ea);
-              x[2 * q + 1] += c0 * exp2(eb);
+            if (__any(!(ea <= -34560.0 && eb <= -34560.0))) {
+              x[2 * q] += c0 * exp2_32(ea, ex2);
+              x[2 * q + 1] += c0 * exp2_32(eb, ex2);
             }
           }
         }
@@ -1332,43 +1371,34 @@ int launch_loglike2d(const Set2Dev& s, const Work2& wk, const RGrid& gmain,
   auto mark = [&](int i) {
     if (ev) (void)hipEventRecord(ev[i], st);
   };
-  // rgrid2d: dynamic LDS for the per-row beam pieces of two sign components
-  int maxc = 0;
-  for (int k = 0; k < 2; ++k) maxc = std::max(maxc, s.comp[2 * k].n + s.comp[2 * k + 1].n);
-  const size_t rg_lds = static_cast<size_t>(3) * std::max(maxc, 1) * sizeof(double);
-  if (rg_lds > kRgridMaxLds) return POFD_E_ARG;
-  if (rg_lds + 8192 > 65536)  // + the static knot tables (4.3 KB)
-    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(rgrid2d_kernel),
-                              hipFuncAttributeMaxDynamicSharedMemorySize,
-                              static_cast<int>(rg_lds));
-  const int rblocks = 64;  // row blocks per walker (grid-stride over rows)
-  // one R grid: its per-row beam pieces, then the grid
+  // a grid's per-row beam pieces
   auto pieces = [&](const RGrid& g) {
     const int pb = static_cast<int>((static_cast<size_t>(g.n1) * (wk.rpieces_w / 3) + kT - 1) / kT);
     hipLaunchKernelGGL(rpieces2d_kernel, dim3(pb, W), dim3(kT), 0, st, s, wk, g);
   };
-  auto rgrid = [&](const RGrid& g, const int blocks) {
-    pieces(g);
-    hipLaunchKernelGGL(rgrid2d_kernel, dim3(blocks, W), dim3(kT), rg_lds, st, s, wk, g);
+  auto edge_rows = [&](const RGrid& g, double* out) {
+    hipLaunchKernelGGL(edge2d_rows_kernel, dim3((g.n1 + kT / 64 - 1) / (kT / 64), W), dim3(kT), 0,
+                       st, s, wk, g, out);
   };
   mark(POFD_STAGE_PREP);
   hipLaunchKernelGGL(prep2d_kernel, dim3(W), dim3(64), 0, st, s, wk, d_theta, stride, d_st,
                      accumulate);
   if (s.bonus) hipLaunchKernelGGL(bonus2d_kernel, dim3(W), dim3(64), 0, st, s, wk);
   mark(POFD_STAGE_FORWARD);
+  // (the edge grids' rows are edge1, then rflux1 as in the main grid: two
+  // sets of pieces serve the four)
   if (s.edge_integ) {
-    rgrid(g00, std::min(rblocks, ne));
-    rgrid(gx, std::min(rblocks, ne));
-    rgrid(gy, rblocks);
-    hipLaunchKernelGGL(edge2d_rows_kernel, dim3((ne + 255) / 256, W), dim3(256), 0, st, s, wk,
-                       ne, wk.e00, g00.wstride, wk.r00rows, wk.edge_stride, 0.0);
-    hipLaunchKernelGGL(edge2d_rows_kernel, dim3((n + 255) / 256, W), dim3(256), 0, st, s, wk,
-                       n, wk.ey, gy.wstride, wk.ry, wk.edge_stride, 0.0);
-    hipLaunchKernelGGL(edge2d_cols_kernel, dim3((n + 255) / 256, W), dim3(256), 0, st, s, wk);
+    const int eparts = std::min(kEdgeParts, ne);
+    pieces(g00);
+    edge_rows(g00, wk.r00rows);
+    hipLaunchKernelGGL(edge2d_cols_kernel,
+                       dim3((n + kT * kEdgePts - 1) / (kT * kEdgePts), eparts, W), dim3(kT), 0, st, s,
+                       wk, gx);
+    hipLaunchKernelGGL(edge2d_sum_kernel, dim3((n + kT - 1) / kT, W), dim3(kT), 0, st, s, wk,
+                       eparts);
   }
   pieces(gmain);
-  if (s.edge_integ)
-    hipLaunchKernelGGL(edge2d_r00_kernel, dim3((W + 63) / 64), dim3(64), 0, st, s, wk);
+  if (s.edge_integ) edge_rows(gy, wk.ry);
   const int nparts = 64;
   const int rg = rows_together(n), cg = cols_together(n);
   // a quarter turn of twiddles and both buffers of each row or column
