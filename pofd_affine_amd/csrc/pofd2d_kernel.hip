@@ -500,9 +500,10 @@ __device__ __forceinline__ void r_values(const Set2Dev& s, const RGrid& g, const
 // edge integrals (initR with setEdge, src/PDFactoryDouble.cc:386-544)
 // ===========================================================================
 // Per row of a grid the trapezoid over its columns (the linear edge in band
-// 2): a wavefront per row, R summed as it is made.  With edge2d_cols_kernel
-// XX us for 32 walkers at 2048 and 256 edge points, bound by the exponentials;
-// three grids to memory and one thread per sum took 306 + 237.
+// 2): a wavefront per row, R summed as it is made.  The edge integrals take
+// 217 us for 32 walkers at 2048 and 256 edge points, bound by the
+// exponentials; three grids to memory and one thread per sum took 306 + 237
+// (and 570 one point at a time, waiting for each element's pieces).
 __global__ __launch_bounds__(kT) void edge2d_rows_kernel(const Set2Dev s, const Work2 wk,
                                                          const RGrid g,
                                                          double* __restrict__ out) {
@@ -681,7 +682,7 @@ __device__ __forceinline__ void load_turns(double2* tw, const double2* __restric
 // YT[k2][i].  R goes to memory nowhere.  rg rows together, T = kTR / rg
 // threads each (whole wavefronts, so that a row's pieces are uniform reads,
 // made once for a thread's eight points).  Bound by the exponentials of R:
-// 1648 us for 32 walkers at 2048, where R to memory, its moments, the row
+// 1590 us for 32 walkers at 2048 (1648 with the library's exp2), where R to memory, its moments, the row
 // transforms from it and their transposition took 1274 + 265 + 588 + 195
 // (2489 with the pieces read again for each point).
 // ===========================================================================
