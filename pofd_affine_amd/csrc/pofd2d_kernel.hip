@@ -7,23 +7,21 @@
 //   prep2d        model set-up per walker: knot spline, colour sigma and
 //                 offset interpolants (numberCountsDoubleLogNormal::setParams,
 //                 src/numberCountsDoubleLogNormal.cc:1010-1052)
-//   rgrid2d       R on a grid of (f1, f2) fluxes, one row per workgroup
-//                 (getR array version, :1788-2007); used for the main grid
-//                 and the three edge grids of initR (src/PDFactoryDouble.cc:
-//                 376-551)
-//   edge2d_*      edge integrals R[0,0], R[0,y], R[x,0] in the reference's
-//                 summation order, patched into the main grid
-//   rstats2d      mean and variance along each axis (getRStats, :593-722)
-//   rowfft2d      r2c transform of every row, columns k2 <= K2 kept
-//   transpose2d   [rows][cols] <-> [cols][rows] through LDS tiles
-//   colfft2d      complex transform down every kept column; spectrum
-//                 exp(R^ - R^0) with the mean shifts (initPD, :1228-1340)
-//   noisecol2d    per dataset: noise factor (getPD, :1396-1431) and the
-//                 inverse transform down every kept column
+//   rpieces2d     the parts of R that depend on the row alone (getR array
+//                 version, :1788-2007)
+//   edge2d_*      edge integrals R[0,0], R[0,y], R[x,0] of initR
+//                 (src/PDFactoryDouble.cc:376-551)
+//   rowfft2d      R row by row, mean and variance along each axis (getRStats,
+//                 :593-722), r2c transform, columns k2 <= K2 kept
+//   rstats2d      the moments' parts combined, the shifts, R^(0)
+//   colpass2d     complex transform down every kept column; spectrum
+//                 exp(R^ - R^0) with the mean shifts (initPD, :1228-1340);
+//                 per dataset the noise factor (getPD, :1396-1431) and the
+//                 inverse transform
 //   rowifft2d     c2r transform of every row, clamp, row marginal
 //   colsum2d      column marginal (unwrapAndNormalizePD, :1001-1011)
 //   split2d       findSplitPoint on both marginals (:784-975)
-//   norm2d_*      rotation by the split points, integral and means
+//   norm2d        rotation by the split points, integral and means
 //                 (PDDouble::getIntegral / getMeans, src/PDDouble.cc:142-452)
 //   like2d        binned or unbinned bilinear log likelihood
 //                 (src/PDDouble.cc:976-1222)
@@ -369,15 +367,13 @@ __global__ __launch_bounds__(64) void bonus2d_kernel(const Set2Dev s, const Work
 }
 
 // ===========================================================================
-// rgrid2d: R on (f1[i], f2[j]) for every walker; one workgroup per
-// (row block, walker).  out[i*ostride + j] = R * scale.
+// R on (f1[i], f2[j])
 // ===========================================================================
 // The pieces of R that depend on the row flux f1 but not on f2, per row
 // of the grid and beam element (RWork, :1868-1950): weight (0 where the
 // element adds nothing), log-flux centre and Gaussian width factor, into
-// wk.rpieces for the kernels that make R.  One thread per (row, element), so that
-// their logs, exp2s and colour splines run in parallel rather than on a
-// few threads of each row's workgroup.
+// wk.rpieces for the kernels that make R.  One thread per (row, element), so
+// that their logs, exp2s and colour splines run in parallel.
 __global__ __launch_bounds__(kT) void rpieces2d_kernel(const Set2Dev s, const Work2 wk,
                                                        const RGrid g) {
   __shared__ double lk[kMaxK], lkcf[4 * kMaxK];
