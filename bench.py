@@ -25,10 +25,10 @@ HBM_PEAK_GBS = 8000.0
 # written = 1.0 x WRITE_SIZE KiB); None where not profiled or for another
 # workload.
 TRAFFIC = {
-    "prep": (2.0 * 2098.1 + 20512.0) * 1024,
-    "forward": (2.0 * 19755.7 + 35308.2) * 1024,
-    "inverse": (2.0 * 2774.5 + 279619.0) * 1024,
-    "finalize": (2.0 * 10061.2 + 64.0) * 1024,
+    "prep": (2.0 * 2091.2 + 20516.7) * 1024,
+    "forward": (2.0 * 10999.6 + 31577.8) * 1024,
+    "inverse": (2.0 * 4249.8 + 1080.0) * 1024,
+    "finalize": (2.0 * 4379.1 + 80.0) * 1024,
 }
 FP64_PEAK_TFLOPS = 78.6
 # FP64 FLOP per launch of each kernel at the default workload, from
@@ -37,10 +37,10 @@ FP64_PEAK_TFLOPS = 78.6
 # 16x16x4 f64 MFMA is 2048 FLOP, counted as 4 MOPS).  Divided by the live
 # kernel time for the FP64 roofline.
 FP64_FLOP = {
-    "prep": 2.738e8,
-    "forward": 2.924e9,
-    "inverse": 1.943e9,
-    "finalize": 6.39e7,
+    "prep": 2.75e8,
+    "forward": 2.53e9,
+    "inverse": 1.22e9,
+    "finalize": 1.02e8,
 }
 
 
