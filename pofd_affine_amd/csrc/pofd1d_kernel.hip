@@ -2736,10 +2736,11 @@ __global__ __launch_bounds__(kThreads) void finalize1d_kernel(const BeamsetDev b
   const SplitRange rg = split_range(bs, dbg[23], st[ST_VAR]);
   const int botidx = rg.bot, topidx = rg.top;
 
-  // the values around the minimum and at the ends of the search range
-  __syncthreads();
-  {
-    const int m0 = static_cast<int>(dbg[2]) < 0 ? botidx : static_cast<int>(dbg[2]);
+  // the values around the minimum and at the ends of the search range: made
+  // ahead by as many threads, or where the P(D) is stored read as they come
+  const int m0 = static_cast<int>(dbg[2]) < 0 ? botidx : static_cast<int>(dbg[2]);
+  if constexpr (kWindows) {
+    __syncthreads();
     if (tid < kNear + 4) {
       const int i = m0 - kNear + tid;
       near[tid] = (i >= 0 && i < N) ? P(i) : 0.0;
@@ -2747,8 +2748,10 @@ __global__ __launch_bounds__(kThreads) void finalize1d_kernel(const BeamsetDev b
       const int i = (tid == 64) ? botidx : topidx;
       ends[tid - 64] = (i >= 0 && i < N) ? P(i) : 0.0;
     }
+    __syncthreads();
   }
-  __syncthreads();
+  auto nearv = [&](const int i) { return kWindows ? near[i] : pofd[m0 - kNear + i]; };
+  auto endv = [&](const int i) { return kWindows ? ends[i] : pofd[i == 0 ? botidx : topidx]; };
 
   // ---- findSplitPoint (src/PDFactory.cc:691-921) -----------------------
   if (tid == 0) {
@@ -2766,7 +2769,7 @@ __global__ __launch_bounds__(kThreads) void finalize1d_kernel(const BeamsetDev b
       status = POFD_E_SPLIT;
     if (status == POFD_OK && minidx < 0) {  // empty range: minidx = botidx
       minidx = botidx;
-      minval = ends[0];
+      minval = endv(0);
     }
     if (status == POFD_OK && minval > f2 * peak) status = POFD_E_SPLIT;
     int decided = 0;
@@ -2774,10 +2777,10 @@ __global__ __launch_bounds__(kThreads) void finalize1d_kernel(const BeamsetDev b
       const int pre_jitter_n = kNear;
       if (minidx > pre_jitter_n) {
         bool mono = true;
-        double prev = near[0];
+        double prev = nearv(0);
         jitter = prev;
         for (int i = 1; i < pre_jitter_n; ++i) {
-          const double cv = near[i];
+          const double cv = nearv(i);
           if (cv >= prev) mono = false;
           jitter += cv;
           prev = cv;
@@ -2804,14 +2807,14 @@ __global__ __launch_bounds__(kThreads) void finalize1d_kernel(const BeamsetDev b
         const int ti = (minidx > topidx - nminup) ? topidx - nminup : minidx + nminup;
         if (bi < 0) bi = 0;
         for (int i = bi; i < ti && i < N; ++i) {  // within kNear before, 2 past
-          const double cv = near[i - minidx + kNear];
+          const double cv = nearv(i - minidx + kNear);
           if (cv > minval) minval = cv;
         }
       }
       if (minval > 0) jitter = (f3 * minval) < jitter ? (f3 * minval) : jitter;
       if (botidx >= topidx)
         status = POFD_E_SPLIT;
-      else if (ends[1] < jitter)
+      else if (endv(1) < jitter)
         status = POFD_E_SPLIT;
     }
     isc[0] = status;
