@@ -241,23 +241,25 @@ inline unsigned nb(size_t n, unsigned t) { return static_cast<unsigned>((n + t -
 }  // namespace
 
 namespace {
+// (launched by name: a kernel that is passed on as a value is a handle in
+// host code, which no function-pointer check can take for a function)
 template <int kTile, int kKs>
 void launch_gemm(int atype, const void* A, int lda, int ta, int btype, const void* B, int ldb,
                  int tb, float* C, int ldc, const float* bias, const float* zg, bf16* act, int M,
                  int N, int K, hipStream_t st) {
   const dim3 grid((N + kTile - 1) / kTile, (M + kTile - 1) / kTile);
-  auto go = [&](auto kernel) {
-    hipLaunchKernelGGL(kernel, grid, dim3(256), 0, st, A, lda, ta, B, ldb, tb, C, ldc, bias, zg,
-                       act, M, N, K);
-  };
   if (atype == 0 && btype == 0)
-    go(gemm_kernel<0, 0, kTile, kKs>);
+    hipLaunchKernelGGL((gemm_kernel<0, 0, kTile, kKs>), grid, dim3(256), 0, st, A, lda, ta, B,
+                       ldb, tb, C, ldc, bias, zg, act, M, N, K);
   else if (atype == 1 && btype == 0)
-    go(gemm_kernel<1, 0, kTile, kKs>);
+    hipLaunchKernelGGL((gemm_kernel<1, 0, kTile, kKs>), grid, dim3(256), 0, st, A, lda, ta, B,
+                       ldb, tb, C, ldc, bias, zg, act, M, N, K);
   else if (atype == 0 && btype == 1)
-    go(gemm_kernel<0, 1, kTile, kKs>);
+    hipLaunchKernelGGL((gemm_kernel<0, 1, kTile, kKs>), grid, dim3(256), 0, st, A, lda, ta, B,
+                       ldb, tb, C, ldc, bias, zg, act, M, N, K);
   else
-    go(gemm_kernel<1, 1, kTile, kKs>);
+    hipLaunchKernelGGL((gemm_kernel<1, 1, kTile, kKs>), grid, dim3(256), 0, st, A, lda, ta, B,
+                       ldb, tb, C, ldc, bias, zg, act, M, N, K);
 }
 }  // namespace
 

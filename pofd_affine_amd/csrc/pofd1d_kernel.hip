@@ -3187,22 +3187,35 @@ int launch_loglike1d(const BeamsetDev& bs, const WorkDev& wk_in, int beamset_idx
   if (split)
     hipLaunchKernelGGL(prepspline1d_kernel, dim3(nwalk), dim3(kThreads), 0, s, bs, wk);
   mark(POFD_STAGE_FORWARD);
-  hipLaunchKernelGGL(bs.nwin ? forward1d_kernel<true> : forward1d_kernel<false>, dim3(nxf),
-                     dim3(kThreads), 0, s, bs, wk);
-  if (split)
-    hipLaunchKernelGGL(bs.nwin ? spectrum1d_kernel<true> : spectrum1d_kernel<false>,
-                       dim3(nwalk), dim3(kThreads), 0, s, bs, wk);
+  // (by name: a kernel chosen as a value is a handle in host code, which no
+  // function-pointer check can take for a function)
+  const bool win = bs.nwin > 0;
+  if (win)
+    hipLaunchKernelGGL((forward1d_kernel<true>), dim3(nxf), dim3(kThreads), 0, s, bs, wk);
+  else
+    hipLaunchKernelGGL((forward1d_kernel<false>), dim3(nxf), dim3(kThreads), 0, s, bs, wk);
+  if (split && win)
+    hipLaunchKernelGGL((spectrum1d_kernel<true>), dim3(nwalk), dim3(kThreads), 0, s, bs, wk);
+  else if (split)
+    hipLaunchKernelGGL((spectrum1d_kernel<false>), dim3(nwalk), dim3(kThreads), 0, s, bs, wk);
   mark(POFD_STAGE_INVERSE);
-  hipLaunchKernelGGL(bs.nwin ? inverse1d_kernel<true> : inverse1d_kernel<false>,
-                     dim3(nxf, bs.nfields), dim3(kThreads), 0, s, bs, wk);
+  if (win)
+    hipLaunchKernelGGL((inverse1d_kernel<true>), dim3(nxf, bs.nfields), dim3(kThreads), 0, s, bs,
+                       wk);
+  else
+    hipLaunchKernelGGL((inverse1d_kernel<false>), dim3(nxf, bs.nfields), dim3(kThreads), 0, s, bs,
+                       wk);
   bool any_unbinned = false;
   for (int f = 0; f < bs.nfields; ++f) any_unbinned |= !bs.fields[f].binned;
   // one binned dataset: finalize does the combine too
   const int fuse = (bs.nfields == 1 && !any_unbinned) ? 1 : 0;
   mark(POFD_STAGE_FINALIZE);
-  hipLaunchKernelGGL(bs.nwin ? finalize1d_kernel<true> : finalize1d_kernel<false>,
-                     dim3(nwalk, bs.nfields), dim3(kThreads), 0,
-                     s, bs, wk, fuse, accumulate, d_loglike, d_status);
+  if (win)
+    hipLaunchKernelGGL((finalize1d_kernel<true>), dim3(nwalk, bs.nfields), dim3(kThreads), 0, s,
+                       bs, wk, fuse, accumulate, d_loglike, d_status);
+  else
+    hipLaunchKernelGGL((finalize1d_kernel<false>), dim3(nwalk, bs.nfields), dim3(kThreads), 0, s,
+                       bs, wk, fuse, accumulate, d_loglike, d_status);
   mark(POFD_STAGE_PIXELS);
   if (any_unbinned)
     hipLaunchKernelGGL(pixels1d_kernel, dim3(nwalk, kPixBlocks, bs.nfields),

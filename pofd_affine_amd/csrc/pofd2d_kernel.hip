@@ -1413,8 +1413,12 @@ int launch_loglike2d(const Set2Dev& s, const Work2& wk, const RGrid& gmain,
   hipLaunchKernelGGL(rstats2d_kernel, dim3(W), dim3(kT), 0, st, s, wk, nparts);
   mark(POFD_STAGE_INVERSE);
   for (int f = 0; f < s.nfields; ++f) {
-    hipLaunchKernelGGL(f == 0 ? colpass2d_kernel<true> : colpass2d_kernel<false>, dim3(64, W),
-                       dim3(kTR), lds_col, st, s, wk, f, cg);
+    if (f == 0)
+      hipLaunchKernelGGL((colpass2d_kernel<true>), dim3(64, W), dim3(kTR), lds_col, st, s, wk, f,
+                         cg);
+    else
+      hipLaunchKernelGGL((colpass2d_kernel<false>), dim3(64, W), dim3(kTR), lds_col, st, s, wk, f,
+                         cg);
     hipLaunchKernelGGL(rowifft2d_kernel, dim3(kRowBlocks2, W), dim3(kTR), lds_row, st, s, wk, f,
                        rg);
     hipLaunchKernelGGL(colsum2d_kernel, dim3((n + 255) / 256, W), dim3(256), 0, st, s, wk, f);
