@@ -13,10 +13,17 @@ import subprocess
 
 import pytest
 
+from test_sanitizer_build import stale_sources
+
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 EXE = os.path.join(ROOT, "tests", "cpp", "_build", "lifetime_check_asan")
 
 pytestmark = pytest.mark.gpu
+
+
+def test_executable_is_not_stale():
+    assert os.path.exists(EXE), "build tests/cpp asan first (__graft_entry__.build)"
+    assert stale_sources() == []
 
 
 def test_lifetimes_under_asan():
