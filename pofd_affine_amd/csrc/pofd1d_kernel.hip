@@ -1097,7 +1097,7 @@ __device__ __forceinline__ void forward_window(const BeamsetDev& bs, const Windo
     const double jd = static_cast<double>(j0);
     double rv[Q];
     {
-      const double off = (bs.headneg && j0 > wr) ? bs.mval : 0.0;
+      const double off = (j0 > wr) ? bs.mval : 0.0;
       const int ns = static_cast<int>(g >> 24);
       const double da = fma(jd, dflux, off - na.x);
 #pragma unroll

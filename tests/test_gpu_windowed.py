@@ -87,3 +87,43 @@ def test_windowed_two_signed_beam(nflux):
     assert np.array_equal(lls[0], lls[1]) and np.array_equal(lls[0], lls[2])
     L = build_oracle(inp, nflux, 700, False, th[0])
     check_exact_parity(ctx, L, th, lls[0], tol=1e-6, nthreads=3)
+
+
+@pytest.mark.parametrize("nflux,shift", [(65536, 0), (131072, 0), (65536, 3)])
+def test_negative_fluxes_only_far_from_zero(nflux, shift):
+    """An R range set by hand to a few mJy with 16 nodes up to 450 mJy: the
+    negative node next to zero is then 170 grid points and more from it, past
+    the head of the grid, and the head has no negative side.  The wrapped
+    fluxes start at a multiple of eight points, so that windows are used, or
+    three points on, where a group of eight has both signs and they are not.
+    Against the pruned transforms, which a cut that keeps more than the
+    windows hold selects.  (The reference fills no negative fluxes where the
+    lowest node is below the range: its index wraps.)"""
+    print("[gpu-window-case] far negative %d %d" % (nflux, shift), flush=True)
+    g, ps = synth.gaussian_beam()
+    sigma = 0.0005
+    d = np.random.default_rng(3).normal(0.0, 1.2 * sigma, 3000)
+    inp = dict(beam=np.hstack([g, -0.9 * g]).ravel(), pixsize=ps, data=d,
+               sigma=sigma, minbeamval=1e-6, nbeamhist=120, nbins=200,
+               knots=synth.knot_positions())
+    th = synth.walker_thetas(3, seed=4)
+    th[:, :len(inp["knots"])] -= 5.5
+    full = 0.010
+    neg = (nflux // 2 + shift + 0.5) * full / (nflux - 1)
+    out = []
+    for cut in (64.0, 3e5):
+        ctx = workload.build_context(inp, nflux, 16, binned=True,
+                                     spectral_cut=cut)
+        ctx.set_rrange(0, -neg, full - neg)
+        for parts in (1, 2, 4):
+            ctx.set_parts(parts)
+            ll, st = ctx.loglike_batch(th)
+            assert np.all(st == 0), st
+            assert (_nrows(ctx) == 0) == (shift == 0 and cut == 64.0)
+            out.append((ll, ctx.get_debug(0)))
+    ref, dref = out[-1]
+    for ll, dbg in out:
+        # sums of 1e4 to 1e5 positive terms, each within some 1e-16
+        for key in ("mn", "var_noi", "r0"):
+            assert dbg[key] == pytest.approx(dref[key], rel=1e-10), key
+        np.testing.assert_allclose(ll, ref, rtol=0, atol=1e-8)
