@@ -430,6 +430,10 @@ __global__ __launch_bounds__(kT) void rpieces2d_kernel(const Set2Dev s, const Wo
                    : cts * ieta1 * isigma * s.prefac);
         c1 = logf1 + colour_eval(ok, ovl, ocf, no, f1prod, 0.0, false) - bc.logratio[jj];
         c2 = -0.5 * isigma * isigma * ilog2toe;
+        // an infinite weight (a colour width of zero) has no value where its
+        // Gaussian is zero: NaN at every point, as a term that the fill may
+        // not skip
+        if (!isfinite(c0)) c1 = __longlong_as_double(0x7ff8000000000000ULL);
       }
     }
   }

@@ -47,3 +47,28 @@ def test_second_dataset_is_the_first(n):
     assert np.array_equal(sa, sb)
     ok = sa == 0
     assert np.array_equal(b[ok], a[ok] + a[ok])
+
+
+@pytest.mark.parametrize("n", [64, 256, 1024])
+@pytest.mark.parametrize("signed", [False, True])
+def test_colour_width_of_zero_is_no_model(n, signed):
+    """A colour width that is interpolated through zero makes weights of R
+    infinite; where their Gaussians are zero R has no value, and the walker
+    must fail as in the reference, whatever the rows in which that happens."""
+    print("[gpu2d-size-case] zero width %d %s" % (n, signed), flush=True)
+    inp = make_inputs2d(npix_side=60, seed=5, nbins=40, nbeamhist=30)
+    if signed:
+        inp["beam1"] = inp["beam1"] - 0.3 * np.roll(inp["beam1"], 5, 0)
+        inp["beam2"] = inp["beam2"] - 0.2 * np.roll(inp["beam2"], 4, 1)
+    th0 = synth2d.true_theta()
+    th = np.tile(th0, (4, 1))
+    for w in (1, 2, 3):  # the width at one of its three knots
+        th[w, len(synth2d.KNOTS_MJY) + w - 1] = -0.5
+    ctx = workload2d.build_context2d(inp, n, th0, edge_integ=False)
+    L = build_oracle2d(inp, n, th0, edge_integ=False)
+    ll, st = ctx.loglike2d_batch(th)
+    ref, rst = L.loglike_batch(th, 4)
+    assert np.array_equal(st, rst), (st, rst)
+    assert np.any(rst[1:] != 0)
+    ok = st == 0
+    np.testing.assert_allclose(ll[ok], ref[ok], rtol=0, atol=1e-6)
