@@ -296,9 +296,10 @@ int pofd1d_get_pd(pofd_ctx *ctx, uint32_t walker, int beamset_id,
    kmax (last spectral index kept), nrows, field loglike (before offset),
    status, 1/integral, minflux, P(D) stored as log2, kmax of the beam set,
    sum P, sum j P, sum of P above the split, sigma, then wall-clock ticks
-   (100 MHz) inside the kernels: prep, (unused), forward transform,
-   spectrum and noisy rows, inverse transform, split search,
-   normalise+logL, sum of these */
+   (100 MHz) inside the kernels: prep, then the window of the transforms
+   (1, 2: the windowed ones, nrows 0; 0: the pruned ones), then ticks of the
+   forward transform, spectrum and noisy rows, inverse transform, split
+   search, normalise+logL, sum of these */
 int pofd1d_get_debug(pofd_ctx *ctx, uint32_t walker, int beamset_id,
                      int field_id, double *info);
 /* prtrans after initPD for k = 0..kmax (interleaved re, im), kmax from

@@ -477,7 +477,7 @@ class Context:
                   "tmn", "sgpos", "sgneg", "mn", "var_noi", "r0", "kmax",
                   "nrows", "field_loglike", "status", "itot", "minflux",
                   "pofd_is_log", "kmax_beamset", "S", "SJ", "Shigh", "sigma",
-                  "t_prep", "t_reserved", "t_forward", "t_spectral",
+                  "t_prep", "window", "t_forward", "t_spectral",
                   "t_inverse", "t_split", "t_loglike", "t_total"]
 
     def get_debug(self, walker, b=0, f=0):

@@ -2848,11 +2848,20 @@ __global__ __launch_bounds__(kThreads) void finalize1d_kernel(const BeamsetDev b
         const int bstar = block_max_int(cb, red);
         if (bstar >= 0) {
           int cand = -1;
+          double v = 0.0;
           if (tid < blk) {
             const int i = bstar * blk + tid;
-            if (P(i) < jitter) cand = i;
+            v = P(i);
+            if (v < jitter) cand = i;
           }
           found = block_max_int(cand, red);
+          // the block has a value below jitter: should the values made again
+          // round otherwise than the inverse's, its smallest is that one
+          if (kWindows && found < 0) {
+            int least = (tid < blk) ? bstar * blk + tid : -1;
+            block_argmin(v, least, red);
+            found = least;
+          }
         }
       }
     }
@@ -2953,7 +2962,7 @@ __global__ __launch_bounds__(kThreads) void finalize1d_kernel(const BeamsetDev b
     dbg[18] = (status == POFD_OK && !fd.binned) ? 1.0 : 0.0;
     dbg[22] = Shigh;
     dbg[24] = st[ST_TPREP];
-    dbg[25] = 0.0;
+    dbg[25] = wsel;
     dbg[26] = st[ST_TFWD];
     dbg[27] = st[ST_TSPEC];
     dbg[29] = static_cast<double>(t_split);

@@ -68,6 +68,35 @@ def test_other_spectral_cuts(cut):
         assert np.all(np.isfinite(b)) and np.max(np.abs(b - r)) < 1e-2 * np.max(np.abs(r))
 
 
+@pytest.mark.parametrize("nflux,cut,window", [
+    # 8, 16 (of both windows) and 32 points to a coarse one
+    (65536, None, 1), (65536, 2.5e5, 2), (131072, None, 1), (131072, 2.5e5, 2),
+    (262144, None, 1)])
+def test_values_made_again_are_the_same_bits(nflux, cut, window):
+    """The split search takes minima and peak from the matrix products of the
+    inverse and the values beside them from sums made again: both round alike.
+    The R range is some ten widths of the noise, so that the smallest value of
+    the P(D) is far above rounding and not clamped."""
+    print("[gpu-window-case] bits %d %s" % (nflux, cut), flush=True)
+    sigma = 0.004
+    inp = dict(workload.make_inputs(npix_side=40, seed=9, sigma=sigma))
+    th = np.tile(synth.true_theta(), (24, 1))
+    th[:, :len(inp["knots"])] -= 12.0  # hardly any sources
+    th[:, len(inp["knots"])] = np.linspace(0.65, 1.0, len(th))
+    ctx = workload.build_context(inp, nflux, 512, binned=True,
+                                 spectral_cut=cut)
+    ctx.set_rrange(0, 0.0, 10.2 * sigma)
+    ll, st = ctx.loglike_batch(th)
+    assert np.all(st == 0), st
+    for w in range(len(th)):
+        dbg = ctx.get_debug(w)
+        raw = ctx.get_pd(w, is_log="raw")[0]
+        assert dbg["window"] == window
+        assert raw.max() == dbg["peak"]
+        assert 0 < dbg["minval"] < 1e-5 * dbg["peak"]
+        assert raw[int(dbg["minidx"])] == dbg["minval"] == raw.min()
+
+
 @pytest.mark.parametrize("nflux", [65536, 131072])
 def test_windowed_two_signed_beam(nflux):
     print("[gpu-window-case] negative beam %d" % nflux, flush=True)
