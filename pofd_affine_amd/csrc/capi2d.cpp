@@ -672,6 +672,8 @@ int prepare_set2(pofd_ctx* c, Ctx2& C2, Set2& s) {
     pofd::gauss_legendre(32, d.glx, d.glw);
   }
   int rc;
+  if ((rc = pofd2::init_kernels2d()))
+    return ctx_fail(c, rc, "pofd2d_prepare: hipFuncSetAttribute failed");
   if ((rc = upload(c, s, rf1, &d.rflux1))) return rc;
   if ((rc = upload(c, s, rf2, &d.rflux2))) return rc;
   if ((rc = upload(c, s, edge1, &d.edge1))) return rc;
@@ -957,7 +959,8 @@ int pofd2d_configure(pofd_ctx* c, uint32_t n, uint32_t nedge, int edge_integ,
                      double min_sigma, double exp_conf1, double exp_conf2) {
   Ctx2* C2 = get2(c);
   if (!C2) return POFD_E_ARG;
-  if (n < 64 || n > 4096 || (n & (n - 1)))
+  if (n < static_cast<uint32_t>(pofd2::kMinN) || n > static_cast<uint32_t>(pofd2::kMaxN) ||
+      (n & (n - 1)))
     return ctx_fail(c, POFD_E_ARG, "pofd2d_configure: n must be a power of two in [64, 4096]");
   if (edge_integ && (nedge < 2 || nedge > n))
     return ctx_fail(c, POFD_E_ARG, "PDFactoryDouble::initR: Nedge is less than R fill size");

@@ -17,6 +17,7 @@ void gauss_legendre(int n, double* x, double* w);
 
 namespace pofd2 {
 
+constexpr int kMinN = 64, kMaxN = 4096;  // grid sizes
 constexpr int kMaxK = 32;          // knots, sigma knots, offset knots (each)
 constexpr int kMaxFields2 = 8;     // datasets per beam set
 constexpr int kLikeBlocks = 64;    // workgroups per (walker, dataset) in like2d
@@ -139,7 +140,9 @@ double ctx_spectral_cut(const pofd_ctx* c);
 int ctx_fail(pofd_ctx* c, int code, const std::string& msg);
 int ctx_stage_events(pofd_ctx* c, hipEvent_t** ev);
 
-// launcher (pofd2d_kernel.hip)
+// launcher (pofd2d_kernel.hip); init_kernels2d on the device (current) before
+// the first launch there
+int init_kernels2d();
 int launch_loglike2d(const Set2Dev& s, const Work2& wk, const RGrid& gmain,
                      const RGrid& g00, const RGrid& gx, const RGrid& gy,
                      const float* d_theta, uint32_t stride, double* d_ll,

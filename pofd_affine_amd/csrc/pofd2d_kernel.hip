@@ -1363,6 +1363,35 @@ __global__ __launch_bounds__(kT) void rstats2d_kernel(const Set2Dev s, const Wor
 
 namespace pofd2 {
 
+// dynamic LDS of the transforms: a quarter turn of twiddles and both buffers
+// of each row or column
+inline size_t row_lds(const int n) {
+  return (static_cast<size_t>(n / 8) + rows_together(n) * (n + 2)) * sizeof(double2);
+}
+inline size_t col_lds(const int n) {
+  return (static_cast<size_t>(n / 4) + cols_together(n) * 2 * n) * sizeof(double2);
+}
+
+// Allows the transforms the LDS of the largest grid on the current device.
+// The attribute belongs to the kernel, not to a context: one value for all,
+// so that no thread lowers it between another's call and launch.
+int init_kernels2d() {
+  size_t row = 0, col = 0;
+  for (int n = kMinN; n <= kMaxN; n *= 2) {
+    row = std::max(row, row_lds(n));
+    col = std::max(col, col_lds(n));
+  }
+  auto allow = [](const void* k, const size_t bytes) {
+    return hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize,
+                               static_cast<int>(bytes)) == hipSuccess;
+  };
+  const bool ok = allow(reinterpret_cast<const void*>(rowfft2d_kernel), row) &&
+                  allow(reinterpret_cast<const void*>(rowifft2d_kernel), row) &&
+                  allow(reinterpret_cast<const void*>(colpass2d_kernel<true>), col) &&
+                  allow(reinterpret_cast<const void*>(colpass2d_kernel<false>), col);
+  return ok ? POFD_OK : POFD_E_INTERNAL;
+}
+
 int launch_loglike2d(const Set2Dev& s, const Work2& wk, const RGrid& gmain,
                      const RGrid& g00, const RGrid& gx, const RGrid& gy,
                      const float* d_theta, uint32_t stride, double* d_ll,
@@ -1402,17 +1431,7 @@ int launch_loglike2d(const Set2Dev& s, const Work2& wk, const RGrid& gmain,
   if (s.edge_integ) edge_rows(gy, wk.ry);
   const int nparts = 64;
   const int rg = rows_together(n), cg = cols_together(n);
-  // a quarter turn of twiddles and both buffers of each row or column
-  const size_t lds_row = (static_cast<size_t>(n / 8) + rg * (n + 2)) * sizeof(double2);
-  const size_t lds_col = (static_cast<size_t>(n / 4) + cg * 2 * n) * sizeof(double2);
-  for (const void* k : {reinterpret_cast<const void*>(rowfft2d_kernel),
-                        reinterpret_cast<const void*>(rowifft2d_kernel)})
-    (void)hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize,
-                              static_cast<int>(lds_row));
-  for (const void* k : {reinterpret_cast<const void*>(colpass2d_kernel<true>),
-                        reinterpret_cast<const void*>(colpass2d_kernel<false>)})
-    (void)hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize,
-                              static_cast<int>(lds_col));
+  const size_t lds_row = row_lds(n), lds_col = col_lds(n);
   hipLaunchKernelGGL(rowfft2d_kernel, dim3(nparts, W), dim3(kTR), lds_row, st, s, wk, gmain, rg);
   hipLaunchKernelGGL(rstats2d_kernel, dim3(W), dim3(kT), 0, st, s, wk, nparts);
   mark(POFD_STAGE_INVERSE);

@@ -3,6 +3,8 @@ differently: eight short rows a workgroup (and transforms too short for the
 swizzled order), four and two long ones, one column at the largest grid; odd
 and even powers of two, with and without the edge integrals, and a second
 dataset, against the CPU oracle."""
+import threading
+
 import numpy as np
 import pytest
 
@@ -72,3 +74,31 @@ def test_colour_width_of_zero_is_no_model(n, signed):
     assert np.any(rst[1:] != 0)
     ok = st == 0
     np.testing.assert_allclose(ll[ok], ref[ok], rtol=0, atol=1e-6)
+
+
+def test_small_and_large_grids_in_two_threads():
+    """A thread each for the smallest and the largest grid: what the kernels
+    may use of LDS is one setting for the process, and a small grid's calls
+    must not take it from a large one's."""
+    print("[gpu2d-size-case] two threads", flush=True)
+    inp = make_inputs2d(npix_side=60, seed=5, nbins=40, nbeamhist=30)
+    th0 = synth2d.true_theta()
+    th = synth2d.walker_thetas(1, seed=19)
+    ctxs = {n: workload2d.build_context2d(inp, n, th0, nedge=16)
+            for n in (4096, 64)}
+    alone = {n: c.loglike2d_batch(th) for n, c in ctxs.items()}
+    got = {n: [] for n in ctxs}
+
+    def work(n, calls):
+        got[n] += [ctxs[n].loglike2d_batch(th) for _ in range(calls)]
+    threads = [threading.Thread(target=work, args=a)
+               for a in ((4096, 20), (64, 100))]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    for n, calls in ((4096, 20), (64, 100)):
+        assert len(got[n]) == calls
+        for ll, st in got[n]:
+            assert np.array_equal(st, alone[n][1])
+            assert np.array_equal(ll, alone[n][0], equal_nan=True)
