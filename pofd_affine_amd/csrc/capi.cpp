@@ -257,13 +257,14 @@ int upload_pixels(pofd_ctx* c, FieldHost& fh, int N, double dflux, FieldDev& fd)
   // The core is the run of cell widths with the largest excess of pixels
   // over cells (a confused map: 99% of its pixels in 8,000 of 60,000 cells):
   // there a sum by cells costs less than one by pixels, outside it more.
-  // Data reaching far beyond the grid (an R range set by hand) get none.
+  // Data reaching far beyond the grid (an R range set by hand) get none, nor
+  // do maps with more pixels than the ranks' 32 bits count.
   fd.pa = fd.pb = fd.rcols = 0;
   fd.rlog = 0;
   fd.ca = cmin;
   fd.rank = nullptr;
   const double ncell = (cmax - cmin) / dflux + 2.0;
-  if (ncell <= 4.0 * N) {
+  if (ncell <= 4.0 * N && n < (size_t(1) << 32)) {
     const uint32_t cols = static_cast<uint32_t>(ncell);
     std::vector<uint32_t> cnt(cols, 0);
     for (size_t i = 0; i < n; ++i)

@@ -3048,7 +3048,7 @@ __global__ __launch_bounds__(kPixThreads) void pixels1d_kernel(const BeamsetDev 
   const int e_hi = static_cast<int>(
       fmin(fmax(dlo + static_cast<double>(rcols) + 3.0, 0.0), static_cast<double>(N - 2)));
   const int nchunk = (pa < pb) ? max((e_hi - e_lo + 62) / 63, 1) : 0;
-  const uint32_t nout = static_cast<uint32_t>(fd.npix) - (pb - pa);
+  const uint64_t nout = fd.npix - (pb - pa);
   const int nstep = nchunk + static_cast<int>((nout + 63) >> 6);
   const double unit = ldexp(1.0, fd.pexp);
   const double tscale = ldexp(idflux, -fd.pexp);
@@ -3060,7 +3060,7 @@ __global__ __launch_bounds__(kPixThreads) void pixels1d_kernel(const BeamsetDev 
     if (st >= nchunk) {
       // 64 pixels outside the core, as PD::getLogLike takes them: L_0 at or
       // below minflux, L_N-1 at or above maxflux - dflux
-      const uint32_t k0 = (static_cast<uint32_t>(st - nchunk) << 6) + lane;
+      const uint64_t k0 = (static_cast<uint64_t>(st - nchunk) << 6) + lane;
       if (k0 < nout) {
         const double c = pix[(k0 < pa) ? k0 : k0 - pa + pb].c;
         const bool lo = c <= minflux, hi = c >= fma(static_cast<double>(N - 2), dflux, minflux);
