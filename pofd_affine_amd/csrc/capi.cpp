@@ -234,9 +234,10 @@ std::vector<double2> twiddles(size_t n, size_t count) {
 // The tables of an unbinned dataset (fh.pix ascending) for a P(D) grid of N
 // fluxes of step dflux: the pixels with their running sums in fixed point,
 // and the ranks of the core's on a sub-grid of the P(D)'s cells.
-int upload_pixels(pofd_ctx* c, FieldHost& fh, int N, double dflux, FieldDev& fd) {
+int upload_pixels(pofd_ctx* c, FieldHost& fh, int N, double dflux, pofd::PixDev& pd) {
   const std::vector<double>& p = fh.pix;
   const size_t n = p.size();
+  pd.npix = n;
   const double cmin = p.front(), cmax = p.back();
   // the unit 2^-pexp: every pixel, the grid's range and a cell's sum of
   // offsets (at most n dflux) stay below 2^62 units
@@ -244,13 +245,13 @@ int upload_pixels(pofd_ctx* c, FieldHost& fh, int N, double dflux, FieldDev& fd)
   const int top = std::max({bits(std::max(std::fabs(cmin), std::fabs(cmax))),
                             bits(static_cast<double>(n) * dflux),
                             bits(static_cast<double>(N) * dflux)});
-  fd.pexp = 61 - top;
+  pd.pexp = 61 - top;
   std::vector<pofd::PixSum> ps(n + 1);
   uint64_t q = 0;
   for (size_t i = 0; i < n; ++i) {
     ps[i].c = p[i];
     ps[i].q = static_cast<int64_t>(q);
-    q += static_cast<uint64_t>(static_cast<int64_t>(std::llrint(std::ldexp(p[i], fd.pexp))));
+    q += static_cast<uint64_t>(static_cast<int64_t>(std::llrint(std::ldexp(p[i], pd.pexp))));
   }
   ps[n].c = INFINITY;
   ps[n].q = static_cast<int64_t>(q);
@@ -259,10 +260,10 @@ int upload_pixels(pofd_ctx* c, FieldHost& fh, int N, double dflux, FieldDev& fd)
   // there a sum by cells costs less than one by pixels, outside it more.
   // Data reaching far beyond the grid (an R range set by hand) get none, nor
   // do maps with more pixels than the ranks' 32 bits count.
-  fd.pa = fd.pb = fd.rcols = 0;
-  fd.rlog = 0;
-  fd.ca = cmin;
-  fd.rank = nullptr;
+  pd.pa = pd.pb = pd.rcols = 0;
+  pd.rlog = 0;
+  pd.ca = cmin;
+  pd.rank = nullptr;
   const double ncell = (cmax - cmin) / dflux + 2.0;
   if (ncell <= 4.0 * N && n < (size_t(1) << 32)) {
     const uint32_t cols = static_cast<uint32_t>(ncell);
@@ -283,48 +284,48 @@ int upload_pixels(pofd_ctx* c, FieldHost& fh, int N, double dflux, FieldDev& fd)
         jb = j + 1;
       }
     }
-    fd.rcols = jb - ja;
-    fd.ca = cmin + static_cast<double>(ja) * dflux;
+    pd.rcols = jb - ja;
+    pd.ca = cmin + static_cast<double>(ja) * dflux;
   }
-  if (fd.rcols) {
-    const uint32_t cols = fd.rcols;
-    const double cb = fd.ca + static_cast<double>(cols) * dflux;
-    fd.pa = static_cast<uint32_t>(std::lower_bound(p.begin(), p.end(), fd.ca) - p.begin());
-    fd.pb = static_cast<uint32_t>(std::lower_bound(p.begin(), p.end(), cb) - p.begin());
+  if (pd.rcols) {
+    const uint32_t cols = pd.rcols;
+    const double cb = pd.ca + static_cast<double>(cols) * dflux;
+    pd.pa = static_cast<uint32_t>(std::lower_bound(p.begin(), p.end(), pd.ca) - p.begin());
+    pd.pb = static_cast<uint32_t>(std::lower_bound(p.begin(), p.end(), cb) - p.begin());
     // a search starts from some two pixels on average, one or two cache
     // lines (from five: pixels1d 111 us, not 96, at 256 walkers and 1e6
     // pixels): 2^rlog sub-steps a cell, at most 2^22 entries
     int rlog = 0;
-    while (rlog < 6 && (static_cast<size_t>(fd.pb - fd.pa) >> rlog) > 3 * size_t(cols) &&
+    while (rlog < 6 && (static_cast<size_t>(pd.pb - pd.pa) >> rlog) > 3 * size_t(cols) &&
            (static_cast<size_t>(cols) << (rlog + 1)) <= (size_t(1) << 22))
       ++rlog;
     const uint32_t R = 1u << rlog;
     const double h = dflux / R;
     std::vector<uint32_t> rank(static_cast<size_t>(R + 1) * cols);
-    uint32_t at = fd.pa;
+    uint32_t at = pd.pa;
     for (uint32_t j = 0; j < cols; ++j) {
       for (uint32_t r = 0; r < R; ++r) {
-        const double edge = fd.ca + (static_cast<double>(j) * R + r) * h;
-        while (at < fd.pb && p[at] < edge) ++at;
+        const double edge = pd.ca + (static_cast<double>(j) * R + r) * h;
+        while (at < pd.pb && p[at] < edge) ++at;
         rank[static_cast<size_t>(r) * cols + j] = at;
         if (r == 0 && j > 0) rank[static_cast<size_t>(R) * cols + j - 1] = at;
       }
     }
-    rank[static_cast<size_t>(R) * cols + cols - 1] = fd.pb;
+    rank[static_cast<size_t>(R) * cols + cols - 1] = pd.pb;
     int rc = dev_alloc(c, fh.drank, rank.size() * sizeof(uint32_t));
     if (rc) return rc;
     hipError_t e = hipMemcpy(fh.drank->p, rank.data(), rank.size() * sizeof(uint32_t),
                              hipMemcpyHostToDevice);
     if (e != hipSuccess) return hip_fail(c, e, "hipMemcpy(rank)");
-    fd.rank = static_cast<const uint32_t*>(fh.drank->p);
-    fd.rlog = rlog;
+    pd.rank = static_cast<const uint32_t*>(fh.drank->p);
+    pd.rlog = rlog;
   }
   int rc = dev_alloc(c, fh.dpix, ps.size() * sizeof(pofd::PixSum));
   if (rc) return rc;
   hipError_t e = hipMemcpy(fh.dpix->p, ps.data(), ps.size() * sizeof(pofd::PixSum),
                            hipMemcpyHostToDevice);
   if (e != hipSuccess) return hip_fail(c, e, "hipMemcpy(pix)");
-  fd.pix = static_cast<const pofd::PixSum*>(fh.dpix->p);
+  pd.pix = static_cast<const pofd::PixSum*>(fh.dpix->p);
   return POFD_OK;
 }
 
@@ -751,7 +752,6 @@ int prepare_beamset(pofd_ctx* c, Beamset& s) {
     fd.nbins = static_cast<uint32_t>(fh.bins.size());
     fd.bincent0 = fh.bincent0;
     fd.bindelta = fh.bindelta;
-    fd.npix = fh.binned ? 0 : fh.pix.size();
     if (fh.binned) {
       if ((rc = dev_alloc(c, fh.dbins, fh.bins.size() * sizeof(uint32_t)))) return rc;
       hipError_t e = hipMemcpy(fh.dbins->p, fh.bins.data(),
@@ -759,10 +759,8 @@ int prepare_beamset(pofd_ctx* c, Beamset& s) {
                                hipMemcpyHostToDevice);
       if (e != hipSuccess) return hip_fail(c, e, "hipMemcpy(bins)");
       fd.bins = static_cast<const uint32_t*>(fh.dbins->p);
-      fd.pix = nullptr;
     } else {
-      if ((rc = upload_pixels(c, fh, static_cast<int>(N), dflux, fd))) return rc;
-      fd.bins = nullptr;
+      if ((rc = upload_pixels(c, fh, static_cast<int>(N), dflux, d.pix[f]))) return rc;
     }
   }
   s.wcap = 0;  // workspace layout depends on the tables

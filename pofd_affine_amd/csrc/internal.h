@@ -56,16 +56,19 @@ struct PixSum {
   int64_t q;
 };
 
-// One field (dataset) of a beam set, device view.
+// One field (dataset) of a beam set, device view: what every kernel reads of
+// it, one 64-byte line
 struct FieldDev {
   double sigma_base;
   double like_offset;
   double like_norm;
   int binned;
-  const uint32_t* bins;   // nbins
   uint32_t nbins;
+  const uint32_t* bins;   // nbins
   double bincent0, bindelta;
-  // unbinned only
+};
+// and the pixels of an unbinned one
+struct PixDev {
   uint64_t npix;
   const PixSum* pix;      // npix + 1, ascending
   int pexp;
@@ -147,14 +150,17 @@ struct BeamsetDev {
   // largest values (fluxes near zero); they are left out of the transform
   // and their part of R^(k) - R^(0) is summed directly (forward_tail)
   int headn, headneg;
+  int nfields;
+  int nwin;               // windows, by growing nc (0: none fits N)
+  FieldDev fields[kMaxFields];
+  // what the windowed transforms and the unbinned sum read, behind what all
+  // kernels do (a kernel argument's lines are cold at each launch)
+  PixDev pix[kMaxFields];
+  WindowDev win[2];
+  const double2* wc;      // kMaxNc/2: exp(-2 pi i t/kMaxNc)
   // below rlow (and within rlown of the grid's end, with a negative beam)
   // eight grid points may lie in more than two node intervals; at most kRlow
   int rlow, rlown;
-  int nwin;               // windows, by growing nc (0: none fits N)
-  WindowDev win[2];
-  const double2* wc;      // kMaxNc/2: exp(-2 pi i t/kMaxNc)
-  int nfields;
-  FieldDev fields[kMaxFields];
 };
 
 // Per-walker device workspace layout (doubles), sized by the host.

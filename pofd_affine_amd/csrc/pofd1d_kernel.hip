@@ -495,6 +495,17 @@ struct WindowSmem {
   int isc[2 + kMaxFields];
 };
 
+// a transform kernel's LDS: the windowed one's too where there are windows
+template <bool kWindows, class W>
+union XformLds {
+  XformSmem x;
+  W w;
+};
+template <class W>
+union XformLds<false, W> {
+  XformSmem x;
+};
+
 __device__ void load_twiddles(const BeamsetDev& bs, XformSmem& sm) {
   for (int i = threadIdx.x; i < kM1; i += blockDim.x) sm.wlo[i] = bs.Wlo[i];
   for (int i = threadIdx.x; i < 3 * kStageTw; i += blockDim.x) {
@@ -663,6 +674,14 @@ __global__ __launch_bounds__(kThreads) void prep1d_kernel(
       sm.be[j] = bs.bieta[j];
     }
   }
+  // the transforms' window, beside the knot spline (behind it the choice
+  // costs every call its latency, 1.6 us)
+  if (part == 0 && tid == kThreads - 1) {
+    int kmaxb = 0;
+    st[ST_WIN] = select_window(
+        bs, static_cast<double>(theta[static_cast<size_t>(walker) * stride + nk]), kmaxb);
+    st[ST_KMAXB] = kmaxb;
+  }
   if (tid < 64) {
     // The knot spline on the 64 lanes of wave 0 (nknots <= 64), lane l for
     // knot or interval l: GSL's natural cubic spline through (logknots,
@@ -725,9 +744,6 @@ __global__ __launch_bounds__(kThreads) void prep1d_kernel(
       if (part == 0) {
         st[ST_STATUS] = status;
         st[ST_SIGMULT] = sigmult;
-        int kmaxb = 0;
-        st[ST_WIN] = (status == POFD_OK) ? select_window(bs, sigmult, kmaxb) : 0;
-        st[ST_KMAXB] = kmaxb;
       }
       sm.isc[0] = status;
       sm.isc[1] = valid ? 1 : 0;
@@ -1597,11 +1613,28 @@ __device__ __forceinline__ void forward_windowed(const BeamsetDev& bs, const Wor
 // spectrum itself; with more, each writes its partial kept rows and partial
 // moments and spectrum1d_kernel combines them by the group tree and
 // finishes.  Either way the rows and moments are the same bits.
-__device__ __forceinline__ void forward_pruned(const BeamsetDev& bs, const WorkDev& wk,
-                                               XformSmem& sm, const int walker, const int part,
-                                               const int parts) {
+// kWindows: the beam set has windows, and a walker whose spectrum fits one
+// takes it
+template <bool kWindows>
+__global__ __launch_bounds__(kThreads) void forward1d_kernel(const BeamsetDev bs,
+                                                              const WorkDev wk) {
+  __shared__ XformLds<kWindows, WindowSmem> smu;
+  XformSmem& sm = smu.x;
   const int tid = threadIdx.x;
+  const int n = batch_n(wk);
+  const int parts = batch_parts(n, wk.force_parts, wk.nslots, wk.parts_tab);
+  const int walker = blockIdx.x / parts;
+  const int part = blockIdx.x - walker * parts;
+  if (walker >= n) return;
   double* st = walker_state(wk, walker);
+  if (st[ST_STATUS] != POFD_OK) return;  // uniform across the workgroup
+  if constexpr (kWindows) {
+    const int wsel = static_cast<int>(st[ST_WIN]);
+    if (wsel) {
+      forward_windowed(bs, wk, smu.w, bs.win[wsel - 1], walker, part, parts);
+      return;
+    }
+  }
   unsigned long long tmark = wall_clock64();
   const int M2 = bs.M2;
   const double dflux = bs.dflux;
@@ -1852,41 +1885,12 @@ __device__ __forceinline__ void forward_pruned(const BeamsetDev& bs, const WorkD
   forward_tail(bs, wk, walker, sm, mn, var, tmark);
 }
 
-// kWindows: the beam set has windows, and a walker whose spectrum fits one
-// takes it
-template <bool kWindows>
-__global__ __launch_bounds__(kThreads) void forward1d_kernel(const BeamsetDev bs,
-                                                              const WorkDev wk) {
-  __shared__ union {
-    XformSmem x;
-    WindowSmem w;
-  } sm;
-  const int n = batch_n(wk);
-  const int parts = batch_parts(n, wk.force_parts, wk.nslots, wk.parts_tab);
-  const int walker = blockIdx.x / parts;
-  const int part = blockIdx.x - walker * parts;
-  if (walker >= n) return;
-  const double* st = walker_state(wk, walker);
-  if (st[ST_STATUS] != POFD_OK) return;  // uniform across the workgroup
-  if constexpr (kWindows) {
-    const int wsel = static_cast<int>(st[ST_WIN]);
-    if (wsel) {
-      forward_windowed(bs, wk, sm.w, bs.win[wsel - 1], walker, part, parts);
-      return;
-    }
-  }
-  forward_pruned(bs, wk, sm.x, walker, part, parts);
-}
-
 // the parts' kept rows (or coarse points) and moments combined by the group
 // tree, then the spectrum and the inverse's input (one workgroup per walker)
 template <bool kWindows>
 __global__ __launch_bounds__(kThreads) void spectrum1d_kernel(const BeamsetDev bs,
                                                                const WorkDev wk) {
-  __shared__ union {
-    XformSmem x;
-    WindowSmem w;
-  } smu;
+  __shared__ XformLds<kWindows, WindowSmem> smu;
   const int tid = threadIdx.x;
   const int walker = blockIdx.x;
   const int n = batch_n(wk);
@@ -1910,33 +1914,35 @@ __global__ __launch_bounds__(kThreads) void spectrum1d_kernel(const BeamsetDev b
   double2* zrows = wk.zrows + walker * wk.zrows_stride;
   const double2* zp = wk.zpart + p0 * wk.zpart_stride;
   const size_t zs = wk.zpart_stride;
-  const int wsel = kWindows ? static_cast<int>(st[ST_WIN]) : 0;
-  if (wsel) {
-    // the parts' coarse points, with what each strip's first points miss
-    WindowSmem& sm = smu.w;
-    const WindowDev& win = bs.win[wsel - 1];
-    window_setup(bs, win, st, sm);
-    const int nc = win.nc, nl = nc / kStrips, cpp = nc / parts, spp = kStrips / parts;
-    const double* seg = reinterpret_cast<const double*>(zp);
-    const size_t ss = 2 * zs;  // doubles per slot
-    for (int i = tid; i < nc; i += kThreads) {
-      const int at = i & (nl - 1), t = at - (nl - 15);
-      double v = seg[(i / cpp) * ss + i % cpp];
-      if (t >= 0) {
-        const int nxt = (i / nl + 1) & (kStrips - 1);
-        v += seg[(nxt / spp) * ss + cpp + (nxt % spp) * kTaps + t];
+  if constexpr (kWindows) {
+    const int wsel = static_cast<int>(st[ST_WIN]);
+    if (wsel) {
+      // the parts' coarse points, with what each strip's first points miss
+      WindowSmem& sm = smu.w;
+      const WindowDev& win = bs.win[wsel - 1];
+      window_setup(bs, win, st, sm);
+      const int nc = win.nc, nl = nc / kStrips, cpp = nc / parts, spp = kStrips / parts;
+      const double* seg = reinterpret_cast<const double*>(zp);
+      const size_t ss = 2 * zs;  // doubles per slot
+      for (int i = tid; i < nc; i += kThreads) {
+        const int at = i & (nl - 1), t = at - (nl - 15);
+        double v = seg[(i / cpp) * ss + i % cpp];
+        if (t >= 0) {
+          const int nxt = (i / nl + 1) & (kStrips - 1);
+          v += seg[(nxt / spp) * ss + cpp + (nxt % spp) * kTaps + t];
+        }
+        put_coarse(bs, sm, nc, (i + 8) & (nc - 1), v);
       }
-      put_coarse(bs, sm, nc, (i + 8) & (nc - 1), v);
+      const HeadLayout hl = head_layout(bs, sm);
+      const int H = bs.headn;
+      const double* hs = seg + cpp + spp * kTaps;
+      for (int i = tid; i < H; i += kThreads) hl.hp[i] = hs[i];
+      for (int i = tid; i < H + kHeadBlk; i += kThreads) hl.hn[i] = hs[(parts - 1) * ss + H + i];
+      __syncthreads();
+      window_head_sums(bs, sm);
+      window_tail<true>(bs, wk, walker, sm, win, mn, var, tmark);
+      return;
     }
-    const HeadLayout hl = head_layout(bs, sm);
-    const int H = bs.headn;
-    const double* hs = seg + cpp + spp * kTaps;
-    for (int i = tid; i < H; i += kThreads) hl.hp[i] = hs[i];
-    for (int i = tid; i < H + kHeadBlk; i += kThreads) hl.hn[i] = hs[(parts - 1) * ss + H + i];
-    __syncthreads();
-    window_head_sums(bs, sm);
-    window_tail<true>(bs, wk, walker, sm, win, mn, var, tmark);
-    return;
   }
   XformSmem& sm = smu.x;
   {
@@ -2148,15 +2154,14 @@ __device__ void forward_tail(const BeamsetDev& bs, const WorkDev& wk, const int 
 // getPD's sgpos / sgneg (src/PDFactory.cc:1225-1232) and findSplitPoint's
 // search range [bot, top] (:790-801) of one dataset
 struct SplitRange {
-  double sigma, sgpos, sgneg;
+  double sgpos, sgneg;
   int bot, top;
 };
-__device__ __forceinline__ SplitRange split_range(const BeamsetDev& bs, const double sigma,
-                                                  const double var) {
+__device__ __forceinline__ SplitRange split_range(const BeamsetDev& bs, const double sgpos,
+                                                  const double sgneg) {
   SplitRange r;
-  r.sigma = sigma;
-  r.sgpos = sqrt(var + sigma * sigma);
-  r.sgneg = (9 * sigma * sigma > var) ? sigma : r.sgpos;
+  r.sgpos = sgpos;
+  r.sgneg = sgneg;
   const double n1sigpos = 2.5 * r.sgpos, n1signeg = 2.5 * r.sgneg;
   double bd = n1sigpos / bs.dflux;
   bd = (bd > 2e9) ? 2e9 : bd;
@@ -2169,6 +2174,11 @@ __device__ __forceinline__ SplitRange split_range(const BeamsetDev& bs, const do
     r.top = static_cast<int>(td);
   }
   return r;
+}
+__device__ __forceinline__ SplitRange split_range_of(const BeamsetDev& bs, const double sigma,
+                                                     const double var) {
+  const double sgpos = sqrt(var + sigma * sigma);
+  return split_range(bs, sgpos, (9 * sigma * sigma > var) ? sigma : sgpos);
 }
 
 // v of the lane n before in a row of 16, round the row
@@ -2313,16 +2323,8 @@ __device__ __forceinline__ void inverse_windowed(const BeamsetDev& bs, const Wor
   const int nc = win.nc, na = nc / parts, a0 = part * na;
   const double* u = coarse_pd(bs, wk, walker, f);
   for (int i = tid; i < na + kTaps - 1; i += kThreads) sm.uw[i] = u[(a0 + i - 7) & (nc - 1)];
-  const SplitRange rg =
-      split_range(bs, st[ST_SIGMULT] * bs.fields[f].sigma_base, st[ST_VAR]);
-  if (part == 0 && tid == kThreads - 1) {
-    dbg[7] = rg.sgpos;
-    dbg[8] = rg.sgneg;
-    dbg[12] = spectral_kmax(rg.sigma, bs.iflux, bs.spectral_cut, bs.M);
-    dbg[13] = 0.0;
-    dbg[19] = st[ST_KMAXB];
-    dbg[23] = rg.sigma;
-  }
+  const double sigma = st[ST_SIGMULT] * bs.fields[f].sigma_base;
+  const SplitRange rg = split_range_of(bs, sigma, st[ST_VAR]);
   double pk = -1.0, mnv = 0.0;
   int mni = -1;
   const int ng = kGroups / parts;
@@ -2349,6 +2351,14 @@ __device__ __forceinline__ void inverse_windowed(const BeamsetDev& bs, const Wor
     sm.mni[wv] = mi;
   }
   __syncthreads();
+  if (part == 0 && tid == kThreads - 1) {
+    dbg[7] = rg.sgpos;
+    dbg[8] = rg.sgneg;
+    dbg[12] = spectral_kmax(sigma, bs.iflux, bs.spectral_cut, bs.M);
+    dbg[13] = 0.0;
+    dbg[19] = st[ST_KMAXB];
+    dbg[23] = sigma;
+  }
   if (tid >= 16) return;
   // the wavefronts' results over 16 lanes, the groups by the tree
   pk = sm.peak[tid];
@@ -2397,10 +2407,7 @@ __device__ __forceinline__ void inverse_windowed(const BeamsetDev& bs, const Wor
 template <bool kWindows>
 __global__ __launch_bounds__(kThreads) void inverse1d_kernel(const BeamsetDev bs,
                                                               const WorkDev wk) {
-  __shared__ union {
-    XformSmem x;
-    InverseSmem w;
-  } smu;
+  __shared__ XformLds<kWindows, InverseSmem> smu;
   XformSmem& sm = smu.x;
   const int tid = threadIdx.x;
   const int n = batch_n(wk);
@@ -2429,25 +2436,27 @@ __global__ __launch_bounds__(kThreads) void inverse1d_kernel(const BeamsetDev bs
   const double2* zp =
       wk.zrows + walker * wk.zrows_stride + static_cast<size_t>(1 + f) * M;
   const double sigmult = st[ST_SIGMULT];
-  const SplitRange rg = split_range(bs, sigmult * fd.sigma_base, st[ST_VAR]);
-  const int botidx = rg.bot, topidx = rg.top;
 
   load_twiddles(bs, sm);
   int kmaxb;
   const int nr_rows = spectral_rows(bs, sigmult, sm.rowk2, sm.rowof, kmaxb);
   if (tid == 0) {
+    const double sigma = sigmult * fd.sigma_base;
+    const SplitRange rg = split_range_of(bs, sigma, st[ST_VAR]);
     sm.isc[0] = nr_rows;
+    sm.isc[1] = rg.bot;
+    sm.isc[2] = rg.top;
     if (part == 0) {
       dbg[7] = rg.sgpos;
       dbg[8] = rg.sgneg;
-      dbg[12] = spectral_kmax(rg.sigma, bs.iflux, bs.spectral_cut, M);
+      dbg[12] = spectral_kmax(sigma, bs.iflux, bs.spectral_cut, M);
       dbg[13] = sm.isc[0];
       dbg[19] = kmaxb;
-      dbg[23] = rg.sigma;
+      dbg[23] = sigma;
     }
   }
   __syncthreads();
-  const int nrows = sm.isc[0];
+  const int nrows = sm.isc[0], botidx = sm.isc[1], topidx = sm.isc[2];
   const int nchunks = M2 / kChunk;
   const int g_lo = part * kGroups / parts, g_hi = (part + 1) * kGroups / parts;
   const int c_lo = group_chunk(g_lo, nchunks), c_hi = group_chunk(g_hi, nchunks);
@@ -2683,14 +2692,16 @@ __global__ __launch_bounds__(kThreads) void finalize1d_kernel(const BeamsetDev b
   // the P(D): stored, or made from the coarse one
   const int wsel = kWindows ? static_cast<int>(st[ST_WIN]) : 0;
   int lp = 0, blk = kBlk, nbc = bs.M2 / kChunk;  // P(D) blocks per transform row
-  if (wsel) {
-    const WindowDev& win = bs.win[wsel - 1];
-    lp = __builtin_ctz(static_cast<unsigned>(win.p));
-    blk = 16 * win.p;
-    nbc = 0;
-    const double* u = coarse_pd(bs, wk, walker, f);
-    for (int i = tid; i < win.nc + kTaps - 1; i += kThreads) uw[i] = u[(i - 7) & (win.nc - 1)];
-    load_window(win, ht);
+  if constexpr (kWindows) {
+    if (wsel) {
+      const WindowDev& win = bs.win[wsel - 1];
+      lp = __builtin_ctz(static_cast<unsigned>(win.p));
+      blk = 16 * win.p;
+      nbc = 0;
+      const double* u = coarse_pd(bs, wk, walker, f);
+      for (int i = tid; i < win.nc + kTaps - 1; i += kThreads) uw[i] = u[(i - 7) & (win.nc - 1)];
+      load_window(win, ht);
+    }
   }
   auto P = [&](const int i) { return wsel ? window_value(uw, ht, lp, i) : pofd[i]; };
   double* dbg = wk.dbg + wf * kDbg;
@@ -2733,7 +2744,7 @@ __global__ __launch_bounds__(kThreads) void finalize1d_kernel(const BeamsetDev b
   const double sgpos = dbg[7], sgneg = dbg[8];
   const double peak = dbg[1];
   const double S = dbg[20], SJ = dbg[21];
-  const SplitRange rg = split_range(bs, dbg[23], st[ST_VAR]);
+  const SplitRange rg = split_range(bs, sgpos, sgneg);
   const int botidx = rg.bot, topidx = rg.top;
 
   // the values around the minimum and at the ends of the search range: made
@@ -2999,6 +3010,7 @@ __global__ __launch_bounds__(kPixThreads) void pixels1d_kernel(const BeamsetDev 
   const int blk = blockIdx.y;
   const int f = blockIdx.z;
   const FieldDev& fd = bs.fields[f];
+  const PixDev& pd = bs.pix[f];
   if (fd.binned || walker >= batch_n(wk)) return;
   const size_t wf = static_cast<size_t>(walker) * bs.nfields + f;
   double* out = wk.upart + wf * kPixBlocks + blk;
@@ -3039,21 +3051,21 @@ __global__ __launch_bounds__(kPixThreads) void pixels1d_kernel(const BeamsetDev 
     }
     return log2_or_small(v * itot);
   };
-  const uint32_t pa = fd.pa, pb = fd.pb, rcols = fd.rcols;
+  const uint32_t pa = pd.pa, pb = pd.pb, rcols = pd.rcols;
   const int lane = threadIdx.x & 63;
-  const PixSum* pix = fd.pix;
+  const PixSum* pix = pd.pix;
   // the edges [e_lo, e_hi] around the core, one cell to spare either side
-  const double dlo = floor((fd.ca - minflux) * idflux) - 1.0;
+  const double dlo = floor((pd.ca - minflux) * idflux) - 1.0;
   const int e_lo = static_cast<int>(fmin(fmax(dlo, 0.0), static_cast<double>(N - 2)));
   const int e_hi = static_cast<int>(
       fmin(fmax(dlo + static_cast<double>(rcols) + 3.0, 0.0), static_cast<double>(N - 2)));
   const int nchunk = (pa < pb) ? max((e_hi - e_lo + 62) / 63, 1) : 0;
-  const uint64_t nout = fd.npix - (pb - pa);
+  const uint64_t nout = pd.npix - (pb - pa);
   const int nstep = nchunk + static_cast<int>((nout + 63) >> 6);
-  const double unit = ldexp(1.0, fd.pexp);
-  const double tscale = ldexp(idflux, -fd.pexp);
-  const double rstep = ldexp(idflux, fd.rlog), rend = ldexp(static_cast<double>(rcols), fd.rlog);
-  const uint32_t rmask = (1u << fd.rlog) - 1u;
+  const double unit = ldexp(1.0, pd.pexp);
+  const double tscale = ldexp(idflux, -pd.pexp);
+  const double rstep = ldexp(idflux, pd.rlog), rend = ldexp(static_cast<double>(rcols), pd.rlog);
+  const uint32_t rmask = (1u << pd.rlog) - 1u;
   double part = 0.0;
   for (int st = blk * (kPixThreads / 64) + (threadIdx.x >> 6); st < nstep;
        st += kPixBlocks * (kPixThreads / 64)) {
@@ -3079,14 +3091,14 @@ __global__ __launch_bounds__(kPixThreads) void pixels1d_kernel(const BeamsetDev 
     const double fe = fma(de, dflux, minflux);
     // the rank of the edge among the core's pixels: from the table's bounds
     uint32_t lo = pa, hi = pa;
-    const double x = (fe - fd.ca) * rstep;
+    const double x = (fe - pd.ca) * rstep;
     if (x >= rend) {
       lo = hi = pb;
     } else if (on && x >= 0.0) {
       const uint32_t xi = static_cast<uint32_t>(x);
-      const uint32_t at = (xi & rmask) * rcols + (xi >> fd.rlog);
-      lo = fd.rank[at];
-      hi = fd.rank[at + rcols];
+      const uint32_t at = (xi & rmask) * rcols + (xi >> pd.rlog);
+      lo = pd.rank[at];
+      hi = pd.rank[at + rcols];
     }
     const double L = on ? Lrot(static_cast<uint32_t>(e)) : 0.0;
     while (lo < hi) {
