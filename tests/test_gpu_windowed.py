@@ -1,8 +1,8 @@
 """The windowed 1D transforms against the pruned ones and the CPU oracle at
 the edges of their range: every grid size that has a window, both coarse
 sizes (a narrow dataset moves the kept spectrum from one to the other and
-past both), split over 1, 2 and 4 workgroups, a two-signed beam, and nodes
-so dense that no window is used."""
+past both) and walkers of each in one batch, split over 1, 2 and 4 workgroups,
+two-signed beams, and nodes so dense that no window is used."""
 import os
 
 import numpy as np
@@ -15,20 +15,23 @@ from pofd_affine_amd import fitsio, synth, workload
 pytestmark = pytest.mark.gpu
 
 
-def _nrows(ctx):
-    """Kept rows of the pruned transform; 0: the windowed one ran."""
-    return int(ctx.get_debug(0)["nrows"])
+def _window(ctx, walker=0):
+    """The window that a walker's transforms took (0: the pruned ones, the
+    only ones that keep rows)."""
+    dbg = ctx.get_debug(walker)
+    assert (dbg["nrows"] == 0) == (dbg["window"] > 0)
+    return int(dbg["window"])
 
 
-@pytest.mark.parametrize("nflux,ninterp,sigma,windowed", [
+@pytest.mark.parametrize("nflux,ninterp,sigma,window", [
     # below 2^16 there is no window
-    (32768, 512, 0.0025, False), (65536, 400, 0.0025, True),
-    (65536, 1023, 0.0025, True), (131072, 2048, 0.0025, True),
-    (262144, 2048, 0.0025, True),
+    (32768, 512, 0.0025, 0), (65536, 400, 0.0025, 1),
+    (65536, 1023, 0.0025, 1), (131072, 2048, 0.0025, 1),
+    (262144, 2048, 0.0025, 1),
     # kept spectra above 1024 (the second window) and above 2048 (none)
-    (65536, 512, 0.0007, True), (131072, 2048, 0.0007, True),
-    (65536, 512, 0.0003, False)])
-def test_windowed_against_exact(nflux, ninterp, sigma, windowed):
+    (65536, 512, 0.0006, 2), (131072, 2048, 0.0006, 2),
+    (65536, 512, 0.0003, 0)])
+def test_windowed_against_exact(nflux, ninterp, sigma, window):
     print("[gpu-window-case] %d %d %g" % (nflux, ninterp, sigma), flush=True)
     inp = dict(workload.make_inputs(npix_side=120, seed=9, sigma=sigma))
     th = synth.walker_thetas(3, seed=21)
@@ -39,33 +42,100 @@ def test_windowed_against_exact(nflux, ninterp, sigma, windowed):
         ll, st = ctx.loglike_batch(th)
         assert np.all(st == 0), st
         lls.append(ll)
-        assert (_nrows(ctx) == 0) == windowed
+        assert _window(ctx) == window
     assert np.array_equal(lls[0], lls[1]) and np.array_equal(lls[0], lls[2])
     L = build_oracle(inp, nflux, ninterp, True, th[0])
     # the contract of every 1D path: 1e-6 of the exact-math value
     check_exact_parity(ctx, L, th, lls[2], tol=1e-6, nthreads=3)
 
 
-@pytest.mark.parametrize("cut", [746.0, 12.0])
-def test_other_spectral_cuts(cut):
-    """A cut that keeps twice the spectrum takes the second window, one that
-    keeps half of it must not take a smaller one than the noise allows."""
-    print("[gpu-window-case] cut %g" % cut, flush=True)
-    inp = dict(workload.make_inputs(npix_side=120, seed=9))
+@pytest.mark.parametrize("sigma,cut,window", [
+    # the default keeps some 290 spectral indices at 2.5 mJy, 1200 at 0.6 mJy
+    (0.0025, 746.0, 2), (0.0025, 12.0, 1),
+    (0.0006, 746.0, 0), (0.0006, 12.0, 2)])
+def test_other_spectral_cuts(sigma, cut, window):
+    """A cut that keeps more of the spectrum takes the next window, or none;
+    one that keeps half of it must not take a smaller one than the noise
+    allows.  The kept spectrum is the default cut's, and the P(D) is the plain
+    inverse transform of what is kept times the noise factor."""
+    print("[gpu-window-case] cut %g %g" % (sigma, cut), flush=True)
+    nflux = 65536
+    inp = dict(workload.make_inputs(npix_side=120, seed=9, sigma=sigma))
     th = synth.walker_thetas(3, seed=22)
-    ref = workload.build_context(inp, 65536, 512, binned=True)
-    ctx = workload.build_context(inp, 65536, 512, binned=True, spectral_cut=cut)
+    ref = workload.build_context(inp, nflux, 512, binned=True)
+    ctx = workload.build_context(inp, nflux, 512, binned=True,
+                                 spectral_cut=cut)
     a, sa = ref.loglike_batch(th)
     b, sb = ctx.loglike_batch(th)
     assert np.all(sa == 0) and np.all(sb == 0)
-    # e^-12 of the DC term is left out at the lower cut: 6e-6 of the peak in
-    # P(D), so only the higher cut is compared with the default one
+    # e^-12 of the DC term is left out at the lower cut, so only the higher
+    # cut's likelihood is the default one's
     if cut > 64:
         np.testing.assert_allclose(a, b, rtol=0, atol=1e-8)
-    else:
-        L = build_oracle(inp, 65536, 512, True, th[0])
-        r, _ = L.loglike_batch(th, 3)
-        assert np.all(np.isfinite(b)) and np.max(np.abs(b - r)) < 1e-2 * np.max(np.abs(r))
+    iflux = 2.0 * np.pi / (nflux * ctx.beamset_info(0)["dflux"])
+    for w in range(len(th)):
+        assert _window(ctx, w) == window
+        kept, full = ctx.get_spectrum(w), ref.get_spectrum(w)
+        n = min(kept.size, full.size)
+        assert kept.size == int(ctx.get_debug(w)["kmax_beamset"]) + 1
+        # |spectrum| <= 1, its exponent's roundings some 1e-14
+        np.testing.assert_allclose(kept[:n], full[:n], rtol=0, atol=1e-12)
+        x = np.zeros(nflux // 2 + 1, dtype=complex)
+        x[:kept.size] = kept
+        x *= np.exp(-0.5 * (sigma * iflux * np.arange(x.size)) ** 2)
+        x[0] = 1.0
+        pd = np.maximum(np.fft.irfft(x) * nflux, 0.0)
+        raw = ctx.get_pd(w, is_log="raw")[0]
+        # the transforms' roundings: log2(n) of 1e-16 of the peak
+        assert np.max(np.abs(raw - pd)) < 1e-14 * pd.max()
+
+
+@pytest.mark.parametrize("binned", [True, False])
+def test_walkers_of_every_window_in_one_batch(binned):
+    """The window is each walker's own, by its noise multiplier: walkers of
+    both windows and of none beside each other, whole and split, have the bits
+    that they have alone."""
+    print("[gpu-window-case] mixed %s" % binned, flush=True)
+    inp = dict(workload.make_inputs(npix_side=120, seed=9))
+    th = synth.walker_thetas(9, seed=23)
+    th[:, len(inp["knots"])] = [1.0, 0.25, 0.1, 0.3, 0.0, 2.0, 0.1, 0.26, 1.1]
+    want = [1, 2, 0, 1, 0, 1, 0, 2, 1]
+    ctx = workload.build_context(inp, 65536, 512, binned=binned)
+    alone = [ctx.loglike_batch(th[w:w + 1]) for w in range(len(th))]
+    for parts in (0, 1, 2, 4):
+        ctx.set_parts(parts)
+        ll, st = ctx.loglike_batch(th)
+        for w in range(len(th)):
+            assert _window(ctx, w) == want[w]
+            assert st[w] == alone[w][1][0] == 0
+            assert ll[w] == alone[w][0][0]
+
+
+def test_nodes_too_dense_for_windows():
+    """A beam of small values between knots a factor of ten apart puts 2048
+    nodes less than six grid points apart at point 2048, past the table of
+    single points: eight points then lie in more than two node intervals, and
+    the walkers keep the pruned transforms."""
+    print("[gpu-window-case] dense nodes", flush=True)
+    g, ps = synth.gaussian_beam()
+    sigma, nflux, ninterp = 2e-5, 65536, 2048
+    d = np.random.default_rng(3).normal(0.0, 1.3 * sigma, 3000)
+    inp = dict(beam=(1.5e-4 * g).ravel(), pixsize=ps, data=d, sigma=sigma,
+               minbeamval=1e-8, nbeamhist=120, nbins=200,
+               knots=np.geomspace(0.1, 1.0, 5))
+    th = np.array([[4.0, 3.5, 3.0, 2.5, 2.0, 1.0, 0, 0],
+                   [4.1, 3.6, 3.1, 2.6, 2.1, 1.0, 0, 0]], dtype=np.float32)
+    ctx = workload.build_context(inp, nflux, ninterp, binned=True)
+    ctx.loglike_batch(th)
+    x = ctx.get_rinterp(0)[0] / ctx.beamset_info(0)["dflux"]
+    assert 2 < np.diff(x[x > 2048.0])[0] < 6
+    L = build_oracle(inp, nflux, ninterp, True, th[0])
+    for parts in (1, 2, 4):
+        ctx.set_parts(parts)
+        ll, st = ctx.loglike_batch(th)
+        assert np.all(st == 0), st
+        assert _window(ctx) == 0
+        check_exact_parity(ctx, L, th, ll, tol=1e-6, nthreads=2)
 
 
 @pytest.mark.parametrize("nflux,cut,window", [
@@ -91,7 +161,7 @@ def test_values_made_again_are_the_same_bits(nflux, cut, window):
     for w in range(len(th)):
         dbg = ctx.get_debug(w)
         raw = ctx.get_pd(w, is_log="raw")[0]
-        assert dbg["window"] == window
+        assert _window(ctx, w) == window
         assert raw.max() == dbg["peak"]
         assert 0 < dbg["minval"] < 1e-5 * dbg["peak"]
         assert raw[int(dbg["minidx"])] == dbg["minval"] == raw.min()
@@ -112,7 +182,7 @@ def test_windowed_two_signed_beam(nflux):
         ll, st = ctx.loglike_batch(th)
         assert np.all(st == 0), st
         lls.append(ll)
-    assert _nrows(ctx) == 0
+    assert _window(ctx) == 1
     assert np.array_equal(lls[0], lls[1]) and np.array_equal(lls[0], lls[2])
     L = build_oracle(inp, nflux, 700, False, th[0])
     check_exact_parity(ctx, L, th, lls[0], tol=1e-6, nthreads=3)
@@ -148,7 +218,7 @@ def test_negative_fluxes_only_far_from_zero(nflux, shift):
             ctx.set_parts(parts)
             ll, st = ctx.loglike_batch(th)
             assert np.all(st == 0), st
-            assert (_nrows(ctx) == 0) == (shift == 0 and cut == 64.0)
+            assert _window(ctx) == (1 if shift == 0 and cut == 64.0 else 0)
             out.append((ll, ctx.get_debug(0)))
     ref, dref = out[-1]
     for ll, dbg in out:
