@@ -220,39 +220,44 @@ def main():
             "nbins": nbins, "ninterp": args.ninterp,
         },
         "status_ok": int(np.sum(b["st"] == 0)),
+        # the transforms are bound by FP64 work: with the default workload's
+        # FLOP (counted, above) achieved and frac are of that peak
         "roofline": {
-            "bound": "hbm",
-            "achieved": achieved,
-            "peak": HBM_PEAK_GBS,
-            "unit": "GB/s",
-            "frac": achieved / HBM_PEAK_GBS,
+            "bound": "fp64",
+            "achieved": None,
+            "peak": FP64_PEAK_TFLOPS,
+            "unit": "TFLOP/s",
+            "frac": None,
             "traffic": TRAFFIC.get(dom) if default_workload else None,
             "kernel": dom + "1d_kernel",
             "kernel_ms": kern_ms,
-            "bytes_alg_per_launch": b_stage[dom] * W,
             "stage_ms": stage_ms,
-            "pipeline": {
-                "achieved": pipe_achieved,
-                "frac": pipe_achieved / HBM_PEAK_GBS,
-                "batch_ms": batch_ms,
-                "bytes_alg_per_eval": b_eval,
+            # the bytes that separate passes would move over the time: what
+            # fusing them is worth, no stream (traffic is what is moved)
+            "hbm_algorithmic": {
+                "achieved": achieved,
+                "peak": HBM_PEAK_GBS,
+                "unit": "GB/s",
+                "frac": achieved / HBM_PEAK_GBS,
+                "bytes_alg_per_launch": b_stage[dom] * W,
+                "pipeline": {
+                    "achieved": pipe_achieved,
+                    "frac": pipe_achieved / HBM_PEAK_GBS,
+                    "batch_ms": batch_ms,
+                    "bytes_alg_per_eval": b_eval,
+                },
             },
         },
     }
     if default_workload:
-        # the same live kernel times against the FP64 peak, with the FLOP
-        # per launch the SQ counters give for this workload
         fp = {k: FP64_FLOP[k] / (stage_ms[k] * 1e-3) / 1e12
               for k in FP64_FLOP if stage_ms.get(k, 0) > 0}
-        out["roofline"]["fp64"] = {
-            "kernel": dom + "1d_kernel", "achieved": fp[dom],
-            "peak": FP64_PEAK_TFLOPS, "unit": "TFLOP/s",
-            "frac": fp[dom] / FP64_PEAK_TFLOPS,
-            "flop_per_launch": FP64_FLOP[dom],
-            "per_kernel": {k + "1d_kernel": {"achieved": v,
-                                             "frac": v / FP64_PEAK_TFLOPS}
-                           for k, v in fp.items()},
-        }
+        out["roofline"].update(
+            achieved=fp[dom], frac=fp[dom] / FP64_PEAK_TFLOPS,
+            flop_per_launch=FP64_FLOP[dom],
+            per_kernel={k + "1d_kernel": {"achieved": v,
+                                          "frac": v / FP64_PEAK_TFLOPS}
+                        for k, v in fp.items()})
     if args.unbinned_steps > 0:
         u = run(False, args.unbinned_steps, 2)
         out["unbinned"] = {
@@ -796,10 +801,10 @@ def bench_2d(args, hiprt):
                     % (n, n, W, args.side, args.side),
         "steps": steps, "batch_ms": batch_ms, "stage_ms": stage_ms,
         "status_ok": int(np.sum(st == 0)),
-        "pipeline": {"bound": "hbm", "achieved": achieved,
-                     "peak": HBM_PEAK_GBS, "unit": "GB/s",
-                     "frac": achieved / HBM_PEAK_GBS,
-                     "bytes_alg_per_eval": b_eval},
+        "hbm_algorithmic": {"achieved": achieved,
+                            "peak": HBM_PEAK_GBS, "unit": "GB/s",
+                            "frac": achieved / HBM_PEAK_GBS,
+                            "bytes_alg_per_eval": b_eval},
     }
     if not args.no_cpu and args.cpu_evals_2d > 0:
         sys.path.insert(0, os.path.join(ROOT, "oracle"))

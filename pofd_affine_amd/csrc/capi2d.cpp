@@ -698,14 +698,14 @@ int prepare_set2(pofd_ctx* c, Ctx2& C2, Set2& s) {
     }
     bc.maxf1 = maxknot * s.bm.max1[k];
   }
-  // the R kernel stages 3 doubles per element of a sign pair in LDS
+  // three doubles per element of a sign pair, row and walker in the workspace
   for (int k = 0; k < 2; ++k) {
     const size_t pair = static_cast<size_t>(d.comp[2 * k].n) + d.comp[2 * k + 1].n;
-    if (3 * pair * sizeof(double) > pofd2::kRgridMaxLds)
+    if (pair > pofd2::kMaxPieces)
       return ctx_fail(c, POFD_E_ARG,
                       "pofd2d_prepare: beam has " + std::to_string(pair) +
                           " elements in one band-1 sign; histogram it (at most " +
-                          std::to_string(pofd2::kRgridMaxLds / 24) + ")");
+                          std::to_string(pofd2::kMaxPieces) + ")");
   }
   // flux-grid tables
   std::vector<double> inv_m, lg_m, inv_e, lg_e;

@@ -27,8 +27,9 @@ constexpr int kRowBlocks2 = 64;    // workgroups per walker in the inverse row t
 // (4 coefficients per interval each), raw sigma and offset values
 constexpr int kModelStride = 8 + 14 * kMaxK;
 constexpr int kStats = 16;
-// limit of a row's beam pieces (3 doubles per beam element)
-constexpr size_t kRgridMaxLds = 144 * 1024;
+// most beam elements of one band-1 sign: a row of R has three doubles of
+// workspace for each
+constexpr size_t kMaxPieces = 6144;
 constexpr int kDbg2 = 32;
 
 enum {  // stats slots (per walker)

@@ -27,7 +27,8 @@ __device__ __forceinline__ float gelu_grad(const float x) {
 }
 
 // One K-slice (kKs long) of a tile's kTile rows of A, or columns of B, into
-// registers, 8 values per thread: element o of the tile at depth k is at
+// registers, 8 values per thread of the 64 x 64 tiles and 16 of the 32 x 32
+// ones: element o of the tile at depth k is at
 // p[k ld + o] (along) or p[o ld + k], and neighbouring lanes take
 // neighbouring addresses.  Zeros outside the matrix (loaded from its edge, so
 // that no load waits behind a branch).

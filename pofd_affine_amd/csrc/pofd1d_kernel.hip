@@ -13,8 +13,8 @@
 //             exp(R^ - R^0) with the mean shift (:1094-1132) and, per
 //             dataset, the noise factor (:1172-1188) applied to the rows
 //             the inverse needs
-//   inverse   per (walker, dataset): inverse transform, clamp, P(D) and its
-//             block statistics to HBM
+//   inverse   per (walker, dataset): inverse transform, clamp, block
+//             statistics of the P(D) to HBM, and of a pruned walker the P(D)
 //   finalize  per (walker, dataset): findSplitPoint (:691-921), rotation,
 //             normalisation and mean (:934-1009), the binned log likelihood
 //             (src/PD.cc:557-619)
@@ -23,7 +23,10 @@
 //   combine   (curr - like_offset)/like_norm summed over the datasets in
 //             order (src/calcLike.cc:425), into the batch outputs
 //
-// Transform design.  The real transform of length N = 2M is a complex
+// Transform design.  From N = 2^16 on a walker's transforms normally go
+// through a window onto a coarse grid, and nothing of size N is stored (the
+// windowed transforms, below; select_window says which walkers).  The others
+// take the pruned transforms: the real transform of length N = 2M is a complex
 // transform of length M = 256 * M2 in four-step form (m = M2*n1 + n2,
 // k = k1 + 256*k2): 256-point column transforms in LDS, a twiddle, then the
 // transform across columns.  After the noise factor only k <= kmax survive
@@ -32,7 +35,7 @@
 // k >= M - kmax, as a direct sum accumulated while the columns stream
 // through LDS; the inverse mirrors it.  R values are generated in the
 // forward column loop and never stored, so the only HBM traffic of size N
-// per walker and dataset is the P(D) itself.
+// per pruned walker and dataset is the P(D) itself.
 #include <hip/hip_runtime.h>
 
 #include <type_traits>

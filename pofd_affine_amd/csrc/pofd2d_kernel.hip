@@ -1150,7 +1150,8 @@ __global__ __launch_bounds__(kT) void split2d_kernel(const Set2Dev s, const Work
 // trapezoid sums of its rows and columns are the marginals of the unrotated
 // array, with the ends' weights moved: A = rsum1 + (P[i][0] + P[i][n-1]) / 2
 // - (P[i][s2] + P[i][s2-1]) / 2, and so for the columns; all terms are
-// non-negative parts of the sum.  Latency of 6 n gathered values; summing
+// non-negative parts of the sum.  Latency of 8 n gathered values and the 2 n
+// of the marginals; summing
 // the array itself again read 1.07 GB (268 us at 32 walkers, n = 2048).
 constexpr int kTN = 1024;
 __global__ __launch_bounds__(kTN) void norm2d_kernel(const Set2Dev s, const Work2 wk,
