@@ -410,6 +410,25 @@ __device__ __forceinline__ double window_value(const double* uw, const double* h
   for (int d = 0; d < kTaps; ++d) v = fma(uw[a + d], ht[(d << lp) + b], v);
   return fmax(v, 0.0);  // unwrapAndNormalizePD positivity
 }
+// the same at j and, into v1, at j + 1 modulo N, which share all coarse values
+// but one (a bin's two values: LDS reads bound the binned sum, 64 of them as
+// two calls, 49 here); uw up to [nc + kTaps - 1]
+__device__ __forceinline__ double window_pair(const double* uw, const double* ht, const int lp,
+                                              const int j, double& v1) {
+  const int p = 1 << lp, a = j >> lp, b = j & (p - 1);
+  const bool next = b + 1 == p;  // j + 1 lies in the next coarse cell
+  const int b1 = next ? 0 : b + 1;
+  double v = 0.0, w = 0.0, u = uw[a];
+#pragma unroll
+  for (int d = 0; d < kTaps; ++d) {
+    const double un = uw[a + d + 1];
+    v = fma(u, ht[(d << lp) + b], v);
+    w = fma(next ? un : u, ht[(d << lp) + b1], w);
+    u = un;
+  }
+  v1 = fmax(w, 0.0);
+  return fmax(v, 0.0);
+}
 // the window by tap into LDS (p x kTaps values)
 __device__ __forceinline__ void load_window(const WindowDev& win, double* ht) {
   for (int i = threadIdx.x; i < win.p * kTaps; i += blockDim.x)
@@ -1342,8 +1361,8 @@ __device__ void window_tail(const BeamsetDev& bs, const WorkDev& wk, const int w
   const int nitems = (kmaxb + 1) << hs;
   // what item `it` reads of the tables
   struct Item {
-    double2 e1, ea, c1, ca, w;
-    double inv, im1;
+    double2 e1, ea, c1, ca;
+    double im1;
   };
   auto item = [&](const int it) {
     const int k = (it < nitems) ? it >> hs : 0, part = it & ((1 << hs) - 1);
@@ -1354,8 +1373,6 @@ __device__ void window_tail(const BeamsetDev& bs, const WorkDev& wk, const int w
     t.ea = em1_load(bs, k8 * static_cast<uint32_t>((part * hl.nbp) >> hs));
     t.c1 = em1_load(bs, static_cast<uint32_t>(kp));
     t.ca = em1_load(bs, k8 * static_cast<uint32_t>(win.p * ((part * ncb) >> hs)));
-    t.w = bs.wc[k * ts];
-    t.inv = win.inv[k];
     t.im1 = win.invm1[k];
     return t;
   };
@@ -1390,7 +1407,13 @@ __device__ void window_tail(const BeamsetDev& bs, const WorkDev& wk, const int w
     for (int k = kf + 1 + tid; k < h - kf; k += kThreads) dst[coarse_at(k)] = make_double2(0.0, 0.0);
   };
   Item im;
-  if (kAhead) im = item(tid);
+  double2 w0 = make_double2(0.0, 0.0);
+  double inv0 = 0.0;
+  if (kAhead) {
+    im = item(tid);
+    w0 = bs.wc[min(tid, kmaxb) * ts];
+    inv0 = win.inv[min(tid, kmaxb)];
+  }
   const double2* z = fft_coarse(sm.bufa, sm.bufb, h, sm.tw);
   double2* zf = (z == sm.bufa) ? sm.bufb : sm.bufa;
   if (tid < 2 * ncb + 1) {
@@ -1454,28 +1477,39 @@ __device__ void window_tail(const BeamsetDev& bs, const WorkDev& wk, const int w
       dh.x += __shfl_xor(dh.x, o);
       dh.y += __shfl_xor(dh.y, o);
     }
-    if (act && part == 0) {
-      double2 pt = make_double2(1.0, 0.0);
-      if (k > 0) {
-        const double2 zk = z[coarse_at(k)], zm = z[coarse_at(h - k)];
-        const double2 A = make_double2(0.5 * (zk.x + zm.x), 0.5 * (zk.y - zm.y));
-        const double2 B = make_double2(0.5 * (zk.y + zm.y), -0.5 * (zk.x - zm.x));
-        const double2 X = cadd(A, cmul(im.w, B));
-        const double iv = im.inv;
-        double expfac, ival;
-        {
-#pragma clang fp contract(off)
-          expfac = exp((X.x * iv - r0) + dh.x);
-          ival = X.y * iv + dh.y;
-          if (doshift) ival -= wfac * static_cast<double>(k);
-        }
-        double s2, c2;
-        sincos(ival, &s2, &c2);
-        pt = make_double2(expfac * c2, expfac * s2);
-      }
-      prtrans[k] = pt;
-      put_noisy(0, k, pt, im.inv, im.w, zf);
+    if (act && part == 0) zf[coarse_at(k)] = dh;
+  }
+  __syncthreads();
+  // the spectrum, a thread per k: exp and sincos on a quarter of the lanes of
+  // the sums above would take up to four times the issue slots (spectrum1d 24.8
+  // -> 22.9 us at 2^16, one walker).  k's slot holds its sum until its own thread
+  // puts the value there.
+  for (int k = tid; k <= kmaxb; k += kThreads) {
+    if (!kAhead || k >= kThreads) {
+      w0 = bs.wc[k * ts];
+      inv0 = win.inv[k];
     }
+    const double2 dh = zf[coarse_at(k)];
+    double2 pt = make_double2(1.0, 0.0);
+    if (k > 0) {
+      const double2 zk = z[coarse_at(k)], zm = z[coarse_at(h - k)];
+      const double2 A = make_double2(0.5 * (zk.x + zm.x), 0.5 * (zk.y - zm.y));
+      const double2 B = make_double2(0.5 * (zk.y + zm.y), -0.5 * (zk.x - zm.x));
+      const double2 X = cadd(A, cmul(w0, B));
+      double expfac, ival;
+      {
+#pragma clang fp contract(off)
+        expfac = exp((X.x * inv0 - r0) + dh.x);
+        ival = X.y * inv0 + dh.y;
+        if (doshift) ival -= wfac * static_cast<double>(k);
+      }
+      double s2, c2;
+      sincos(ival, &s2, &c2);
+      pt = make_double2(expfac * c2, expfac * s2);
+    }
+    prtrans[k] = pt;
+    if (k > sm.isc[2]) zf[coarse_at(k)] = make_double2(0.0, 0.0);
+    put_noisy(0, k, pt, inv0, w0, zf);
   }
   if (tid >= kThreads - 64) {
     double vh = 0.0;
@@ -1496,9 +1530,8 @@ __device__ void window_tail(const BeamsetDev& bs, const WorkDev& wk, const int w
     if (f > 0) {
       // (each thread reads the spectrum values that it wrote)
       put_zeros(f, zf);
-      for (int it = tid; it < nitems; it += kThreads)
-        if ((it & ((1 << hs) - 1)) == 0)
-          put_noisy(f, it >> hs, prtrans[it >> hs], win.inv[it >> hs], bs.wc[(it >> hs) * ts], zf);
+      for (int k = tid; k <= kmaxb; k += kThreads)
+        put_noisy(f, k, prtrans[k], win.inv[k], bs.wc[k * ts], zf);
     }
     __syncthreads();
     const double2* u = fft_coarse(zf, zf == sm.bufa ? sm.bufb : sm.bufa, h, sm.tw);
@@ -2702,7 +2735,7 @@ __global__ __launch_bounds__(kThreads) void finalize1d_kernel(const BeamsetDev b
       blk = 16 * win.p;
       nbc = 0;
       const double* u = coarse_pd(bs, wk, walker, f);
-      for (int i = tid; i < win.nc + kTaps - 1; i += kThreads) uw[i] = u[(i - 7) & (win.nc - 1)];
+      for (int i = tid; i < win.nc + kTaps; i += kThreads) uw[i] = u[(i - 7) & (win.nc - 1)];
       load_window(win, ht);
     }
   }
@@ -2953,7 +2986,15 @@ __global__ __launch_bounds__(kThreads) void finalize1d_kernel(const BeamsetDev b
           const double delt = (cflux - minflux) * idflux;
           const int idx = static_cast<int>(delt);
           const double t = delt - static_cast<double>(idx);
-          part += ((1.0 - t) * Lrot(idx) + t * Lrot(idx + 1)) * nb;
+          const int jj = (idx + split) & (N - 1);
+          double p0, p1;
+          if (wsel) {
+            p0 = window_pair(uw, ht, lp, jj, p1);
+          } else {
+            p0 = pofd[jj];
+            p1 = pofd[(jj + 1) & (N - 1)];
+          }
+          part += ((1.0 - t) * log2_or_small(p0 * itot) + t * log2_or_small(p1 * itot)) * nb;
         }
       }
       curr = 0.69314718055994530942 * block_sum(part, red);  // log2toe

@@ -226,3 +226,36 @@ def test_negative_fluxes_only_far_from_zero(nflux, shift):
         for key in ("mn", "var_noi", "r0"):
             assert dbg[key] == pytest.approx(dref[key], rel=1e-10), key
         np.testing.assert_allclose(ll, ref, rtol=0, atol=1e-8)
+
+
+@pytest.mark.parametrize("sigmas,window", [((0.0006, 0.0025), 2),
+                                           ((0.0025, 0.0006), 2),
+                                           ((0.0025, 0.004), 1)])
+def test_datasets_of_different_noise(sigmas, window):
+    """Two datasets share the spectrum, kept up to the narrower noise's last
+    index: more of them than a workgroup has threads in the second window,
+    and zeros between in the other dataset's transform."""
+    print("[gpu-window-case] two datasets %g %g" % sigmas, flush=True)
+    nflux, ninterp = 65536, 512
+    inp = dict(workload.make_inputs(npix_side=120, seed=9, sigma=sigmas[0]))
+    other = dict(workload.make_inputs(npix_side=100, seed=10, sigma=sigmas[1]))
+    th = synth.walker_thetas(3, seed=25)
+    ctx = workload.build_context(inp, nflux, ninterp, binned=True)
+    ctx.add_field(0, pix=other["data"], sigma_base=sigmas[1])
+    ctx.prepare()
+    L = build_oracle(inp, nflux, ninterp, True, th[0])
+    L.add_field(0, pix=other["data"], sigma_base=sigmas[1])
+    L.finalize(th[0])
+    L.set_precise(1)
+    ref, rst = L.loglike_batch(th, 3)
+    assert np.all(rst == 0), rst
+    lls = []
+    for parts in (1, 2, 4):
+        ctx.set_parts(parts)
+        ll, st = ctx.loglike_batch(th)
+        assert np.all(st == 0), st
+        assert _window(ctx) == window
+        # the contract of every 1D path, for each dataset
+        np.testing.assert_allclose(ll, ref, rtol=0, atol=2e-6)
+        lls.append(ll)
+    assert np.array_equal(lls[0], lls[1]) and np.array_equal(lls[0], lls[2])
