@@ -349,12 +349,13 @@ long double window_at(long double x) {
   }
   return sum * phi0;
 }
-// Grids from this size take windows.  Measured per call at 2^14, 2^15 and
-// 2^16, 512 nodes: 256 walkers 110, 120 and 133 us against 107, 140 and 203
-// of the pruned transforms, 4 walkers over four workgroups each 88, 93 and
-// 100 us against 77, 78 and 95: below 2^16 the small calls lose what the
-// large ones gain (the choice may not follow the batch: a walker's bits do
-// not depend on it).
+// Grids from this size take windows.  Measured per call at 2^15 and 2^16, 512
+// nodes: 256 walkers 114 and 125 us against 139 and 202 of the pruned
+// transforms; 1 walker over four workgroups 87 and 95 against 76 and 93, 4
+// walkers 89 and 96 against 79 and 96: below 2^16 the small calls lose what
+// the large ones gain (the choice may not follow the batch: a walker's bits do
+// not depend on it).  At 2^16 a single walker loses 1 to 7%, most with a
+// two-signed beam and binned data.
 constexpr uint32_t kWinMinN = 1u << 16;
 int upload_windows(pofd_ctx* c, Beamset& s, int N, const std::vector<uint16_t>& kst) {
   BeamsetDev& d = s.dev;

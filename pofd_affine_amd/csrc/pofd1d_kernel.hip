@@ -1096,7 +1096,7 @@ __device__ __forceinline__ double row_shift(const double v) {
 // from the table rl that all threads made before (R(j) at j, R(N - v) at
 // kRlow + v).
 // Bound by the VALU work of R (26 instructions a point); the matrix cores
-// are busy for half of that, in its shadow.  With the tail 103 us for 256
+// are busy for half of that, in its shadow.  With the tail 102 us for 256
 // walkers at 2^17, where the pruned transform took 193 (its column
 // transforms through LDS, a barrier a stage).
 template <int Q>
