@@ -25,10 +25,10 @@ HBM_PEAK_GBS = 8000.0
 # written = 1.0 x WRITE_SIZE KiB); None where not profiled or for another
 # workload.
 TRAFFIC = {
-    "prep": (2.0 * 2091.2 + 20516.7) * 1024,
-    "forward": (2.0 * 10999.6 + 31577.8) * 1024,
-    "inverse": (2.0 * 4249.8 + 1080.0) * 1024,
-    "finalize": (2.0 * 4379.1 + 80.0) * 1024,
+    "prep": (2.0 * 2092.3 + 20513.2) * 1024,
+    "forward": (2.0 * 7627.0 + 13631.5) * 1024,
+    "inverse": (2.0 * 4241.3 + 1080.0) * 1024,
+    "finalize": (2.0 * 4363.8 + 80.0) * 1024,
 }
 FP64_PEAK_TFLOPS = 78.6
 # FP64 FLOP per launch of each kernel at the default workload, from
@@ -38,9 +38,9 @@ FP64_PEAK_TFLOPS = 78.6
 # kernel time for the FP64 roofline.
 FP64_FLOP = {
     "prep": 2.75e8,
-    "forward": 2.53e9,
+    "forward": 2.51e9,
     "inverse": 1.22e9,
-    "finalize": 1.02e8,
+    "finalize": 9.8e7,
 }
 
 
